@@ -5,6 +5,7 @@ parallel and links them into ``pyvibdmc_amd/libpyvibdmc_amd.so`` in place:
 * ``pvd_capi.hip``: the C ABI entry points and auxiliary kernels;
 * ``pvd_step_f32.hip`` / ``pvd_step_f64.hip``: the step kernels and their launches for
   float and double walkers;
+* ``pvd_resident.hip``: many discrete steps per launch, the walkers kept on chip;
 * ``pvd_mlp.hip``: the surrogate kernels.
 """
 import os
@@ -22,8 +23,12 @@ ARCH = os.environ.get('PVD_OFFLOAD_ARCH', 'gfx950')
 FLAGS = ['-O3', f'--offload-arch={ARCH}', '-std=c++17', '-fPIC', '-ffp-contract=off',
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops']
 
+# pvd_resident.hip: machine-level hoisting moves the constants of the mathematical functions out of
+# the step loop and spills them (FP64 triatomics: 104 spilled registers against none).
+EXTRA = {'pvd_resident.hip': ['-mllvm', '-disable-machine-licm']}
+
 TARGETS = [
-    ('libpyvibdmc_amd.so', ['pvd_capi.hip', 'pvd_step_f32.hip', 'pvd_step_f64.hip', 'pvd_mlp.hip']),
+    ('libpyvibdmc_amd.so', ['pvd_capi.hip', 'pvd_step_f32.hip', 'pvd_step_f64.hip', 'pvd_resident.hip', 'pvd_mlp.hip']),
 ]
 
 
@@ -60,7 +65,7 @@ def build(verbose=True, only=None):
         if not all(os.path.exists(p) for p in src_paths):
             continue
         objs = [os.path.join(OBJ, os.path.splitext(s)[0] + '.o') for s in srcs]
-        jobs = [([hipcc()] + FLAGS + ['-c', sp, '-o', o], os.path.basename(sp)) for sp, o in zip(src_paths, objs)]
+        jobs = [([hipcc()] + FLAGS + EXTRA.get(os.path.basename(sp), []) + ['-c', sp, '-o', o], os.path.basename(sp)) for sp, o in zip(src_paths, objs)]
         workers = max(1, min(len(jobs), int(os.environ.get('MAX_JOBS', '0')) or (os.cpu_count() or 1)))
         with ThreadPoolExecutor(max_workers=workers) as ex:
             for f in [ex.submit(_run, c, w, verbose) for c, w in jobs]:
@@ -89,7 +94,7 @@ def asan_runtime():
 
 def build_asan(verbose=True):
     """Build ASAN_LIB (after build(), whose other objects it links); returns its path."""
-    others = [os.path.join(OBJ, s) for s in ('pvd_step_f32.o', 'pvd_step_f64.o', 'pvd_mlp.o')]
+    others = [os.path.join(OBJ, s) for s in ('pvd_step_f32.o', 'pvd_step_f64.o', 'pvd_resident.o', 'pvd_mlp.o')]
     if not all(os.path.exists(o) for o in others):
         build(verbose)
     obj = os.path.join(OBJ, 'pvd_capi_asan.o')

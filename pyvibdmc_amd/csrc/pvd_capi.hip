@@ -3,7 +3,7 @@
 // potential / trial evaluation).  Declarations and conventions: include/pyvibdmc_amd.h.
 #include <initializer_list>
 
-#include "pvd_sim.hpp"
+#include "pvd_resident.hpp"
 
 using namespace pvd;
 
@@ -238,7 +238,7 @@ void free_sim(pvd_sim* s) {
   drop_surrogate_graphs(s);
   if (s->cap_stream) (void)hipStreamDestroy(s->cap_stream);
   void* ptrs[] = {s->coords[0], s->coords[1], s->who[0], s->who[1], s->w, s->E, s->ke, s->kmask,
-                  s->ctrl, s->flags, s->gflags, s->rec, s->drec, s->accs, s->tr_vref, s->tr_pop, s->tr_dteff, s->tr_births,
+                  s->ctrl, s->flags, s->gflags, s->rec, s->drec, s->accs, s->xch, s->tr_vref, s->tr_pop, s->tr_dteff, s->tr_births,
                   s->tr_deaths, s->pend, s->fin, s->klist, s->killtag, s->rstage, s->cand, s->rsg, s->ncnt, s->asg, s->cpy, s->stage, s->parent, s->parent_w, s->desc,
                   s->cnt, s->dacc, s->vsur, s->jlog, s->xc[0], s->xc[1]};
   for (void* p : ptrs)
@@ -347,6 +347,7 @@ int pvd_sim_create(const pvd_config* cfg, pvd_sim** out) {
   ALLOC(s->tr_dteff, sizeof(double) * s->tmax);
   ALLOC(s->tr_births, sizeof(int) * s->tmax);
   ALLOC(s->tr_deaths, sizeof(int) * s->tmax);
+  if (!s->cont) ALLOC(s->xch, sizeof(uint64_t) * RES_XWORDS);
   if (s->cont) {
     ALLOC(s->pend, sizeof(Piece) * RP_PCAP * 2);
     ALLOC(s->fin, sizeof(Piece) * RP_FCAP);
@@ -369,6 +370,7 @@ int pvd_sim_create(const pvd_config* cfg, pvd_sim** out) {
   if (e == hipSuccess) e = hipMemset(s->gflags, 0, sizeof(uint64_t) * (ntiles / LB_GROUP + 1));
   if (e == hipSuccess) e = hipMemset(s->drec, 0, sizeof(uint64_t) * 3 * ntiles);
   if (e == hipSuccess) e = hipMemset(s->accs, 0, sizeof(unsigned) * 2 * ACC_SLOTS * ACC_STRIDE);
+  if (e == hipSuccess && s->xch) e = hipMemset(s->xch, 0, sizeof(uint64_t) * RES_XWORDS);
   if (e == hipSuccess) e = hipMemset(s->ctrl, 0, sizeof(Ctrl));
   if (e == hipSuccess) e = hipMemset(s->tr_vref, 0, sizeof(double) * s->tmax);
   if (e == hipSuccess) e = hipMemset(s->tr_pop, 0, sizeof(double) * s->tmax);

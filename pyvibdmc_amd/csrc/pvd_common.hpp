@@ -25,6 +25,15 @@ struct Philox4 {
 
 PVD_DEV uint32_t mulhi32(uint32_t a, uint32_t b) { return __umulhi(a, b); }
 
+// a ^ b ^ c in one instruction (v_bitop3_b32; left to the compiler, the two exclusive ors stay two)
+PVD_DEV uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 // Philox4x32 with 10 rounds.  ctr = (c0..c3), key = (k0, k1).
 PVD_DEV Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
                               uint32_t k1) {
@@ -37,8 +46,8 @@ PVD_DEV Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3
     const uint64_t p1 = (uint64_t)M1 * (uint64_t)c2;
     const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
     const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
-    const uint32_t n0 = hi1 ^ c1 ^ k0;
-    const uint32_t n2 = hi0 ^ c3 ^ k1;
+    const uint32_t n0 = xor3(hi1, c1, k0);
+    const uint32_t n2 = xor3(hi0, c3, k1);
     c0 = n0;
     c1 = lo1;
     c2 = n2;

@@ -276,8 +276,8 @@ PVD_DEV uint32_t spare_byte(const uint32_t* w, int b) {
 // caller's arrays (the reference's draw order).  Philox, FP32: DrawLayout words from
 // ceil(NW / 4) blocks of one stream per (slot, step) - 2 blocks for 9 components.
 // Philox, FP64: 53-bit uniforms from separate blocks per purpose.
-template <typename R, int NP, bool INJ, bool IS>
-PVD_DEV void draw_step(const StepArgs<R>& A, long long i, unsigned long long step, R* disp, double& um,
+template <typename R, int NP, bool INJ, bool IS, typename AT>
+PVD_DEV void draw_step(const AT& A, long long i, unsigned long long step, R* disp, double& um,
                        double& ub, bool want_branch) {
   if constexpr (INJ) {
 #pragma unroll
@@ -315,8 +315,8 @@ PVD_DEV void draw_step(const StepArgs<R>& A, long long i, unsigned long long ste
   }
 }
 
-template <typename R, bool INJ>
-PVD_DEV double draw_u(const StepArgs<R>& A, long long i, unsigned long long step, uint32_t purpose) {
+template <typename R, bool INJ, typename AT>
+PVD_DEV double draw_u(const AT& A, long long i, unsigned long long step, uint32_t purpose) {
   if constexpr (INJ) {
     return purpose == RNG_BRANCH ? A.inj_ubr[i] : A.inj_umet[i];
   } else {
@@ -361,8 +361,8 @@ PVD_DEV R local_kin(const StepArgs<R>& A, const R* sec) {
 // mass-weighted Laplacian only (trial_water_fast / trial_gauss_fast).  Same mathematics as the
 // literal path below (imp_samp.py:28-53): Metropolis in log form, local kinetic energy
 // -1/2 sum_p (1/m_p) (g_p^2 + d2 ln psi / dx_p^2) summed over components.
-template <typename R, int NP, int MS>
-PVD_DEV R is_move_fast(const StepArgs<R>& A, const R* disp, double u, R* x, bool& acc) {
+template <typename R, int NP, int MS, typename AT>
+PVD_DEV R is_move_fast(const AT& A, const R* disp, double u, R* x, bool& acc) {
   const R dt = (R)A.dt;
   R lx, ly, lapx, lapy, gx[NP], gy[NP], y[NP];
   if constexpr ((MS & MS_TRIAL_WATER) != 0 && NP == 9) {
@@ -661,6 +661,30 @@ PVD_DEV void finalize_discrete(const StepArgs<R>& A, Ctrl* C, int par, int n, in
   }
 }
 
+// Branching weight and copy count of one walker (pyvibdmc.py:392-407); bad = 1 for a weight that
+// is not finite or beyond the population bound.  F32: the single-precision weight of the FP32
+// production path; otherwise NumPy's double arithmetic (parity).
+template <bool F32>
+PVD_DEV int branch_copies(double E, double vref, double dte, double u, double pop_hi, int& bad) {
+  if constexpr (F32) {
+    const float wf = pvd_exp<float>((float)((-1. * (E - vref)) * dte));
+    if (!isfinite(wf) || (double)wf > pop_hi + 1.0) {
+      bad = 1;
+      return 0;
+    }
+    const float fl = floorf(wf);
+    return (int)fl + ((float)u < (wf - fl) ? 1 : 0);
+  } else {
+    const double w = exp((-1. * (E - vref)) * dte);
+    if (!isfinite(w) || w > pop_hi + 1.0) {
+      bad = 1;
+      return 0;
+    }
+    const double fl = floor(w);
+    return (int)fl + (u < (w - fl) ? 1 : 0);
+  }
+}
+
 // MODE: INJ = injected draws; IS = importance sampling (analytic trial); EXT = energies
 // from V_ext (walkers already moved; NP = 0 reads the component count at run time).
 // Tile b is block b.  Workgroups are dispatched in index order within each XCD, so the
@@ -718,31 +742,10 @@ __global__ __launch_bounds__(TILE) void k_discrete(StepArgs<R> A) {
         E = (double)pes_eval_s<R, NP, MS>(A.pes, x[k]);
       }
     }
-    // branching weight and copy count (pyvibdmc.py:392-407)
     int ck = valid ? 1 : 0;
     if (valid && A.branch) {
       const double u = (EXT || IS) ? draw_u<R, INJ>(A, i, step, RNG_BRANCH) : ub;
-      if constexpr (sizeof(R) == 4 && !INJ) {
-        // FP32 production path: single-precision weight (the FP64 parity path below
-        // follows NumPy's double arithmetic)
-        const float wf = pvd_exp<float>((float)((-1. * (E - vref)) * dte));
-        if (!isfinite(wf) || (double)wf > A.pop_hi + 1.0) {
-          bad = 1;
-          ck = 0;
-        } else {
-          const float fl = floorf(wf);
-          ck = (int)fl + ((float)u < (wf - fl) ? 1 : 0);
-        }
-      } else {
-        const double w = exp((-1. * (E - vref)) * dte);
-        if (!isfinite(w) || w > A.pop_hi + 1.0) {
-          bad = 1;
-          ck = 0;
-        } else {
-          const double fl = floor(w);
-          ck = (int)fl + (u < (w - fl) ? 1 : 0);
-        }
-      }
+      ck = branch_copies<sizeof(R) == 4 && !INJ>(E, vref, dte, u, A.pop_hi, bad);
     }
     c[k] = ck;
     sce += (double)ck * E;

@@ -146,12 +146,14 @@ PVD_DEV void gather3(const R* x, const int* idx, R* g) {
   }
 }
 
-// Evaluate a device PES.  NP is the number of Cartesian components per walker.
+// Evaluate a device PES.  NP is the number of Cartesian components per walker; PT is PesParams
+// or a struct of the same members with the parameters already in R (R(0.5) * R(p) has the value
+// of R(0.5 * p): halving is exact).
 // The [O, H, H, O, H, H] cluster: two Morse+bend monomers, an O-O Morse term and the
 // Coulomb energy of the inter-monomer atom pairs.
-template <typename R>
-PVD_DEV R cluster6_v(const PesParams& P, const R* x) {
-  const R De = R(P.p[0]), a = R(P.p[1]), re = R(P.p[2]), hk = R(0.5 * P.p[3]), th0 = R(P.p[4]);
+template <typename R, typename PT>
+PVD_DEV R cluster6_v(const PT& P, const R* x) {
+  const R De = R(P.p[0]), a = R(P.p[1]), re = R(P.p[2]), hk = R(0.5) * R(P.p[3]), th0 = R(P.p[4]);
   R v = morse_bend_v<R>(x, 3, 6, 0, De, a, re, hk, th0) + morse_bend_v<R>(x, 12, 15, 9, De, a, re, hk, th0);
   const R roo = norm3(x[0] - x[9], x[1] - x[10], x[2] - x[11]);
   const R m = R(1) - pvd_exp<R>(-R(P.p[6]) * (roo - R(P.p[7])));
@@ -239,8 +241,8 @@ PVD_DEV R ps_water_v(const R* x) {
   return (((poly * damp + R(PS_C[0])) + voh1) + voh2) + vhh;
 }
 
-template <typename R, int NP>
-PVD_DEV R pes_eval(const PesParams& P, const R* x) {
+template <typename R, int NP, typename PT>
+PVD_DEV R pes_eval(const PT& P, const R* x) {
   switch (P.kind) {
     case PES_HARMONIC_X: {
       const R x0 = x[0];
@@ -253,11 +255,11 @@ PVD_DEV R pes_eval(const PesParams& P, const R* x) {
     case PES_MORSE_BEND:
       if constexpr (NP >= 9) {
         if (P.idx[0] == 0 && P.idx[1] == 1 && P.idx[2] == 2)  // [H, H, O], the usual order
-          return morse_bend_v<R>(x, 0, 3, 6, R(P.p[0]), R(P.p[1]), R(P.p[2]), R(0.5 * P.p[3]), R(P.p[4]));
+          return morse_bend_v<R>(x, 0, 3, 6, R(P.p[0]), R(P.p[1]), R(P.p[2]), R(0.5) * R(P.p[3]), R(P.p[4]));
         // other orders: gather (h1, h2, o) with selects so the walker stays in registers
         R g[9];
         gather3<R, NP>(x, P.idx, g);
-        return morse_bend_v<R>(g, 0, 3, 6, R(P.p[0]), R(P.p[1]), R(P.p[2]), R(0.5 * P.p[3]), R(P.p[4]));
+        return morse_bend_v<R>(g, 0, 3, 6, R(P.p[0]), R(P.p[1]), R(P.p[2]), R(0.5) * R(P.p[3]), R(P.p[4]));
       }
       break;
     case PES_CLUSTER6:
@@ -539,10 +541,10 @@ enum ModelSpec : int { MS_ANY = 0, MS_PES_WATER = 1, MS_TRIAL_WATER = 2, MS_PES_
 constexpr int MS_PES_ANY_SPEC = MS_PES_WATER | MS_PES_CLUSTER;
 constexpr int MS_TRIAL_ANY_SPEC = MS_TRIAL_WATER | MS_TRIAL_CLUSTER;
 
-template <typename R, int NP, int MS>
-PVD_DEV R pes_eval_s(const PesParams& P, const R* x) {
+template <typename R, int NP, int MS, typename PT>
+PVD_DEV R pes_eval_s(const PT& P, const R* x) {
   if constexpr ((MS & MS_PES_WATER) != 0 && NP == 9) {
-    return morse_bend_v<R>(x, 0, 3, 6, R(P.p[0]), R(P.p[1]), R(P.p[2]), R(0.5 * P.p[3]), R(P.p[4]));
+    return morse_bend_v<R>(x, 0, 3, 6, R(P.p[0]), R(P.p[1]), R(P.p[2]), R(0.5) * R(P.p[3]), R(P.p[4]));
   } else if constexpr ((MS & MS_PES_CLUSTER) != 0 && NP == 18) {
     return cluster6_v<R>(P, x);
   } else {
@@ -650,8 +652,8 @@ PVD_DEV void trial_gauss_fast(const TrialParams& T, const double* inv_m, const R
 //   |grad_k|^2 = 1/rv^2, |grad_j|^2 = 1/ru^2 + 1/rv^2 - 2 cos/(ru rv); lap_i = cot/ru^2,
 //   lap_k = cot/rv^2, lap_j = cot (1/ru^2 + 1/rv^2) - 2/(ru rv sin).
 // im_h, im_o: 1/m of the hydrogens and of the oxygen.
-template <typename R>
-PVD_DEV void trial_water_fast(const TrialParams& T, const R* x, R im_h, R im_o, R& lnpsi, R* g, R& lap) {
+template <typename R, typename TT>
+PVD_DEV void trial_water_fast(const TT& T, const R* x, R im_h, R im_o, R& lnpsi, R* g, R& lap) {
   R u[3], v[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -695,8 +697,8 @@ PVD_DEV void trial_water_fast(const TrialParams& T, const R* x, R im_h, R im_o, 
 // h1-o and h2-o (parameters KB, KB + 1) and the angle h1-o-h2 (parameter KA), atoms at the
 // compile-time component offsets H1, H2, O.  Adds to q2 = sum alpha (q - q0)^2, to the
 // gradient g of ln psi and to the mass-weighted Laplacian lap.
-template <typename R, int H1, int H2, int O, int KB, int KA>
-PVD_DEV void trial_mono_acc(const TrialParams& T, const R* x, R im_h, R im_o, R& q2, R* g, R& lap) {
+template <typename R, int H1, int H2, int O, int KB, int KA, typename TT>
+PVD_DEV void trial_mono_acc(const TT& T, const R* x, R im_h, R im_o, R& q2, R* g, R& lap) {
   R u[3], v[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -737,8 +739,8 @@ PVD_DEV void trial_mono_acc(const TrialParams& T, const R* x, R im_h, R im_o, R&
 
 // The [O, H, H, O, H, H] cluster trial (bonds 1-0, 2-0, 4-3, 5-3; angles 1-0-2, 4-3-5) as
 // two monomers; im_h, im_o: 1/m of the hydrogens and of the oxygens.
-template <typename R>
-PVD_DEV void trial_cluster_fast(const TrialParams& T, const R* x, R im_h, R im_o, R& lnpsi, R* g, R& lap) {
+template <typename R, typename TT>
+PVD_DEV void trial_cluster_fast(const TT& T, const R* x, R im_h, R im_o, R& lnpsi, R* g, R& lap) {
 #pragma unroll
   for (int p = 0; p < 18; ++p) g[p] = R(0);
   R q2 = R(0);

@@ -1,0 +1,186 @@
+// Resident discrete steps (pvd_resident.hpp): the launch plan of a simulation and its launches.
+#include "pvd_resident.hpp"
+
+namespace pvd {
+
+namespace {
+
+// Largest dynamic LDS a workgroup of k_resident may ask for: 160 KB less its static arrays.
+constexpr int RES_LDS = 160 * 1024 - 5 * 1024;
+
+struct Instance {
+  const void* fn;
+  int W, ntmax, stride;
+};
+
+// FP32 and FP64 plain steps for the fused component counts, and FP32 importance sampling with the
+// compiled trials.  Two shapes each: `small`, at most two rounds of 512 threads per workgroup (the
+// step is latency then: fewer rounds to rank, 256 registers a wave), and W rounds of up to 1024
+// threads, which hold the population's whole range, 1.5 N0, wherever the LDS holds N0.  ntmax 512
+// where a walker needs more than the 128 registers a wave of 1024 threads has.
+template <typename R, int NP, bool IS, int MS, int W, int NTM>
+Instance shapes(bool small) {
+  if (small) return Instance{(const void*)k_resident<R, NP, IS, MS, 2, 512, false>, 2, 512, res_stride<R, NP>()};
+  return Instance{(const void*)k_resident<R, NP, IS, MS, W, NTM, true>, W, NTM, res_stride<R, NP>()};
+}
+
+template <typename R>
+Instance instance(const pvd_sim* s, bool small) {
+  const int ms = s->mspec;
+  if constexpr (sizeof(R) == 4) {
+    if (s->is) {
+      if (s->np == 9 && ms == (MS_PES_WATER | MS_TRIAL_WATER))
+        return shapes<R, 9, true, MS_PES_WATER | MS_TRIAL_WATER, 6, 1024>(small);
+      if (s->np == 9 && ms == MS_TRIAL_WATER) return shapes<R, 9, true, MS_TRIAL_WATER, 6, 1024>(small);
+      if (s->np == 18 && ms == (MS_PES_CLUSTER | MS_TRIAL_CLUSTER))
+        return shapes<R, 18, true, MS_PES_CLUSTER | MS_TRIAL_CLUSTER, 6, 512>(small);
+    } else {
+      if (s->np == 1) return shapes<R, 1, false, MS_ANY, 6, 1024>(small);
+      if (s->np == 3) return shapes<R, 3, false, MS_ANY, 6, 1024>(small);
+      if (s->np == 9 && (ms & MS_PES_WATER)) return shapes<R, 9, false, MS_PES_WATER, 6, 1024>(small);
+      if (s->np == 9) return shapes<R, 9, false, MS_ANY, 6, 1024>(small);
+      if (s->np == 18 && (ms & MS_PES_CLUSTER)) return shapes<R, 18, false, MS_PES_CLUSTER, 3, 1024>(small);
+    }
+  } else if (!s->is) {
+    if (s->np == 1) return shapes<R, 1, false, MS_ANY, 6, 1024>(small);
+    if (s->np == 3) return shapes<R, 3, false, MS_ANY, 6, 1024>(small);
+    if (s->np == 9 && (ms & MS_PES_WATER)) return shapes<R, 9, false, MS_PES_WATER, 6, 512>(small);
+    if (s->np == 9) return shapes<R, 9, false, MS_ANY, 6, 512>(small);
+  }
+  return Instance{nullptr, 0, 0, 0};
+}
+
+// Workgroups, threads and LDS of the resident launch, or fn = nullptr where it does not serve:
+// N0 walkers must fit the LDS of the workgroups with 2 % to spare (the rest of the population's
+// range lives in the per-workgroup extension), every capacity's worth of walkers the rounds, and
+// the grid must be resident at once.
+struct Plan {
+  const void* fn;
+  int grid, nt, capl;
+  size_t lds;
+};
+
+template <typename R>
+Plan make_plan(pvd_sim* s, bool who) {
+  Plan P{nullptr, 0, 0, 0, 0};
+  const long long n0 = s->cfg.num_walkers;
+  const int gmax = std::min(s->cus, RES_MAXG);
+  const int share = 256;
+  const int g = (int)std::max(1ll, std::min<long long>(gmax, (n0 + share - 1) / share));
+  const long long per = (n0 + g - 1) / g, most = (s->cap + g - 1) / g;
+  const bool small = most <= 2 * 512 && per + per / 16 <= 512;
+  const Instance I = instance<R>(s, small);
+  if (!I.fn) return P;
+  int nt = 64;
+  while (nt < I.ntmax && (nt < per + per / 16 || nt * I.W < most)) nt *= 2;
+  const int unit = I.stride * (int)sizeof(R) + (who ? (int)sizeof(int) : 0);
+  const int capb = nt * I.W;
+  const int capl = std::min(capb, RES_LDS / unit / PVD_WAVE * PVD_WAVE);
+  if (per + per / 50 > (who ? capb : capl) || most > capb || (small && capl < capb)) return P;
+  // the extension lives in the staging buffer (np doubles per slot)
+  if ((long long)g * (capb - capl) * (I.stride + 1) * (long long)sizeof(R) > (long long)sizeof(double) * s->np * s->cap)
+    return P;
+  P.lds = (size_t)unit * capl;
+  if (hipFuncSetAttribute(I.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return P;
+  }
+  int per_cu = 0, coop = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, I.fn, nt, P.lds) != hipSuccess ||
+      (long long)per_cu * s->cus < g) {
+    (void)hipGetLastError();
+    return P;
+  }
+  P.fn = I.fn;
+  P.grid = g;
+  P.nt = nt;
+  P.capl = capl;
+  return P;
+}
+
+}  // namespace
+
+// Steps of one cooperative launch at most (a bound on how long one kernel runs: about 60 ms at a
+// million walkers), and the fewest for which it is used: a call costs about 40 us more than a step
+// kernel's launch does (the cooperative queue, the second launch, walkers in and out).  us a step
+// in calls of 16 steps, here and launch per step: water 1 000 walkers 6.7, 9.0; 100 000 6.9, 10.5;
+// 1 000 000 17.5, 20.9; with importance sampling 34.5, 51.1; cluster 200 000 13.2, 17.3.
+constexpr int RES_STEPS = 4096;
+constexpr int RES_MIN = 16;
+
+template <typename R>
+int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
+  done = 0;
+  if (s->cont || !s->xch || s->htrial || s->cfg.pes.kind == PES_EXTERNAL || n_steps < RES_MIN) return 0;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  const Plan P = make_plan<R>(s, s->who_on);
+  if (!P.fn) return 0;
+  ResArgs<R> A;
+  std::memset(&A, 0, sizeof(A));
+  for (int b = 0; b < 2; ++b) {
+    A.buf[b] = (R*)s->coords[b];
+    A.who[b] = s->who[b];
+  }
+  A.ext = (R*)s->stage;
+  A.ctrl = s->ctrl;
+  A.xch = s->xch;
+  A.tr_vref = s->tr_vref;
+  A.tr_pop = s->tr_pop;
+  A.tr_dteff = s->tr_dteff;
+  A.tr_births = s->tr_births;
+  A.tr_deaths = s->tr_deaths;
+  A.cap = s->cap;
+  A.tmax = s->tmax;
+  const StepArgs<R> S = make_args<R>(s);
+  A.dt = S.dt;
+  A.alpha = S.alpha;
+  A.n0 = S.n0;
+  A.pop_lo = S.pop_lo;
+  A.pop_hi = S.pop_hi;
+  A.branch_every = s->cfg.branch_every > 0 ? s->cfg.branch_every : 1;
+  A.capl = P.capl;
+  A.who_on = s->who_on ? 1 : 0;
+  A.rng = S.rng;
+  A.pes.kind = S.pes.kind;
+  std::memcpy(A.pes.idx, S.pes.idx, sizeof(A.pes.idx));
+  for (int k = 0; k < 12; ++k) A.pes.p[k] = (R)S.pes.p[k];
+  for (int k = 0; k < PVD_MAX_TB; ++k) {
+    A.trial.balpha[k] = (R)S.trial.balpha[k];
+    A.trial.br0[k] = (R)S.trial.br0[k];
+  }
+  for (int k = 0; k < PVD_MAX_TA; ++k) {
+    A.trial.aalpha[k] = (R)S.trial.aalpha[k];
+    A.trial.ath0[k] = (R)S.trial.ath0[k];
+  }
+  A.trial.c0 = (R)S.trial.c0;
+  for (int p = 0; p < s->np; ++p) {
+    A.sigma[p] = (R)S.sigma[p];
+    A.inv_m[p] = (R)S.inv_m[p];
+    A.h2s[p] = S.h2s[p];
+  }
+  while (done < n_steps) {
+    A.steps = std::min(RES_STEPS, n_steps - done);
+    A.par = (int)(s->next_step & 1);
+    void* args[] = {&A};
+    s->res_gate += 2;
+    for (unsigned second = 0; second < (P.grid > 1 ? 2u : 1u); ++second) {
+      A.gate = s->res_gate | second;
+      HIPCHK(hipLaunchCooperativeKernel(P.fn, dim3(P.grid), dim3(P.nt), args, (unsigned)P.lds, st));
+    }
+    s->next_step += A.steps;
+    s->epoch_next += 2 * (unsigned)A.steps + 2;  // a failed launch retraces its steps under new epochs
+    done += A.steps;
+  }
+  return 0;
+}
+
+template int run_resident<float>(pvd_sim*, int, hipStream_t, int&);
+template int run_resident<double>(pvd_sim*, int, hipStream_t, int&);
+
+}  // namespace pvd

@@ -59,6 +59,8 @@ struct pvd_sim {
   pvd::TileRec* rec;
   uint64_t* drec;
   unsigned* accs;
+  uint64_t* xch;  // exchange words of the resident steps (discrete weighting)
+  unsigned res_gate;  // tag of the last resident launch
   double* tr_vref;
   double* tr_pop;
   double* tr_dteff;
@@ -257,6 +259,11 @@ int do_is_accept(pvd_sim* s, const double* y, const double* psi, const double* f
                  const double* um, hipStream_t st);
 template <typename R>
 int do_pes(pvd_sim* s, double* v, hipStream_t st);
+
+// Fused discrete steps with the walkers kept on chip (pvd_resident.hip): runs `done` of n_steps
+// (all, or none where the resident launch does not serve this simulation, size or stream).
+template <typename R>
+int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done);
 
 #define PVD_SIM_OPS(R)                                                                                   \
   template int run_steps<R>(pvd_sim*, int, const double*, const double*, const double*, hipStream_t);  \

@@ -280,7 +280,11 @@ int run_steps(pvd_sim* s, int n_steps, const double* disp, const double* um, con
     return run_surrogate_steps<R>(s, n_steps, st);
   }
   int k = 0;
-  const bool graphs = !disp && s->use_graphs && (s->cfg.branch_every <= 1) && n_steps >= PVD_GRAPH_STEPS + 1;
+  if (!disp) {
+    const int rc = run_resident<R>(s, n_steps, st, k);
+    if (rc || k == n_steps) return rc;
+  }
+  const bool graphs = !disp && s->use_graphs && (s->cfg.branch_every <= 1) && n_steps - k >= PVD_GRAPH_STEPS + 1;
   if (graphs) {
     if (s->next_step & 1) {
       StepArgs<R> A = make_args<R>(s);
