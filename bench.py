@@ -485,7 +485,7 @@ def cluster_study(n, steps, epochs, zpe_steps):
             tf = MLP256_FLOP_PER_WALKER * mean_n / (e_ms * 1e-3) / 1e12
             row["mlp_roofline"] = {"bound": "mfma", "achieved": tf, "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                                    "frac": tf / MFMA_BF16_PEAK_TFLOPS, "avg_launch_ms": e_ms,
-                                   "kernel": "k_mlp_energy_st<float,18,256> + k_mlp_fallback",
+                                   "kernel": "k_mlp_energy_reg<float,18,256> + k_mlp_fallback",
                                    "flop_per_walker": MLP256_FLOP_PER_WALKER}
             del vbuf
         out[name] = row

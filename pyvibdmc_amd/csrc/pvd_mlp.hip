@@ -93,8 +93,10 @@ PVD_DEV int phys_unit(int c, int g, int j) { return 16 * (2 * c + (j >> 2)) + 4 
 //     removes).
 // The permutation is packed as 4-bit fields (position p holds atom (perm >> 4p) & 15), so
 // no lane indexes a register array at run time; every table lookup has a compile-time index.
+// With `scratch` (LDS, element q of this thread at scratch[q * step]) the pair distances are taken
+// from there: 15 writes and reads instead of 225 compares and selects for six atoms.
 template <typename R, int NP>
-PVD_DEV void mlp_descriptor(const MlpNet& M, const R* x, float* f) {
+PVD_DEV void mlp_descriptor(const MlpNet& M, const R* x, float* f, float* scratch = nullptr, int step = 0) {
   constexpr int NA = NP / 3, NPR = NA * (NA - 1) / 2;
   static_assert(NA <= MLP_MAXA && NPR <= MLP_MAXP, "too many atoms");
   float dc[NPR];
@@ -174,7 +176,23 @@ PVD_DEV void mlp_descriptor(const MlpNet& M, const R* x, float* f) {
     }
     perm = fp;
   }
-  {
+  if (scratch) {
+    // pair (lo, hi) is number first(lo) + hi, with first(lo) + 1 in the nibbles of a constant
+    unsigned first = 0;
+#pragma unroll
+    for (int a = 0; a < NA - 1; ++a) first |= (unsigned)(a * NA - a * (a + 1) / 2 - a) << (4 * a);
+#pragma unroll
+    for (int q = 0; q < NPR; ++q) scratch[q * step] = dc[q];
+    int q = 0;
+#pragma unroll
+    for (int p1 = 0; p1 < NA; ++p1)
+#pragma unroll
+      for (int p2 = p1 + 1; p2 < NA; ++p2) {
+        const unsigned a1 = (perm >> (4 * p1)) & 15u, a2 = (perm >> (4 * p2)) & 15u;
+        const unsigned lo = a1 < a2 ? a1 : a2, hi = a1 < a2 ? a2 : a1;
+        f[q++] = scratch[(int)(((first >> (4 * lo)) & 15u) + hi - 1u) * step];
+      }
+  } else {
     int q = 0;
 #pragma unroll
     for (int p1 = 0; p1 < NA; ++p1)
@@ -693,24 +711,59 @@ bool build_net(const pvd_mlp* m, MlpNet& N) {
 
 // ------------------------------------------------------------------------------------
 // Inference on walkers, H = 128: persistent workgroups keep all three weight packs (72 KB),
-// the biases and the output weights in LDS for the whole launch and loop over walker
-// chunks (E_WAVES waves x NT_E tiles of 16 walkers).  Each A fragment read from LDS feeds NT_E MFMAs; the
-// biases enter as the MFMA accumulator input.  Walkers outside the training range get the
-// FALLBACK_MARK bit pattern, which k_mlp_fallback replaces with the analytic potential.
+// the biases and the output weights in LDS for the whole launch; each wave has its own range of
+// walkers and activations never leave its registers.  A wave takes 64 walkers at a time: their
+// descriptors, one lane each, then the network on two tiles of NT_E x 16 (each A fragment read
+// from LDS feeds NT_E MFMAs; the biases enter as the MFMA accumulator input).  Walkers outside
+// the training range get the FALLBACK_MARK bit pattern, which k_mlp_fallback replaces with the
+// analytic potential.
+// Bound by VALU issue (SiLU: two transcendentals of 8 cycles and three other instructions an
+// activation).  With the descriptor of a walker computed by the four lanes that share its tile
+// column, and workgroups taking whole chunks of 256 walkers: water, 400 000 walkers FP32 75.5 us,
+// now 65.7 (k_mlp_fallback and the launches included); six atoms, 200 000 walkers FP64 133, 60.
 constexpr int NT_E = 2;
 constexpr int E_WAVES = 8;  // waves per workgroup sharing one LDS copy of the weights
 constexpr unsigned long long FALLBACK_MARK = 0x7FF4D1CEFA11BAC4ull;  // a signalling-NaN payload
+constexpr unsigned OUT_OF_RANGE = 0x7FA11BACu;                        // the same for a baseline, in FP32
 
 template <int H>
 constexpr size_t energy_lds_bytes() {
   return (size_t)((H / 16) * 64 + 2 * (H / 16) * (H / 32) * 64) * 16 + (size_t)(4 * H + 4) * 4;
 }
 
+// Normalised features of a walker as bf16 (16, the rest zero) and its quadratic baseline, or
+// OUT_OF_RANGE.  `scratch`: see mlp_descriptor.
+template <typename R, int NP>
+PVD_DEV float energy_features(const MlpNet& M, const R* x, bf16x8 (&v)[2], float* scratch, int step) {
+  constexpr int NPR = NP / 3 * (NP / 3 - 1) / 2;
+  float f[MLP_MAXP];
+  mlp_descriptor<R, NP>(M, x, f, scratch, step);
+  bool out = false;
+  if (M.use_range) {
+#pragma unroll
+    for (int k = 0; k < NPR; ++k) out |= !(f[k] >= M.lo[k] && f[k] <= M.hi[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < NPR; ++k) f[k] = (f[k] - M.xmean[k]) * M.xinv[k];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k >> 3][k & 7] = (__bf16)(k < NPR ? f[k < NPR ? k : 0] : 0.0f);
+  return out ? __uint_as_float(OUT_OF_RANGE) : quad_baseline<NPR>(M, f);
+}
+
+// The description (a kernel's first argument), read again where it is used: kept over a kernel's
+// loop its numbers would be spilled.
+PVD_DEV const MlpNet& cold_net() {
+  typedef const __attribute__((address_space(4))) MlpNet Cold;
+  Cold* cold = (Cold*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(cold));
+  return *(const MlpNet*)cold;
+}
+
 template <typename R, int NP, int H>
-__global__ __launch_bounds__(64 * E_WAVES, 2) void k_mlp_energy(MlpNet M, const R* planes, long long stride, const int* n_dev,
-                                                       long long n_fix, double* V) {
+__global__ __launch_bounds__(64 * E_WAVES, 4) void k_mlp_energy(MlpNet M, const R* planes, long long stride,
+                                                                const int* n_dev, long long n_fix, double* V) {
   extern __shared__ bf16x8 lds[];
-  constexpr int MT = H / 16, KC = H / 32;
+  constexpr int MT = H / 16, KC = H / 32, NPR = NP / 3 * (NP / 3 - 1) / 2;
   bf16x8* L0 = lds;
   bf16x8* L1 = L0 + MT * 64;
   bf16x8* L2 = L1 + MT * KC * 64;
@@ -729,237 +782,274 @@ __global__ __launch_bounds__(64 * E_WAVES, 2) void k_mlp_energy(MlpNet M, const 
   if (threadIdx.x == 0) lb[4 * H] = M.b3[0];
   __syncthreads();
   const int n = n_dev ? *n_dev : (int)n_fix;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, col = lane & 15;
-  constexpr long long CHUNK = (long long)E_WAVES * 16 * NT_E;
-  for (long long c0 = (long long)blockIdx.x * CHUNK; c0 < n; c0 += (long long)gridDim.x * CHUNK) {
-    // compiler-only barrier: the weight fragments are re-read from LDS each chunk instead of
-    // being hoisted out of the loop into (spilled) registers
+  constexpr int TILE_E = 16 * NT_E;
+  static_assert(TILE_E == 32, "two tiles to a batch of descriptors");
+  const int tiles = (int)(((long long)n + TILE_E - 1) / TILE_E), nw = gridDim.x * E_WAVES;
+  // neighbouring ranges go to different workgroups: where the tiles do not divide by the waves, the
+  // longer ranges are spread over the chip
+  const int wid = wave * gridDim.x + blockIdx.x;
+  const int t0 = (int)((long long)tiles * wid / nw), t1 = (int)((long long)tiles * (wid + 1) / nw);
+  for (int tb = t0; tb < t1; tb += 2) {
+    // compiler-only barrier: the weight fragments are re-read from LDS instead of being hoisted out
+    // of the loop into (spilled) registers
     asm volatile("" ::: "memory");
-    const long long base = c0 + (long long)wave * 16 * NT_E;
-    constexpr int NPR = NP / 3 * (NP / 3 - 1) / 2;
-    bf16x8 bin0[NT_E][1];
-    bf16x8 bin[NT_E][KC];
-    bool fbk[NT_E];
-    float qb[NT_E];
-#pragma unroll
-    for (int t = 0; t < NT_E; ++t) {
-      const long long w = base + t * 16 + col;
-      const bool ok = w < n;
-      float f[MLP_MAXP];
+    bf16x8 fw[2];
+    float qb;
+    {
+      const long long w = (long long)tb * TILE_E + lane;
       R x[NP];
 #pragma unroll
-      for (int p = 0; p < NP; ++p) x[p] = ok ? planes[p * stride + w] : R(0);
-      mlp_descriptor<R, NP>(M, x, f);
-      bool out = false;
-      if (M.use_range) {
-#pragma unroll
-        for (int k = 0; k < NPR; ++k) out |= !(f[k] >= M.lo[k] && f[k] <= M.hi[k]);
-      }
-      fbk[t] = out;
-      bin0[t][0] = input_chunk<NPR>(M, f, g, ok);
-      qb[t] = 0.0f;
-      if (g == 0) {
-        float xn[NPR];
-#pragma unroll
-        for (int k = 0; k < NPR; ++k) xn[k] = (f[k] - M.xmean[k]) * M.xinv[k];
-        qb[t] = quad_baseline<NPR>(M, xn);
-      }
+      for (int p = 0; p < NP; ++p) x[p] = planes[p * stride + (w < n ? w : 0)];
+      qb = energy_features<R, NP>(cold_net(), x, fw, nullptr, 0);
     }
-    f32x4 acc[NT_E][MT];
-    float part[NT_E];
+#pragma unroll 1
+    for (int s = 0; s < 2 && tb + s < t1; ++s) {
+      bf16x8 bin0[NT_E], bin[NT_E][KC];
+      f32x4 acc[NT_E][MT];
 #pragma unroll
-    for (int layer = 0; layer < 3; ++layer) {
-      asm volatile("" ::: "memory");
-      const float* bl = lb + layer * H;
+      for (int t = 0; t < NT_E; ++t) {
+        const int from = 4 * (TILE_E * s + 16 * t + col);
+        int d[4];
+        int4 w0 = __builtin_bit_cast(int4, fw[0]), w1 = __builtin_bit_cast(int4, fw[1]);
+        const int a0[4] = {w0.x, w0.y, w0.z, w0.w}, a1[4] = {w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const f32x4 bias = *(const f32x4*)(bl + 16 * m + 4 * g);
-        if (layer == 0) {
-          const bf16x8 a = L0[m * 64 + lane];
+        for (int k = 0; k < 4; ++k) {
+          const int u0 = 2 * k < NPR ? __builtin_amdgcn_ds_bpermute(from, a0[k]) : 0;
+          const int u1 = 8 + 2 * k < NPR ? __builtin_amdgcn_ds_bpermute(from, a1[k]) : 0;
+          d[k] = g == 0 ? u0 : g == 1 ? u1 : 0;
+        }
+        bin0[t] = __builtin_bit_cast(bf16x8, int4{d[0], d[1], d[2], d[3]});
+      }
 #pragma unroll
-          for (int t = 0; t < NT_E; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bin0[t][0], bias, 0, 0, 0);
-        } else {
-          const bf16x8* Wl = layer == 1 ? L1 : L2;
+      for (int layer = 0; layer < 3; ++layer) {
+        asm volatile("" ::: "memory");
+        const float* bl = lb + layer * H;
 #pragma unroll
-          for (int c = 0; c < KC; ++c) {
-            const bf16x8 a = Wl[(m * KC + c) * 64 + lane];
+        for (int m = 0; m < MT; ++m) {
+          const f32x4 bias = *(const f32x4*)(bl + 16 * m + 4 * g);
+          if (layer == 0) {
+            const bf16x8 a = L0[m * 64 + lane];
 #pragma unroll
-            for (int t = 0; t < NT_E; ++t)
-              acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bin[t][c], c == 0 ? bias : acc[t][m], 0, 0, 0);
+            for (int t = 0; t < NT_E; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bin0[t], bias, 0, 0, 0);
+          } else {
+            const bf16x8* Wl = layer == 1 ? L1 : L2;
+#pragma unroll
+            for (int c = 0; c < KC; ++c) {
+              const bf16x8 a = Wl[(m * KC + c) * 64 + lane];
+#pragma unroll
+              for (int t = 0; t < NT_E; ++t)
+                acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bin[t][c], c == 0 ? bias : acc[t][m], 0, 0, 0);
+            }
           }
         }
-      }
-      if (layer < 2) {
+        if (layer < 2) {
 #pragma unroll
-        for (int t = 0; t < NT_E; ++t)
+          for (int t = 0; t < NT_E; ++t)
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
+            for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)silu_f(acc[t][m][i]);
-      } else {
-#pragma unroll
-        for (int t = 0; t < NT_E; ++t) {
-          float s = 0.0f;
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            const f32x4 w3 = *(const f32x4*)(lb + 3 * H + 16 * m + 4 * g);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s += w3[i] * silu_f(acc[t][m][i]);
-          }
-          part[t] = s;
+              for (int i = 0; i < 4; ++i) bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)silu_f(acc[t][m][i]);
         }
       }
-    }
-    const float b3 = lb[4 * H];
+      const float b3 = lb[4 * H];
 #pragma unroll
-    for (int t = 0; t < NT_E; ++t) {
-      float s = part[t];
-      s += __shfl_xor(s, 16, 64);
-      s += __shfl_xor(s, 32, 64);
-      const long long w = base + t * 16 + col;
-      if (g == 0 && w < n) {
-        const float y = s + b3;
-        V[w] = fbk[t] ? __longlong_as_double((long long)FALLBACK_MARK) : (double)(y * M.ystd + M.ymean + qb[t]);
+      for (int t = 0; t < NT_E; ++t) {
+        float s3 = 0.0f;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const f32x4 w3 = *(const f32x4*)(lb + 3 * H + 16 * m + 4 * g);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s3 += w3[i] * silu_f(acc[t][m][i]);
+        }
+        s3 += __shfl_xor(s3, 16, 64);
+        s3 += __shfl_xor(s3, 32, 64);
+        const int r = TILE_E * s + 16 * t + col;
+        const float q = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * r, __float_as_int(qb)));
+        const long long w = (long long)tb * TILE_E + r;
+        if (g == 0 && w < n) {
+          const float y = s3 + b3;
+          V[w] = __float_as_uint(q) == OUT_OF_RANGE ? __longlong_as_double((long long)FALLBACK_MARK)
+                                                    : (double)(y * M.ystd + M.ymean + q);
+        }
       }
     }
   }
 }
 
-// Inference on walkers when the two hidden-layer packs do not fit LDS together (H = 256:
-// 128 KB each).  Persistent workgroups of E_WAVES waves keep layer 0's pack, the biases and
-// the output weights in LDS for the whole launch, and stage the packs of layers 1 and 2 in
-// turn through one slot, once per chunk of WV x 16 x NTS walkers (the packs come from L2;
-// the chunk's activations stay in registers between the layers).
-template <int H>
-constexpr size_t staged_lds_bytes() {
-  return (size_t)((H / 16) * 64 + (H / 16) * (H / 32) * 64) * 16 + (size_t)(4 * H + 4) * 4;
-}
+// Inference on walkers, H = 256, where the packs of two hidden layers do not fit LDS together.
+// Wave w of a workgroup keeps its 32 output units of both hidden layers in registers for the
+// whole launch (128 registers), so no weight is read again; what travels through LDS are the
+// activations (bf16, 512 bytes a walker and layer, read by every wave).  A tile of 32 walkers
+// passes layer 0, layer 1, layer 2 and the output in successive rounds of one barrier each; a round
+// works on four tiles at once, one per layer, so that the SiLUs of one layer cover the matrix
+// products of another.  The descriptors of 512 walkers are computed at a time, one thread each.
+// A layer's D registers of unit tiles 2w and 2w + 1 are word 4w + g of a walker's row: the next
+// layer's B operand of input chunk w, lane group g (phys_unit).  Every sum has the order of the
+// H = 128 kernel, the output's included: its 64 products a lane group go through LDS.
+// Six atoms, 1 000 000 walkers FP32: 878 us when the packs were staged through LDS for every 128
+// walkers, 410 now (0.65 PFLOP/s): VALU issue 66 % of the time, matrix cores 28 %, LDS 30 %.  With H = 128
+// it is slower than the kernel above (six atoms, 200 000 walkers FP64: 71 us against 60).
+template <int NP, int H>
+struct EnergyShape {
+  static constexpr int NPR = NP / 3 * (NP / 3 - 1) / 2;
+  static constexpr int NW = H / 32, NTH = 64 * NW, BT = NTH / 32;  // waves, threads, tiles per descriptor batch
+  static constexpr int FW = NPR > 8 ? 2 : 1;                        // 16-byte words of a walker's features
+  static constexpr int ROW = H / 8 + 1, PROW = H + 4;               // padded rows: activations (words), products (floats)
+  static constexpr size_t words = 4 * 32 * (size_t)ROW + FW * NTH;
+  static constexpr size_t floats = 2 * NTH + 2 * 32 * PROW + 4 * H;
+  static constexpr size_t lds = words * 16 + floats * 4;
+  static_assert(H == 256, "one workgroup of eight waves a CU");
+};
 
-template <typename R, int NP, int H, int NTS, int WV>
-__global__ __launch_bounds__(64 * WV, 1) void k_mlp_energy_st(MlpNet M, const R* planes, long long stride,
-                                                                  const int* n_dev, long long n_fix, double* V) {
+template <typename R, int NP, int H>
+__global__ __launch_bounds__(2 * H, 2) void k_mlp_energy_reg(
+    MlpNet M, const R* planes, long long stride, const int* n_dev, long long n_fix, double* V) {
+  using S = EnergyShape<NP, H>;
+  constexpr int KC = H / 32, MT = H / 16, NPR = S::NPR;
   extern __shared__ bf16x8 lds[];
-  constexpr int MT = H / 16, KC = H / 32, NTH = 64 * WV;
-  bf16x8* L0 = lds;
-  bf16x8* LW = L0 + MT * 64;
-  float* lb = (float*)(LW + MT * KC * 64);  // b0 | b1 | b2 | w3 | b3
-  for (int q = threadIdx.x; q < MT * 64; q += NTH) L0[q] = M.Wf[0][q];
-  for (int q = threadIdx.x; q < H; q += NTH) {
+  bf16x8* act1 = lds;                                  // [2][32][ROW]
+  bf16x8* act2 = act1 + 2 * 32 * S::ROW;               // [2][32][ROW]
+  bf16x8* feat = act2 + 2 * 32 * S::ROW;               // [NTH][FW]
+  float* s_q = (float*)(feat + S::FW * S::NTH);        // [2][NTH] baseline, or OUT_OF_RANGE
+  float* s_prod = s_q + 2 * S::NTH;                    // [2][32][PROW] w3 times the last layer's activations
+  float* lb = s_prod + 2 * 32 * S::PROW;               // b0 | b1 | b2 | w3
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, col = lane & 15;
+  const int n = n_dev ? *n_dev : (int)n_fix;
+  const int tiles = (int)(((long long)n + 31) / 32);
+  const int t0 = (int)((long long)tiles * blockIdx.x / gridDim.x);
+  const int nt = (int)((long long)tiles * (blockIdx.x + 1) / gridDim.x) - t0;
+  if (nt == 0) return;
+  bf16x8 W0[2], W1[2][KC], W2[2][KC];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    W0[m] = M.Wf[0][(2 * wv + m) * 64 + lane];
+#pragma unroll
+    for (int c = 0; c < KC; ++c) {
+      W1[m][c] = M.Wf[1][((2 * wv + m) * KC + c) * 64 + lane];
+      W2[m][c] = M.Wf[2][((2 * wv + m) * KC + c) * 64 + lane];
+    }
+  }
+  for (int q = tid; q < H; q += S::NTH) {
     lb[q] = M.b[0][q];
     lb[H + q] = M.b[1][q];
     lb[2 * H + q] = M.b[2][q];
     lb[3 * H + q] = M.w3[q];
   }
-  if (threadIdx.x == 0) lb[4 * H] = M.b3[0];
-  __syncthreads();
-  const int n = n_dev ? *n_dev : (int)n_fix;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, col = lane & 15;
-  constexpr long long CHUNK = (long long)WV * 16 * NTS;
-  // the loop bounds depend on the workgroup only: every wave meets every barrier
-  for (long long c0 = (long long)blockIdx.x * CHUNK; c0 < n; c0 += (long long)gridDim.x * CHUNK) {
-    asm volatile("" ::: "memory");
-    const long long base = c0 + (long long)wave * 16 * NTS;
-    constexpr int NPR = NP / 3 * (NP / 3 - 1) / 2;
-    bf16x8 bin0[NTS][1];
-    bf16x8 bin[NTS][KC];
-    bool fbk[NTS];
-    float qb[NTS];
+  const float b3 = M.b3[0];
+  auto descriptors = [&](int batch) {
+    const long long w = 32ll * t0 + (long long)batch * S::NTH + tid;
+    R x[NP];
 #pragma unroll
-    for (int t = 0; t < NTS; ++t) {
-      const long long w = base + t * 16 + col;
-      const bool ok = w < n;
-      float f[MLP_MAXP];
-      R x[NP];
+    for (int p = 0; p < NP; ++p) x[p] = planes[p * stride + (w < n ? w : 0)];
+    // scratch: the products' area that this round writes, which nobody reads any more
+    static_assert(NPR * S::NTH <= 32 * S::PROW, "scratch");
+    float* scratch = s_prod + 32 * (batch * S::BT & 1) * S::PROW + tid;
+    bf16x8 v[2];
+    s_q[(batch & 1) * S::NTH + tid] = energy_features<R, NP>(cold_net(), x, v, NP == 18 ? scratch : nullptr, S::NTH);
 #pragma unroll
-      for (int p = 0; p < NP; ++p) x[p] = ok ? planes[p * stride + w] : R(0);
-      mlp_descriptor<R, NP>(M, x, f);
-      bool out = false;
-      if (M.use_range) {
-#pragma unroll
-        for (int k = 0; k < NPR; ++k) out |= !(f[k] >= M.lo[k] && f[k] <= M.hi[k]);
-      }
-      fbk[t] = out;
-      bin0[t][0] = input_chunk<NPR>(M, f, g, ok);
-      qb[t] = 0.0f;
-      if (g == 0) {
-        float xn[NPR];
-#pragma unroll
-        for (int k = 0; k < NPR; ++k) xn[k] = (f[k] - M.xmean[k]) * M.xinv[k];
-        qb[t] = quad_baseline<NPR>(M, xn);
-      }
+    for (int k = 0; k < S::FW; ++k) feat[S::FW * tid + k] = v[k];
+  };
+  // four units 16(2 wv + m) + 4g + i of a bias or output weight vector
+  auto units = [&](const float* b, int m) { return *(const f32x4*)(b + 32 * wv + 16 * m + 4 * g); };
+  // rounds past the last tile only drain the layers behind it (what the first layers make of old
+  // rows is read by nobody)
+  for (int it = 0; it < nt + 3; ++it) {
+    if (it % S::BT == 0 && it < nt) {
+      descriptors(it / S::BT);
+      __syncthreads();
     }
-    f32x4 acc[NTS][MT];
-    float part[NTS];
-    // layer 0 from the resident pack
+    const int cur = it & 1, old = cur ^ 1;
+    // output of tile it - 3, one wave of each SIMD, the two in turn: lane l sums the units of group l / 8, in
+    // the order of the units, then the groups are added.  First in the round: at its end the other
+    // waves would wait for this chain of additions
+    if (it >= 3 && wv >> 2 == (it & (S::NW / 4 - 1)) && lane < 32) {
+      const int t = it - 3, r = 8 * (wv & 3) + (lane & 7);
+      const long long w = 32ll * (t0 + t) + r;
+      const float* p = s_prod + (32 * old + r) * S::PROW + 4 * (lane >> 3);
+      const float qb = s_q[t % (2 * S::BT) * 32 + r];
+      f32x4 v[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const f32x4 bias = *(const f32x4*)(lb + 16 * m + 4 * g);
-      const bf16x8 a = L0[m * 64 + lane];
-#pragma unroll
-      for (int t = 0; t < NTS; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bin0[t][0], bias, 0, 0, 0);
-    }
-#pragma unroll
-    for (int t = 0; t < NTS; ++t)
+      for (int m = 0; m < MT; ++m) v[m] = *(const f32x4*)(p + 16 * m);
+      float s = 0.0f;
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)silu_f(acc[t][m][i]);
-    // layers 1 and 2 through the staging slot
-#pragma unroll
-    for (int layer = 1; layer < 3; ++layer) {
-      __syncthreads();  // every wave is done with the slot
-      const bf16x8* src = M.Wf[layer];
-      for (int q = threadIdx.x; q < MT * KC * 64; q += NTH) LW[q] = src[q];
-      __syncthreads();
-      const float* bl = lb + layer * H;
-      // input chunk outer, output tile inner: consecutive MFMAs write different
-      // accumulators, so none waits on the previous one's result
-#pragma unroll
-      for (int c = 0; c < KC; ++c) {
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          const bf16x8 a = LW[(m * KC + c) * 64 + lane];
-#pragma unroll
-          for (int t = 0; t < NTS; ++t)
-            acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                a, bin[t][c], c == 0 ? *(const f32x4*)(bl + 16 * m + 4 * g) : acc[t][m], 0, 0, 0);
-        }
-      }
-      if (layer == 1) {
-#pragma unroll
-        for (int t = 0; t < NTS; ++t)
-#pragma unroll
-          for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)silu_f(acc[t][m][i]);
-      } else {
-#pragma unroll
-        for (int t = 0; t < NTS; ++t) {
-          float s = 0.0f;
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            const f32x4 w3 = *(const f32x4*)(lb + 3 * H + 16 * m + 4 * g);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s += w3[i] * silu_f(acc[t][m][i]);
-          }
-          part[t] = s;
-        }
-      }
-    }
-    const float b3 = lb[4 * H];
-#pragma unroll
-    for (int t = 0; t < NTS; ++t) {
-      float s = part[t];
+        for (int i = 0; i < 4; ++i) s += v[m][i];
+      s += __shfl_xor(s, 8, 64);
       s += __shfl_xor(s, 16, 64);
-      s += __shfl_xor(s, 32, 64);
-      const long long w = base + t * 16 + col;
-      if (g == 0 && w < n) {
-        const float y = s + b3;
-        V[w] = fbk[t] ? __longlong_as_double((long long)FALLBACK_MARK) : (double)(y * M.ystd + M.ymean + qb[t]);
+      const float y = s + b3;
+      if (lane < 8 && w < n)
+        V[w] = __float_as_uint(qb) == OUT_OF_RANGE ? __longlong_as_double((long long)FALLBACK_MARK)
+                                                   : (double)(y * M.ystd + M.ymean + qb);
+    }
+    // layer 0 of tile it, layer 1 of tile it - 1, layer 2 of tile it - 2: the matrix instructions of
+    // layers 1 and 2 run between the SiLUs of the layer before (16 / KC to an input chunk's four),
+    // the input chunks are read AHEAD chunks before their use
+    constexpr int EL = 16 / KC, AHEAD = 2;
+    f32x4 z[3][2][2];
+    bf16x8 x[2 * KC][2], x0[2], u;
+    auto read = [&](int k) {
+      const bf16x8* rows = k < KC ? act1 + 32 * old * S::ROW : act2 + 32 * cur * S::ROW;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) x[k][t] = rows[(16 * t + col) * S::ROW + 4 * (k % KC) + g];
+    };
+    auto start = [&](int layer) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) z[layer][0][m] = z[layer][1][m] = units(lb + layer * H, m);
+    };
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      x0[t] = feat[S::FW * (it % S::BT * 32 + 16 * t + col) + (S::FW == 2 ? g & 1 : 0)];
+      if (g >= S::FW) x0[t] = bf16x8{};
+    }
+    start(0);
+    start(1);
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) read(k);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) z[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W0[m], x0[t], z[0][t][m], 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < 2 * KC; ++k) {
+      const int c = k % KC, l = 1 + k / KC;
+      if (k + AHEAD < 2 * KC) read(k + AHEAD);
+      if (k == KC - AHEAD) start(2);
+      float h[EL];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int t = q >> 1, m = q & 1;
+        z[l][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l == 1 ? W1[m][c] : W2[m][c], x[k][t], z[l][t][m], 0, 0, 0);
+#pragma unroll
+        for (int e = q * EL / 4; e < (q + 1) * EL / 4; ++e) {
+          const int o = EL * c + e;
+          h[e] = silu_f(z[l - 1][o >> 3][(o >> 2) & 1][o & 3]);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < EL; ++e) u[(EL * c + e) & 7] = (__bf16)h[e];
+      if (EL * (c + 1) % 8 == 0) {
+        bf16x8* out = l == 1 ? act1 + 32 * cur * S::ROW : act2 + 32 * old * S::ROW;
+        out[(16 * (EL * c / 8) + col) * S::ROW + 4 * wv + g] = u;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const f32x4 w3 = units(lb + 3 * H, m);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        f32x4 p;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = w3[i] * silu_f(z[2][t][m][i]);
+        *(f32x4*)(s_prod + (32 * cur + 16 * t + col) * S::PROW + 32 * wv + 16 * m + 4 * g) = p;
       }
     }
+    __syncthreads();
   }
 }
 
@@ -1031,39 +1121,24 @@ constexpr int NT_FWD = 2;
 template <typename R, int NP, int H>
 int launch_energy(const MlpNet& N, const void* planes, long long stride, const int* n_dev, long long n_max,
                   double* V, const PesParams& fb, hipStream_t st) {
+  int dev = 0, cus = 256;
+  MHIP(hipGetDevice(&dev));
+  MHIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   if constexpr (H == 128) {
-    // persistent: two workgroups per CU (LDS-bound), each looping over walker chunks
-    int dev = 0, cus = 256;
-    MHIP(hipGetDevice(&dev));
-    MHIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const long long chunks = (n_max + (long long)E_WAVES * 16 * NT_E - 1) / ((long long)E_WAVES * 16 * NT_E);
-    const unsigned grid = (unsigned)std::max(1ll, std::min(chunks, 2ll * cus));
+    // two workgroups per CU (LDS-bound)
+    const long long wgs = (n_max + 32 * E_WAVES - 1) / (32 * E_WAVES);
+    const unsigned grid = (unsigned)std::max(1ll, std::min(wgs, 2ll * cus));
     const size_t lds = energy_lds_bytes<H>();
     auto k = k_mlp_energy<R, NP, H>;
     MHIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, dim3(grid), dim3(64 * E_WAVES), lds, st, N, (const R*)planes, stride, n_dev, n_max, V);
-    MHIP(hipGetLastError());
-    if (N.use_range) {
-      const unsigned gf = (unsigned)std::max(1ll, std::min((n_max + 255) / 256, 4ll * cus));
-      hipLaunchKernelGGL((k_mlp_fallback<R, NP>), dim3(gf), dim3(256), 0, st, (const R*)planes, stride, n_dev, n_max,
-                         V, fb);
-      MHIP(hipGetLastError());
-    }
-    return 0;
   } else {
-  // H = 256: persistent, one workgroup per CU (LDS-bound), layers 1 and 2 staged per chunk
-  int dev = 0, cus = 256;
-  MHIP(hipGetDevice(&dev));
-  MHIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  // one 16-walker tile per wave, 8 waves: two tiles per wave at one wave per SIMD (no spills)
-  // measured 18.5 ms against 14.0 ms at 16M walkers (too little latency hiding)
-  constexpr int NTS = 1, WV = E_WAVES;
-  const long long chunks = (n_max + (long long)WV * 16 * NTS - 1) / ((long long)WV * 16 * NTS);
-  const unsigned grid = (unsigned)std::max(1ll, std::min(chunks, (long long)cus));
-  const size_t lds = staged_lds_bytes<H>();
-  auto k = k_mlp_energy_st<R, NP, H, NTS, WV>;
-  MHIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * WV), lds, st, N, (const R*)planes, stride, n_dev, n_max, V);
+    using S = EnergyShape<NP, H>;
+    const unsigned grid = (unsigned)std::max(1ll, std::min((n_max + 31) / 32, (long long)cus));
+    auto k = k_mlp_energy_reg<R, NP, H>;
+    MHIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::lds));
+    hipLaunchKernelGGL(k, dim3(grid), dim3(S::NTH), S::lds, st, N, (const R*)planes, stride, n_dev, n_max, V);
+  }
   MHIP(hipGetLastError());
   if (N.use_range) {
     const unsigned gf = (unsigned)std::max(1ll, std::min((n_max + 255) / 256, 4ll * cus));
@@ -1072,7 +1147,6 @@ int launch_energy(const MlpNet& N, const void* planes, long long stride, const i
     MHIP(hipGetLastError());
   }
   return 0;
-  }
 }
 
 }  // namespace
