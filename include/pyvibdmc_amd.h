@@ -279,6 +279,9 @@ int pvd_mlp_grads_noalloc(const pvd_mlp* m, const float* x_t, const float* targe
 /* One Adam step (Kingma & Ba) with bias correction at step t >= 1. */
 int pvd_mlp_adam(float* params, float* m1, float* m2, const float* grads, int64_t size, float lr, float beta1,
                  float beta2, float eps, int64_t t, void* stream);
+/* The same step on m->params and then pvd_mlp_pack, in one pass over the parameters. */
+int pvd_mlp_adam_pack(const pvd_mlp* m, float* m1, float* m2, const float* grads, float lr, float beta1, float beta2,
+                      float eps, int64_t t, void* stream);
 /* Device view of the current walkers without a host sync: SoA planes, stride, and a
  * device pointer to the current population. */
 int pvd_sim_device_view(pvd_sim* sim, void** planes, int64_t* stride, int32_t** n_dev);

@@ -530,17 +530,24 @@ __global__ __launch_bounds__(256) void k_mlp_loss(long long n, const float* Y, c
   if (threadIdx.x == 0) parts[blockIdx.x] = e;
 }
 
-// Adam with bias correction on the flat FP32 parameter vector
-__global__ void k_adam(float* p, float* m, float* v, const float* g, long long size, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
+// Adam with bias correction: parameter p with moments m, v and gradient g after the step
+struct AdamStep {
+  float lr, b1, b2, eps, c1, c2;
+  PVD_DEV float operator()(float p, float& m, float& v, float g) const {
+    m = b1 * m + (1.0f - b1) * g;
+    v = b2 * v + (1.0f - b2) * g * g;
+    return p - lr * (m / c1) / (sqrtf(v / c2) + eps);
+  }
+};
+
+// on the flat FP32 parameter vector
+__global__ void k_adam(float* p, float* m, float* v, const float* g, long long size, AdamStep A) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= size) return;
-  const float gg = g[q];
-  const float mm = b1 * m[q] + (1.0f - b1) * gg;
-  const float vv = b2 * v[q] + (1.0f - b2) * gg * gg;
+  float mm = m[q], vv = v[q];
+  p[q] = A(p[q], mm, vv, g[q]);
   m[q] = mm;
   v[q] = vv;
-  p[q] = p[q] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
 }
 
 // FP32 master weights -> packed BF16 operands.  Forward pack of layer l (A = W_l):
@@ -570,6 +577,81 @@ __global__ void k_mlp_pack(const float* W, int rows, int cols, int in_natural, i
     v[j] = (__bf16)x;
   }
   out[q] = v;
+}
+
+// Adam and the repacked operands in one pass.  A thread takes a 4 x 4 block of a hidden layer (four
+// consecutive inputs, or four consecutive outputs, are 8 bytes of one pack word, so no store is
+// smaller), or a word of layer 0's pack, or one of the remaining parameters.  Bound by the launch:
+// 26 us a step as Adam and five pack launches (H = 128), now 7.
+template <int H>
+__global__ __launch_bounds__(64) void k_adam_pack(int D, float* p, float* m, float* v, const float* g, AdamStep A,
+                                                  bf16x8* packs) {
+  constexpr int MT = H / 16, KC = H / 32, BLK = H / 4;
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+  const int HH = H * H, w1 = H * D + H;  // offset of W1; W2 follows at HH + H
+  bf16x8* hidden = packs + MT * 64;
+  int q = blockIdx.x * 64 + threadIdx.x;
+  if (q < 2 * BLK * BLK) {
+    const int layer = q / (BLK * BLK), o0 = q / BLK % BLK * 4, i0 = q % BLK * 4;
+    const long long at = w1 + layer * (HH + H) + (long long)o0 * H + i0;
+    f32x4 P[4], Mo[4], Vo[4], G[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      P[a] = *(const f32x4*)(p + at + a * H);
+      Mo[a] = *(const f32x4*)(m + at + a * H);
+      Vo[a] = *(const f32x4*)(v + at + a * H);
+      G[a] = *(const f32x4*)(g + at + a * H);
+    }
+    bf16x4 row[4], col[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        float mm = Mo[a][b], vv = Vo[a][b];
+        P[a][b] = A(P[a][b], mm, vv, G[a][b]);
+        Mo[a][b] = mm;
+        Vo[a][b] = vv;
+        row[a][b] = col[b][a] = (__bf16)P[a][b];
+      }
+      *(f32x4*)(p + at + a * H) = P[a];
+      *(f32x4*)(m + at + a * H) = Mo[a];
+      *(f32x4*)(v + at + a * H) = Vo[a];
+    }
+    // units k0 .. k0 + 3 of row r: half (k0 / 16) % 2 of word (r / 16, k0 / 32), lane 16 (k0 / 4 % 4) + r % 16
+    auto half = [&](bf16x8* pack, int r, int k0) {
+      bf16x8* w = pack + ((r >> 4) * KC + (k0 >> 5)) * 64 + 16 * ((k0 >> 2) & 3) + (r & 15);
+      return (bf16x4*)w + ((k0 >> 4) & 1);
+    };
+    bf16x8* fwd = hidden + layer * MT * KC * 64;
+    bf16x8* tr = hidden + (2 + layer) * MT * KC * 64;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      *half(fwd, o0 + a, i0) = row[a];
+      *half(tr, i0 + a, o0) = col[a];
+    }
+    return;
+  }
+  q -= 2 * BLK * BLK;
+  auto one = [&](long long k) {
+    float mm = m[k], vv = v[k];
+    const float x = A(p[k], mm, vv, g[k]);
+    p[k] = x;
+    m[k] = mm;
+    v[k] = vv;
+    return x;
+  };
+  if (q < MT * 64) {  // layer 0: units in natural order, zeros beyond D
+    const int lane = q & 63, r = 16 * (q >> 6) + (lane & 15), k0 = 8 * (lane >> 4);
+    bf16x8 w;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = (__bf16)(k0 + j < D ? one((long long)r * D + k0 + j) : 0.0f);
+    packs[q] = w;
+    return;
+  }
+  q -= MT * 64;
+  if (q < H) one((long long)H * D + q);             // b0
+  else if (q < 2 * H) one(w1 + HH + q - H);         // b1
+  else if (q < 4 * H + 1) one(w1 + 2ll * HH + q - H);  // b2, w3, b3
 }
 
 // descriptors of AoS walkers (n, M, 3) -> raw features F^T (D x n), float32
@@ -1399,9 +1481,29 @@ extern "C" {
 int pvd_mlp_adam(float* params, float* m1, float* m2, const float* grads, int64_t size, float lr, float beta1,
                  float beta2, float eps, int64_t t, void* stream) {
   if (!params || !m1 || !m2 || !grads || size <= 0 || t <= 0) return mfail(7, "bad arguments");
-  const float c1 = 1.0f - powf(beta1, (float)t), c2 = 1.0f - powf(beta2, (float)t);
+  const AdamStep A{lr, beta1, beta2, eps, 1.0f - powf(beta1, (float)t), 1.0f - powf(beta2, (float)t)};
   hipLaunchKernelGGL(k_adam, dim3((unsigned)((size + 255) / 256)), dim3(256), 0, (hipStream_t)stream, params, m1, m2,
-                     grads, (long long)size, lr, beta1, beta2, eps, c1, c2);
+                     grads, (long long)size, A);
+  MHIP(hipGetLastError());
+  return 0;
+}
+
+int pvd_mlp_adam_pack(const pvd_mlp* m, float* m1, float* m2, const float* grads, float lr, float beta1, float beta2,
+                      float eps, int64_t t, void* stream) {
+  if (!m || !m->params || !m->packs || !m1 || !m2 || !grads || t <= 0) return mfail(7, "bad arguments");
+  const int D = m->D, H = m->H;
+  if (D < 1 || D > 32 || (H != 128 && H != 256)) return mfail(7, "hidden width must be 128 or 256");
+  float* p = const_cast<float*>(m->params);
+  // the one-pass kernel reads four parameters at a time
+  if (((uintptr_t)p | (uintptr_t)m1 | (uintptr_t)m2 | (uintptr_t)grads | (uintptr_t)m->packs) & 15) {
+    const int rc = pvd_mlp_adam(p, m1, m2, grads, pvd_mlp_param_count(D, H), lr, beta1, beta2, eps, t, stream);
+    return rc ? rc : pvd_mlp_pack(m, stream);
+  }
+  const AdamStep A{lr, beta1, beta2, eps, 1.0f - powf(beta1, (float)t), 1.0f - powf(beta2, (float)t)};
+  const int items = H * H / 8 + 4 * H + 4 * H + 1;
+  auto k = H == 128 ? k_adam_pack<128> : k_adam_pack<256>;
+  hipLaunchKernelGGL(k, dim3((unsigned)((items + 63) / 64)), dim3(64), 0, (hipStream_t)stream, D, p, m1, m2, grads, A,
+                     (bf16x8*)m->packs);
   MHIP(hipGetLastError());
   return 0;
 }

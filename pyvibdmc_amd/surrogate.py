@@ -47,6 +47,8 @@ _MSIGS = {
     'pvd_mlp_noalloc_scratch_bytes': (ctypes.c_int64, []),
     'pvd_mlp_adam': (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_float, ctypes.c_float,
                                     ctypes.c_float, ctypes.c_float, ctypes.c_int64, _P]),
+    'pvd_mlp_adam_pack': (ctypes.c_int, [ctypes.POINTER(MLPDesc), _P, _P, _P, ctypes.c_float, ctypes.c_float,
+                                         ctypes.c_float, ctypes.c_float, ctypes.c_int64, _P]),
     'pvd_sim_device_view': (ctypes.c_int, [_P, ctypes.POINTER(_P), ctypes.POINTER(ctypes.c_int64),
                                            ctypes.POINTER(_P)]),
     'pvd_mlp_judge': (ctypes.c_int, [ctypes.POINTER(N.PesDesc), ctypes.c_int32, ctypes.c_int32, _P, ctypes.c_int64,
@@ -257,10 +259,14 @@ class SurrogateModel:
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.t += 1
-        _check(_lib().pvd_mlp_adam(self.params.data_ptr(), self.m1.data_ptr(), self.m2.data_ptr(),
-                                   self.grads.data_ptr(), self.params.numel(), lr, b1, b2, eps, self.t,
-                                   N.stream_handle()), 'pvd_mlp_adam')
-        self.repack()
+        if self.desc.params != self.params.data_ptr():  # replaced by the caller: the operands stay the description's
+            _check(_lib().pvd_mlp_adam(self.params.data_ptr(), self.m1.data_ptr(), self.m2.data_ptr(),
+                                       self.grads.data_ptr(), self.params.numel(), lr, b1, b2, eps, self.t,
+                                       N.stream_handle()), 'pvd_mlp_adam')
+            return self.repack()
+        _check(_lib().pvd_mlp_adam_pack(ctypes.byref(self.desc), self.m1.data_ptr(), self.m2.data_ptr(),
+                                        self.grads.data_ptr(), lr, b1, b2, eps, self.t, N.stream_handle()),
+               'pvd_mlp_adam_pack')
 
     def quad_design(self, xn):
         """Design matrix (n, 1 + D + D(D+1)/2) of the quadratic baseline on normalised

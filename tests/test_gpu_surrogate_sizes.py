@@ -71,3 +71,36 @@ def test_energy_sizes(elements, hidden, precision):
     np.testing.assert_allclose(mixed[out], pes(xd), rtol=0, atol=1e-6 if precision == 'fp32' else 1e-12)
     for k in sizes:
         np.testing.assert_array_equal(energy(k, 1), mixed[:k], err_msg=str(k))
+
+
+@pytest.mark.parametrize('features,hidden', [(1, 128), (3, 128), (15, 256), (32, 128), (32, 256), (17, 256)])
+@pytest.mark.parametrize('offset', [0, 1])
+def test_adam_pack_equals_adam_then_pack(features, hidden, offset):
+    """The one-pass update against pvd_mlp_adam and pvd_mlp_pack, bit for bit (the same operations),
+    from aligned buffers and from ones at an odd float (which take the two calls)."""
+    import ctypes
+    import torch
+    from pyvibdmc_amd import _native as N
+    from pyvibdmc_amd.surrogate import MLPDesc, _lib
+    lib = _lib()
+    size = int(lib.pvd_mlp_param_count(features, hidden))
+    g = torch.Generator().manual_seed(features * hidden)
+    base = [torch.randn(size + offset, generator=g), 1e-3 * torch.randn(size + offset, generator=g),
+            1e-6 * torch.rand(size + offset, generator=g), 1e-3 * torch.randn(size + offset, generator=g)]
+    results = []
+    for fused in (False, True):
+        p, m1, m2, gr = (b.cuda()[offset:] for b in base)
+        packs = torch.full((int(lib.pvd_mlp_pack_bytes(hidden)),), 0x5A, dtype=torch.uint8, device='cuda')
+        d = MLPDesc()
+        d.D, d.H, d.params, d.packs = features, hidden, p.data_ptr(), packs.data_ptr()
+        for t in (1, 2, 1000):
+            if fused:
+                rc = lib.pvd_mlp_adam_pack(ctypes.byref(d), m1.data_ptr(), m2.data_ptr(), gr.data_ptr(), 1e-3, 0.9, 0.999,
+                                           1e-8, t, N.stream_handle())
+            else:
+                rc = lib.pvd_mlp_adam(p.data_ptr(), m1.data_ptr(), m2.data_ptr(), gr.data_ptr(), size, 1e-3, 0.9, 0.999,
+                                      1e-8, t, N.stream_handle()) or lib.pvd_mlp_pack(ctypes.byref(d), N.stream_handle())
+            assert rc == 0
+        results.append([v.cpu() for v in (p, m1, m2, packs)])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
