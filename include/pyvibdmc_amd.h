@@ -266,6 +266,9 @@ int pvd_mlp_judge(const pvd_pes_desc* pes, int32_t precision, int32_t n_atoms, c
  * x_t (D x n) and targets (n); y_out (n) or NULL; loss_parts (ceil(n/256) doubles). */
 int pvd_mlp_grads(const pvd_mlp* m, const float* x_t, const float* targets, int64_t n, float* grads, float* y_out,
                   double* loss_parts, void* workspace, void* stream);
+/* pvd_mlp_grads and the loss itself (device, one double). */
+int pvd_mlp_loss_grads(const pvd_mlp* m, const float* x_t, const float* targets, int64_t n, float* grads, float* y_out,
+                       double* loss_parts, double* loss, void* workspace, void* stream);
 /* pvd_mlp_grads without a workspace argument and without any device allocation.  No
  * counterpart in the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, training loops that forbid hipMalloc).  The workspace is a static

@@ -212,322 +212,322 @@ PVD_DEV void mlp_descriptor(const MlpNet& M, const R* x, float* f, float* scratc
   for (int k = NPR; k < MLP_MAXP; ++k) f[k] = 0.0f;
 }
 
-// normalised features 8g..8g+7 of one walker as a B operand chunk (D = NPR features)
-template <int NPR>
-PVD_DEV bf16x8 input_chunk(const MlpNet& M, const float* f, int g, bool valid) {
-  float fn[NPR];
-#pragma unroll
-  for (int k = 0; k < NPR; ++k) fn[k] = (f[k] - M.xmean[k]) * M.xinv[k];
-  bf16x8 v;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    float s = 0.0f;
-#pragma unroll
-    for (int k = j; k < NPR; k += 8)
-      if (k == 8 * g + j) s = fn[k];
-    v[j] = (__bf16)(valid ? s : 0.0f);
-  }
-  return v;
-}
-
-// D(m) += sum_c A(m, c) B(c) for NT walker tiles; A read from LDS
-template <int NT, int MT, int KC>
-PVD_DEV void mfma_layer(const bf16x8* __restrict__ Wl, const bf16x8 (&bin)[NT][KC], f32x4 (&acc)[NT][MT], int lane) {
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // input chunk outer, output tile inner: consecutive MFMAs write different accumulators
-  // (each accumulator still sums its chunks in order c = 0, 1, ...)
-#pragma unroll
-  for (int c = 0; c < KC; ++c) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const bf16x8 a = Wl[(m * KC + c) * 64 + lane];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bin[t][c], acc[t][m], 0, 0, 0);
-    }
-  }
-}
-
-template <int N>
-PVD_DEV void stage(bf16x8* lds, const bf16x8* __restrict__ src, int words) {
-  __syncthreads();
-  for (int q = threadIdx.x; q < words; q += N) lds[q] = src[q];
-  __syncthreads();
-}
-
 // ------------------------------------------------------------------------------------
-// Network forward.  MODE 0: inference on walkers (SoA planes of R) -> V (double), with the
-// analytic fallback outside the training range.  MODE 1: training forward on normalised
-// descriptors X^T (D x B) -> pre-activations Z^T (3 x H x B) and y (B).
-template <typename R, int NP, int H, int NT, int MODE>
-__global__ __launch_bounds__(256) void k_mlp_forward(MlpNet M, const R* planes, long long stride,
-                                                     const int* n_dev, long long n_fix, double* V, PesParams fb,
-                                                     const float* XT, float* ZT, float* Y) {
-  extern __shared__ bf16x8 lds[];
-  constexpr int MT = H / 16, KC = H / 32;
-  const int n = n_dev ? *n_dev : (int)n_fix;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Training: forward and backward of a batch (k_mlp_fwd_bwd), the weight gradients from the BF16
+// operands that it leaves (k_mlp_wgrad), and the sums of both kernels' parts (k_mlp_collect).
+
+// What the three kernels share.  Batch element b of row u at [u * np + b], np = n rounded up to 32.
+struct TrainBuf {
+  __bf16* h[2];   // silu(z_0), silu(z_1)
+  __bf16* dz[3];  // dL/dz_l
+  float* Y;       // network outputs
+  float* B;       // per 32 batch elements: sums of dz_0, dz_1, dz_2, dy h_2 (H each), dy
+  float* P;       // per batch slice: W0, W1, W2 gradients
+  const float* XT;
+  const float* T;
+  long long n, np;
+};
+
+template <int H>
+constexpr int train_slice() { return H == 256 ? 512 : 256; }  // batch elements of a weight gradient part
+
+// One workgroup takes 32 batch elements through all layers and back.  Wave w owns units 32w to
+// 32w + 31 of every layer: their pre-activations stay in its registers for the backward pass, its
+// share of the four packs is read once, a layer ahead, and only the BF16 operands of the next
+// product travel through LDS.  Lane (g, col) holds elements 2 col and 2 col + 1 of the 32 (walker
+// tiles t = 0, 1), so that its two values of a unit are one 4-byte store.
+// Bound by the latency of the chain of seven products and their barriers: 8192 elements are 256
+// workgroups, one to a CU.
+template <int H>
+__global__ __launch_bounds__(2 * H, H == 256 ? 2 : 1) void k_mlp_fwd_bwd(MlpNet M, TrainBuf D) {
+  constexpr int KC = H / 32, MT = H / 16, ROW = H / 8 + 1, PROW = H + 4;
+  __shared__ bf16x8 s_act[2][32 * ROW];
+  __shared__ __align__(16) float s_prod[32 * PROW];
+  __shared__ float s_dy[32];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, col = lane & 15;
-  const long long base = ((long long)blockIdx.x * 4 + wave) * (16 * NT);
-  if ((long long)blockIdx.x * 4 * 16 * NT >= n) return;  // whole block past the end
-  bf16x8 bin0[NT][1];
-  bf16x8 bin[NT][KC];
-  bool fbk[NT];
-  double vfb[NT];
-  float qb[NT];
+  const long long base = 32ll * blockIdx.x, n = D.n, np = D.np;
+  const long long w0 = base + 2 * col;
+  const bool ok[2] = {w0 < n, w0 + 1 < n};
+  auto unit = [&](int m, int i) { return 32 * wv + 16 * m + 4 * g + i; };
+  bf16x8 Wa[2][KC], Wb[2][KC];
+  auto weights = [&](bf16x8 (&W)[2][KC], const bf16x8* pack) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const long long w = base + t * 16 + col;
-    const bool ok = w < n;
-    fbk[t] = false;
-    vfb[t] = 0.0;
-    qb[t] = 0.0f;
-    if constexpr (MODE == 0) {
-      float f[MLP_MAXP];
-      R x[NP];
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int p = 0; p < NP; ++p) x[p] = ok ? planes[p * stride + w] : R(0);
-      mlp_descriptor<R, NP>(M, x, f);
-      if (ok && M.use_range) {
-        bool out = false;
+      for (int c = 0; c < KC; ++c) W[m][c] = pack[((2 * wv + m) * KC + c) * 64 + lane];
+  };
+  f32x4 b[3][2], w3[2];
 #pragma unroll
-        for (int k = 0; k < MLP_MAXP; ++k)
-          if (k < M.D) out |= !(f[k] >= M.lo[k] && f[k] <= M.hi[k]);
-        if (out) {
-          fbk[t] = true;
-          vfb[t] = (double)pes_eval<R, NP>(fb, x);
-        }
-      }
-      constexpr int NPR = NP / 3 * (NP / 3 - 1) / 2;
-      bin0[t][0] = input_chunk<NPR>(M, f, g, ok);
-      if (g == 0) {
-        float xn[NPR];
+  for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int k = 0; k < NPR; ++k) xn[k] = (f[k] - M.xmean[k]) * M.xinv[k];
-        qb[t] = quad_baseline<NPR>(M, xn);
-      }
-    } else {
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int l = 0; l < 3; ++l) b[l][m][i] = M.b[l][unit(m, i)];
+      w3[m][i] = M.w3[unit(m, i)];
+    }
+  weights(Wa, M.Wf[1]);
+  f32x4 z[3][2][2];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  {  // layer 0
+    bf16x8 W0[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) W0[m] = M.Wf[0][(2 * wv + m) * 64 + lane];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
       bf16x8 v;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int k = 8 * g + j;
-        v[j] = (__bf16)((ok && k < M.D) ? XT[(long long)k * n + w] : 0.0f);
+        v[j] = (__bf16)((ok[t] && k < M.D) ? D.XT[(long long)k * n + w0 + t] : 0.0f);
       }
-      bin0[t][0] = v;
+#pragma unroll
+      for (int m = 0; m < 2; ++m) z[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W0[m], v, zero, 0, 0, 0) + b[0][m];
     }
   }
-  f32x4 acc[NT][MT];
-  float part[NT];
-  // layer 0 (input chunk c = 0 in natural order)
-  stage<256>(lds, M.Wf[0], MT * 64);
-  mfma_layer<NT, MT, 1>(lds, bin0, acc, lane);
+  weights(Wb, M.Wf[2]);
+  // a pair of batch elements of every unit to the weight gradient's operands (zero past the batch),
+  // and both to the rows of the next product
+  auto publish = [&](const float (&x)[2][2][4], __bf16* to, bf16x8* rows) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    bf16x8 u[2];
 #pragma unroll
-  for (int layer = 0; layer < 3; ++layer) {
-    if (layer > 0) {
-      stage<256>(lds, M.Wf[layer], MT * KC * 64);
-      mfma_layer<NT, MT, KC>(lds, bin, acc, lane);
-    }
-    const float* bl = M.b[layer];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const long long w = base + t * 16 + col;
-      const bool ok = w < n;
-      if (layer == 2) part[t] = 0.0f;
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int u = 16 * m + 4 * g + i;
-          const float z = acc[t][m][i] + bl[u];
-          if constexpr (MODE == 1) {
-            if (ok) ZT[((long long)layer * H + u) * n + w] = z;
-          }
-          const float h = silu_f(z);
-          if (layer < 2) bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)h;
-          else part[t] += M.w3[u] * h;
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    float s = part[t];
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
-    const long long w = base + t * 16 + col;
-    if (g == 0 && w < n) {
-      const float y = s + M.b3[0];
-      if constexpr (MODE == 0) {
-        V[w] = fbk[t] ? vfb[t] : (double)(y * M.ystd + M.ymean + qb[t]);
-      } else {
-        Y[w] = y;
-      }
-    }
-  }
-}
-
-// Backward through the hidden layers for one batch: dZ_l^T = dL/dz_l (3 x H x B) from the
-// stored pre-activations and dy = dL/dy.  dh_{l-1} = W_l^T dz_l uses the transposed packs.
-template <int H, int NT>
-__global__ __launch_bounds__(256) void k_mlp_backward(MlpNet M, long long n, const float* ZT, const float* dY,
-                                                      float* DZT) {
-  extern __shared__ bf16x8 lds[];
-  constexpr int MT = H / 16, KC = H / 32;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, col = lane & 15;
-  const long long base = ((long long)blockIdx.x * 4 + wave) * (16 * NT);
-  if ((long long)blockIdx.x * 4 * 16 * NT >= n) return;
-  bf16x8 bin[NT][KC];
-  f32x4 acc[NT][MT];
-  // layer 2: dz2 = w3 * dy * silu'(z2)
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const long long w = base + t * 16 + col;
-    const bool ok = w < n;
-    const float dy = ok ? dY[w] : 0.0f;
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int u = 16 * m + 4 * g + i;
-        const float z = ok ? ZT[((long long)2 * H + u) * n + w] : 0.0f;
-        const float dz = M.w3[u] * dy * dsilu_f(z);
-        if (ok) DZT[((long long)2 * H + u) * n + w] = dz;
-        bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)dz;
-      }
-  }
+        bf16x2 v;
 #pragma unroll
-  for (int layer = 2; layer >= 1; --layer) {
-    stage<256>(lds, M.Wt[layer - 1], MT * KC * 64);
-    mfma_layer<NT, MT, KC>(lds, bin, acc, lane);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const long long w = base + t * 16 + col;
-      const bool ok = w < n;
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int u = 16 * m + 4 * g + i;
-          const float z = ok ? ZT[((long long)(layer - 1) * H + u) * n + w] : 0.0f;
-          const float dz = acc[t][m][i] * dsilu_f(z);
-          if (ok) DZT[((long long)(layer - 1) * H + u) * n + w] = dz;
-          bin[t][m >> 1][(m & 1) * 4 + i] = (__bf16)dz;
+        for (int t = 0; t < 2; ++t) {
+          u[t][4 * m + i] = (__bf16)x[t][m][i];
+          v[t] = ok[t] ? u[t][4 * m + i] : (__bf16)0.0f;
         }
+        if (to) *(bf16x2*)(to + unit(m, i) * np + w0) = v;
+      }
+    if (rows) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) rows[(16 * t + col) * ROW + 4 * wv + g] = u[t];
+    }
+  };
+  auto product = [&](const bf16x8 (&W)[2][KC], const bf16x8* rows, f32x4 (&a)[2][2]) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) a[0][m] = a[1][m] = zero;
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const bf16x8 x = rows[(16 * t + col) * ROW + 4 * c + g];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) a[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[m][c], x, a[t][m], 0, 0, 0);
+      }
+  };
+  float x[2][2][4];
+#define PVD_EACH(expr)                                  \
+  _Pragma("unroll") for (int t = 0; t < 2; ++t)         \
+      _Pragma("unroll") for (int m = 0; m < 2; ++m)     \
+          _Pragma("unroll") for (int i = 0; i < 4; ++i) expr
+  // layers 1 and 2
+  PVD_EACH(x[t][m][i] = silu_f(z[0][t][m][i]));
+  publish(x, D.h[0], s_act[0]);
+  __syncthreads();
+  product(Wa, s_act[0], z[1]);
+  weights(Wa, M.Wt[1]);
+  PVD_EACH(z[1][t][m][i] = z[1][t][m][i] + b[1][m][i]);
+  PVD_EACH(x[t][m][i] = silu_f(z[1][t][m][i]));
+  publish(x, D.h[1], s_act[1]);
+  __syncthreads();
+  product(Wb, s_act[1], z[2]);
+  weights(Wb, M.Wt[0]);
+  PVD_EACH(z[2][t][m][i] = z[2][t][m][i] + b[2][m][i]);
+  PVD_EACH(x[t][m][i] = silu_f(z[2][t][m][i]));
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      f32x4 p;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = w3[m][i] * x[t][m][i];
+      *(f32x4*)(s_prod + (16 * t + col) * PROW + 32 * wv + 16 * m + 4 * g) = p;
+    }
+  __syncthreads();
+  // the output: four lanes to an element sum a lane group's units each, in order; then the loss
+  if (tid < 128) {
+    const int r = tid >> 2;
+    const float* p = s_prod + r * PROW + 4 * (tid & 3);
+    float s = 0.0f;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const f32x4 v = *(const f32x4*)(p + 16 * m);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s += v[i];
+    }
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    const long long w = base + 2 * (r & 15) + (r >> 4);
+    if ((tid & 3) == 0) {
+      const float y = s + M.b3[0];
+      float dy = 0.0f;
+      if (w < n) {
+        const float e = y - D.T[w];
+        dy = 2.0f * e / (float)n;
+        D.Y[w] = y;
+      }
+      s_dy[r] = dy;
     }
   }
+  __syncthreads();
+  const float dy[2] = {s_dy[col], s_dy[16 + col]};
+  float* B = D.B + (long long)blockIdx.x * (4 * H + 1);
+  // sum of a unit's 32 elements (its 16 lanes, two each) into row k
+  auto rowsum = [&](const float (&v)[2][2][4], int k) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float s = v[0][m][i] + v[1][m][i];
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+        if (col == 0) B[k * H + unit(m, i)] = s;
+      }
+  };
+  PVD_EACH(x[t][m][i] = ok[t] ? dy[t] * x[t][m][i] : 0.0f);
+  rowsum(x, 3);
+  if (tid == 0) {
+    float s = 0.0f;
+    for (int r = 0; r < 32; ++r) s += s_dy[r];
+    B[4 * H] = s;
+  }
+  // back: dz_2, dz_1, dz_0
+  PVD_EACH(x[t][m][i] = ok[t] ? w3[m][i] * dy[t] * dsilu_f(z[2][t][m][i]) : 0.0f);
+  publish(x, D.dz[2], s_act[0]);
+  __syncthreads();
+  rowsum(x, 2);
+  f32x4 a[2][2];
+  product(Wa, s_act[0], a);
+  PVD_EACH(x[t][m][i] = ok[t] ? a[t][m][i] * dsilu_f(z[1][t][m][i]) : 0.0f);
+  publish(x, D.dz[1], s_act[1]);
+  __syncthreads();
+  rowsum(x, 1);
+  product(Wb, s_act[1], a);
+  PVD_EACH(x[t][m][i] = ok[t] ? a[t][m][i] * dsilu_f(z[0][t][m][i]) : 0.0f);
+  publish(x, D.dz[0], nullptr);
+  rowsum(x, 0);
+#undef PVD_EACH
 }
 
-// Weight gradient of layer l over a batch slice: P[split][o][i] = sum_b dz[o][b] * hin[i][b]
-// with hin = X (l = 0) or silu(z_{l-1}).  One wave per 32 x 32 output block.
-__global__ __launch_bounds__(64) void k_mlp_wgrad(int layer, int H, int Din, long long n, int kslice,
-                                                  const float* XT, const float* ZT, const float* DZT, float* P) {
-  const int lane = threadIdx.x;
-  const int g = lane >> 4, col = lane & 15;
-  const int ob = blockIdx.x * 32, ib = blockIdx.y * 32, split = blockIdx.z;
-  const long long k0 = (long long)split * kslice;
-  const long long k1 = k0 + kslice < n ? k0 + kslice : n;
-  const float* dz = DZT + (long long)layer * H * n;
-  const float* hz = layer == 0 ? XT : ZT + (long long)(layer - 1) * H * n;
-  f32x4 acc[2][2];
+// Weight gradients of a batch slice: P[o][i] = sum_b dz[o][b] hin[i][b].  A workgroup takes 64 x 64
+// of a hidden layer, a wave 32 x 32 of it, or 64 rows of layer 0 (16 a wave).  Both operands are
+// read as they lie, 16 bytes a lane; slices of 256 (H = 128) and 512 elements give 256 and 512
+// workgroups at 8192 elements.
+template <int H>
+__global__ __launch_bounds__(256) void k_mlp_wgrad(int Din, TrainBuf D) {
+  constexpr int TI = H / 64;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, col = lane & 15, tile = blockIdx.x;
+  const long long k0 = (long long)blockIdx.y * train_slice<H>();
+  const long long k1 = k0 + train_slice<H>() < D.np ? k0 + train_slice<H>() : D.np;
+  float* P = D.P + (long long)blockIdx.y * ((long long)H * Din + 2 * H * H);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (tile < 2 * TI * TI) {
+    const int l = 1 + tile / (TI * TI), ob = tile / TI % TI * 64 + 32 * (wv >> 1), ib = tile % TI * 64 + 32 * (wv & 1);
+    const __bf16* pa = D.dz[l] + (ob + col) * D.np + 8 * g;
+    const __bf16* pb = D.h[l - 1] + (ib + col) * D.np + 8 * g;
+    f32x4 acc[2][2];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+    for (int q = 0; q < 4; ++q) acc[q >> 1][q & 1] = zero;
+#pragma unroll 4
+    for (long long k = k0; k < k1; k += 32) {
+      bf16x8 A[2], Bv[2];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long long kb = k0; kb < k1; kb += 32) {
-    bf16x8 A[2], B[2];
+      for (int q = 0; q < 2; ++q) {
+        A[q] = *(const bf16x8*)(pa + 16 * q * D.np + k);
+        Bv[q] = *(const bf16x8*)(pb + 16 * q * D.np + k);
+      }
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const int o = ob + 16 * a + col;
+      for (int q = 0; q < 4; ++q)
+        acc[q >> 1][q & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[q >> 1], Bv[q & 1], acc[q >> 1][q & 1], 0, 0, 0);
+    }
+    float* out = P + (long long)H * Din + (l - 1) * H * H;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[(ob + 16 * (q >> 1) + 4 * g + i) * H + ib + 16 * (q & 1) + col] = acc[q >> 1][q & 1][i];
+    return;
+  }
+  const int ob = (tile - 2 * TI * TI) * 64 + 16 * wv;
+  const __bf16* pa = D.dz[0] + (ob + col) * D.np + 8 * g;
+  f32x4 acc[2] = {zero, zero};
+  for (long long k = k0; k < k1; k += 32) {
+    const bf16x8 A = *(const bf16x8*)(pa + k);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int u = 16 * q + col;
+      bf16x8 v;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const long long b = kb + 8 * g + j;
-        A[a][j] = (__bf16)((b < k1 && o < H) ? dz[(long long)o * n + b] : 0.0f);
+        const long long e = k + 8 * g + j;
+        v[j] = (__bf16)(u < Din && e < D.n ? D.XT[(long long)u * D.n + e] : 0.0f);
       }
-    }
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int i = ib + 16 * c + col;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const long long b = kb + 8 * g + j;
-        float h = 0.0f;
-        if (b < k1 && i < Din) {
-          const float v = hz[(long long)i * n + b];
-          h = layer == 0 ? v : silu_f(v);
-        }
-        B[c][j] = (__bf16)h;
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a], B[c], acc[a][c], 0, 0, 0);
-  }
-  const int Hin = layer == 0 ? Din : H;
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int o = ob + 16 * a + 4 * g + i4;
-        const int i = ib + 16 * c + col;
-        if (o < H && i < Hin) P[((long long)split * H + o) * Hin + i] = acc[a][c][i4];
-      }
-}
-
-// fixed-order sum of the split partials into the gradient vector
-__global__ void k_mlp_wgrad_reduce(const float* P, int splits, long long size, float* G) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= size) return;
-  float s = 0.0f;
-  for (int k = 0; k < splits; ++k) s += P[k * size + q];
-  G[q] = s;
-}
-
-// bias gradients and the output layer: one block per row, fixed-order reduction
-__global__ __launch_bounds__(256) void k_mlp_rowsum(int H, long long n, const float* ZT, const float* DZT,
-                                                    const float* dY, float* gb0, float* gb1, float* gb2, float* gw3,
-                                                    float* gb3) {
-  __shared__ float sh[4];
-  const int row = blockIdx.x;  // 0..3H: b0, b1, b2 rows, then w3 rows, then b3
-  float s = 0.0f;
-  for (long long b = threadIdx.x; b < n; b += 256) {
-    if (row < 3 * H) {
-      s += DZT[(long long)row * n + b];
-    } else if (row < 4 * H) {
-      const int u = row - 3 * H;
-      s += dY[b] * silu_f(ZT[((long long)2 * H + u) * n + b]);
-    } else {
-      s += dY[b];
+      if (16 * q < Din) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, v, acc[q], 0, 0, 0);
     }
   }
-  s = block_sum<256>(s, sh);
-  if (threadIdx.x == 0) {
-    if (row < H) gb0[row] = s;
-    else if (row < 2 * H) gb1[row - H] = s;
-    else if (row < 3 * H) gb2[row - 2 * H] = s;
-    else if (row < 4 * H) gw3[row - 3 * H] = s;
-    else gb3[0] = s;
-  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (16 * q + col < Din) P[(long long)(ob + 4 * g + i) * Din + 16 * q + col] = acc[q][i];
 }
 
-// residual of the MSE loss: dy = 2 (y - t) / n; per-block squared error into loss parts
-__global__ __launch_bounds__(256) void k_mlp_loss(long long n, const float* Y, const float* T, float* dY,
-                                                  double* parts) {
-  __shared__ double sh[4];
-  const long long b = (long long)blockIdx.x * 256 + threadIdx.x;
+// Sums of the parts, in their order: weights, then the vectors (64 columns a workgroup, its waves
+// take a quarter of the rows each), then the squared error per 256 elements, then the loss.
+template <int H>
+__global__ __launch_bounds__(256) void k_mlp_collect(int Din, TrainBuf D, float* G, double* parts, double* loss) {
+  __shared__ float s_f[4][64];
+  __shared__ double s_d[4];
+  const long long size = (long long)H * Din + 2 * H * H;
+  const int wb = (int)((size + 255) / 256), vb = (4 * H + 1 + 63) / 64;
+  int blk = blockIdx.x;
+  if (blk < wb) {
+    const long long q = blk * 256ll + threadIdx.x;
+    if (q >= size) return;
+    const int splits = (int)((D.np + train_slice<H>() - 1) / train_slice<H>());
+    float s = 0.0f;
+#pragma unroll 8
+    for (int k = 0; k < splits; ++k) s += D.P[k * size + q];
+    G[q < (long long)H * Din ? q : q < (long long)H * Din + H * H ? q + H : q + 2 * H] = s;
+    return;
+  }
+  blk -= wb;
+  if (blk < vb) {
+    const int c = blk * 64 + (threadIdx.x & 63), part = threadIdx.x >> 6;
+    const long long rows = D.np / 32;
+    float s = 0.0f;
+    if (c < 4 * H + 1) {
+#pragma unroll 8
+      for (long long r = rows * part / 4; r < rows * (part + 1) / 4; ++r) s += D.B[r * (4 * H + 1) + c];
+    }
+    s_f[part][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (part == 0 && c < 4 * H + 1) {
+      s = (s_f[0][c & 63] + s_f[1][c & 63]) + (s_f[2][c & 63] + s_f[3][c & 63]);
+      const long long b0 = (long long)H * Din;
+      // b0, b1 and b2 follow their weights; w3 and b3 follow b2
+      G[c < H ? b0 + c : c < 2 * H ? b0 + H * H + c : b0 + 2ll * H * H + c] = s;
+    }
+    return;
+  }
+  blk -= vb;
+  const long long nb = (D.n + 255) / 256;
+  const long long lo = blk < nb ? blk * 256ll : 0, hi = blk < nb ? (lo + 256 < D.n ? lo + 256 : D.n) : D.n;
   double e = 0.0;
-  if (b < n) {
-    const float r = Y[b] - T[b];
-    dY[b] = 2.0f * r / (float)n;
-    e = (double)r * (double)r;
+  for (long long k = lo + threadIdx.x; k < hi; k += 256) {
+    const float r = D.Y[k] - D.T[k];
+    e += (double)r * (double)r;
   }
-  e = block_sum<256>(e, sh);
-  if (threadIdx.x == 0) parts[blockIdx.x] = e;
+  e = block_sum<256>(e, s_d);
+  if (threadIdx.x == 0) {
+    if (blk < nb) parts[blk] = e;
+    else *loss = e / (double)D.n;
+  }
 }
 
 // Adam with bias correction: parameter p with moments m, v and gradient g after the step
@@ -1198,8 +1198,6 @@ __global__ __launch_bounds__(1024) void k_mlp_judge(const R* planes, long long s
   }
 }
 
-constexpr int NT_FWD = 2;
-
 template <typename R, int NP, int H>
 int launch_energy(const MlpNet& N, const void* planes, long long stride, const int* n_dev, long long n_max,
                   double* V, const PesParams& fb, hipStream_t st) {
@@ -1346,13 +1344,45 @@ int pvd_mlp_judge(const pvd_pes_desc* pes, int32_t precision, int32_t n_atoms, c
   return 0;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The training buffers in a workspace, and their bytes (64 of them to align its start)
+size_t train_layout(int D, int H, int64_t n, char* ws, TrainBuf& B) {
+  const int64_t np = (n + 31) / 32 * 32, slice = H == 256 ? train_slice<256>() : train_slice<128>();
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    char* p = ws + at;
+    at += (bytes + 63) / 64 * 64;
+    return p;
+  };
+  for (auto& h : B.h) h = (__bf16*)take(2 * (size_t)H * np);
+  for (auto& d : B.dz) d = (__bf16*)take(2 * (size_t)H * np);
+  B.Y = (float*)take(4 * (size_t)np);
+  B.B = (float*)take(4 * (size_t)(np / 32) * (4 * H + 1));
+  B.P = (float*)take(4 * (size_t)((np + slice - 1) / slice) * ((size_t)H * D + 2 * (size_t)H * H));
+  B.n = n;
+  B.np = np;
+  return at + 64;
+}
+int64_t train_bytes(int D, int H, int64_t n) {
+  TrainBuf B;
+  return n <= 0 ? 0 : (int64_t)train_layout(D, H, n, nullptr, B);
+}
+
+}  // namespace
+
+extern "C" {
+
 // Gradients of the mean squared error of the network on (X, T) into grads (flat, the
 // parameter order), plus the loss.  ws: device workspace of pvd_mlp_workspace_bytes().
 int64_t pvd_mlp_workspace_bytes(int32_t D, int32_t H, int64_t batch) {
   const int64_t n = batch;
   const int64_t splits = (n + 255) / 256;
   const int64_t P = splits * (int64_t)H * (H > D ? H : D);
-  return (3 * H * n * 2 + 2 * n + P + (n + 255) / 256 * 2) * 4 + 64;
+  // at least what earlier versions asked for: it bounds the batches that the static scratch takes
+  return std::max<int64_t>((3 * H * n * 2 + 2 * n + P + (n + 255) / 256 * 2) * 4 + 64, train_bytes(D, H, n));
 }
 
 }  // extern "C"
@@ -1385,16 +1415,22 @@ int scratch_for_current_device(void** out) {
 }
 
 int mlp_grads(const pvd_mlp* m, const float* x_t, const float* targets, int64_t n, float* grads, float* y_out,
-              double* loss_parts, void* workspace, void* stream);
+              double* loss_parts, double* loss, void* workspace, void* stream);
 
 }  // namespace
 
 extern "C" {
 
+int pvd_mlp_loss_grads(const pvd_mlp* m, const float* x_t, const float* targets, int64_t n, float* grads, float* y_out,
+                       double* loss_parts, double* loss, void* workspace, void* stream) {
+  if (!workspace || !loss) return mfail(7, "bad arguments");
+  return mlp_grads(m, x_t, targets, n, grads, y_out, loss_parts, loss, workspace, stream);
+}
+
 int pvd_mlp_grads(const pvd_mlp* m, const float* x_t, const float* targets, int64_t n, float* grads, float* y_out,
                   double* loss_parts, void* workspace, void* stream) {
   if (!workspace) return mfail(7, "bad arguments");
-  return mlp_grads(m, x_t, targets, n, grads, y_out, loss_parts, workspace, stream);
+  return mlp_grads(m, x_t, targets, n, grads, y_out, loss_parts, nullptr, workspace, stream);
 }
 
 int64_t pvd_mlp_noalloc_scratch_bytes(void) { return PVD_MLP_SCRATCH_BYTES; }
@@ -1410,68 +1446,38 @@ int pvd_mlp_grads_noalloc(const pvd_mlp* m, const float* x_t, const float* targe
   void* ws = nullptr;
   const int rc = scratch_for_current_device(&ws);
   if (rc) return rc;
-  return mlp_grads(m, x_t, targets, n, grads, y_out, loss_parts, ws, stream);
+  return mlp_grads(m, x_t, targets, n, grads, y_out, loss_parts, nullptr, ws, stream);
 }
 
 }  // extern "C"
 
 namespace {
 
+template <int H>
+int launch_grads(const MlpNet& N, TrainBuf B, float* grads, double* loss_parts, double* loss, hipStream_t st) {
+  const int D = N.D;
+  const unsigned slices = (unsigned)((B.np + train_slice<H>() - 1) / train_slice<H>());
+  hipLaunchKernelGGL(k_mlp_fwd_bwd<H>, dim3((unsigned)(B.np / 32)), dim3(2 * H), 0, st, N, B);
+  hipLaunchKernelGGL(k_mlp_wgrad<H>, dim3(2 * (H / 64) * (H / 64) + H / 64, slices), dim3(256), 0, st, D, B);
+  const long long blocks = ((long long)H * D + 2 * H * H + 255) / 256 + (4 * H + 64) / 64 + (B.n + 255) / 256 + (loss ? 1 : 0);
+  hipLaunchKernelGGL(k_mlp_collect<H>, dim3((unsigned)blocks), dim3(256), 0, st, D, B, grads, loss_parts, loss);
+  MHIP(hipGetLastError());
+  return 0;
+}
+
 int mlp_grads(const pvd_mlp* m, const float* x_t, const float* targets, int64_t n, float* grads, float* y_out,
-              double* loss_parts, void* workspace, void* stream) {
+              double* loss_parts, double* loss, void* workspace, void* stream) {
   MlpNet N;
   if (!m || !x_t || !targets || !grads || !workspace || !build_net(m, N)) return mfail(7, "bad arguments");
   if (n <= 0) return mfail(7, "empty batch");
   hipStream_t st = (hipStream_t)stream;
-  const int D = N.D, H = N.H;
-  float* ZT = (float*)workspace;
-  float* DZT = ZT + 3ll * H * n;
-  float* Y = DZT + 3ll * H * n;
-  float* dY = Y + n;
-  float* P = dY + n;
-  const long long per_block = 4ll * 16 * NT_FWD;
-  const unsigned grid = (unsigned)((n + per_block - 1) / per_block);
-  const size_t lds = (size_t)(H / 16) * (H / 32) * 64 * 16;
-  PesParams fb;
-  std::memset(&fb, 0, sizeof(fb));
-  if (H == 128) {
-    auto kf = k_mlp_forward<float, 9, 128, NT_FWD, 1>;
-    auto kb = k_mlp_backward<128, NT_FWD>;
-    MHIP(hipFuncSetAttribute((const void*)kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    MHIP(hipFuncSetAttribute((const void*)kb, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kf, dim3(grid), dim3(256), lds, st, N, (const float*)nullptr, 0ll, (const int*)nullptr,
-                       (long long)n, (double*)nullptr, fb, x_t, ZT, Y);
-    hipLaunchKernelGGL(k_mlp_loss, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (long long)n, Y, targets, dY,
-                       loss_parts);
-    hipLaunchKernelGGL(kb, dim3(grid), dim3(256), lds, st, N, (long long)n, ZT, dY, DZT);
-  } else {
-    auto kf = k_mlp_forward<float, 9, 256, 1, 1>;
-    auto kb = k_mlp_backward<256, 1>;
-    const unsigned grid1 = (unsigned)((n + 63) / 64);
-    MHIP(hipFuncSetAttribute((const void*)kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    MHIP(hipFuncSetAttribute((const void*)kb, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kf, dim3(grid1), dim3(256), lds, st, N, (const float*)nullptr, 0ll, (const int*)nullptr,
-                       (long long)n, (double*)nullptr, fb, x_t, ZT, Y);
-    hipLaunchKernelGGL(k_mlp_loss, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (long long)n, Y, targets, dY,
-                       loss_parts);
-    hipLaunchKernelGGL(kb, dim3(grid1), dim3(256), lds, st, N, (long long)n, ZT, dY, DZT);
-  }
-  const int kslice = 256;
-  const int splits = (int)((n + kslice - 1) / kslice);
-  for (int l = 0; l < 3; ++l) {
-    const int Din = l == 0 ? D : H;
-    dim3 g3((unsigned)(H / 32), (unsigned)((Din + 31) / 32), (unsigned)splits);
-    hipLaunchKernelGGL(k_mlp_wgrad, g3, dim3(64), 0, st, l, H, Din, (long long)n, kslice, x_t, ZT, DZT, P);
-    const long long size = (long long)H * Din;
-    hipLaunchKernelGGL(k_mlp_wgrad_reduce, dim3((unsigned)((size + 255) / 256)), dim3(256), 0, st, P, splits, size,
-                       grads + off_W(l, D, H));
-  }
-  hipLaunchKernelGGL(k_mlp_rowsum, dim3((unsigned)(4 * H + 1)), dim3(256), 0, st, H, (long long)n, ZT, DZT, dY,
-                     grads + off_b(0, D, H), grads + off_b(1, D, H), grads + off_b(2, D, H), grads + off_w3(D, H),
-                     grads + off_w3(D, H) + H);
-  if (y_out) MHIP(hipMemcpyAsync(y_out, Y, sizeof(float) * n, hipMemcpyDeviceToDevice, st));
-  MHIP(hipGetLastError());
-  return 0;
+  TrainBuf B;
+  (void)train_layout(N.D, N.H, n, (char*)(((uintptr_t)workspace + 63) & ~(uintptr_t)63), B);
+  B.XT = x_t;
+  B.T = targets;
+  if (y_out) B.Y = y_out;
+  return N.H == 128 ? launch_grads<128>(N, B, grads, loss_parts, loss, st)
+                    : launch_grads<256>(N, B, grads, loss_parts, loss, st);
 }
 
 }  // namespace

@@ -43,6 +43,7 @@ _MSIGS = {
     'pvd_mlp_energy': (ctypes.c_int, [ctypes.POINTER(MLPDesc), ctypes.c_int32, ctypes.c_int32, _P, ctypes.c_int64,
                                       _P, ctypes.c_int64, _P, ctypes.POINTER(N.PesDesc), _P]),
     'pvd_mlp_grads': (ctypes.c_int, [ctypes.POINTER(MLPDesc), _P, _P, ctypes.c_int64, _P, _P, _P, _P, _P]),
+    'pvd_mlp_loss_grads': (ctypes.c_int, [ctypes.POINTER(MLPDesc), _P, _P, ctypes.c_int64, _P, _P, _P, _P, _P, _P]),
     'pvd_mlp_grads_noalloc': (ctypes.c_int, [ctypes.POINTER(MLPDesc), _P, _P, ctypes.c_int64, _P, _P, _P, _P]),
     'pvd_mlp_noalloc_scratch_bytes': (ctypes.c_int64, []),
     'pvd_mlp_adam': (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_float, ctypes.c_float,
@@ -252,10 +253,11 @@ class SurrogateModel:
         n = targets.shape[0]
         ws, lp = self._workspace(n)
         y = torch.empty(n, dtype=torch.float32, device='cuda')
-        _check(_lib().pvd_mlp_grads(ctypes.byref(self.desc), x_t.data_ptr(), targets.data_ptr(), n,
-                                    self.grads.data_ptr(), y.data_ptr(), lp.data_ptr(), ws.data_ptr(),
-                                    N.stream_handle()), 'pvd_mlp_grads')
-        return lp[:(n + 255) // 256].sum() / n, y
+        loss = torch.empty((), dtype=torch.float64, device='cuda')
+        _check(_lib().pvd_mlp_loss_grads(ctypes.byref(self.desc), x_t.data_ptr(), targets.data_ptr(), n,
+                                         self.grads.data_ptr(), y.data_ptr(), lp.data_ptr(), loss.data_ptr(),
+                                         ws.data_ptr(), N.stream_handle()), 'pvd_mlp_loss_grads')
+        return loss, y
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.t += 1

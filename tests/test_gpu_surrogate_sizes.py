@@ -104,3 +104,43 @@ def test_adam_pack_equals_adam_then_pack(features, hidden, offset):
         results.append([v.cpu() for v in (p, m1, m2, packs)])
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('elements,hidden', [(WATER, 128), (WATER, 256), (CLUSTER, 128), (CLUSTER, 256)])
+@pytest.mark.parametrize('n', [1, 2, 31, 33, 255, 257, 511, 513, 4099])
+def test_gradient_sizes(elements, hidden, n):
+    """Batches at the ends of the tiles (32), slices (256, 512) and loss parts (256) against the
+    oracle.  Both sides round the same operands to bfloat16; the accumulation order flips a few of
+    those roundings, each of up to 2^-8 of its value: a tensor is held to that, and the mean over a
+    large batch to 5e-4.  Nothing is written past the outputs."""
+    import ctypes
+    import torch
+    import pyvibdmc_amd as pv
+    from pyvibdmc_amd import _native as N
+    from pyvibdmc_amd.surrogate import _lib
+    lib = _lib()
+    m = pv.SurrogateModel(elements, hidden=hidden, seed=5)
+    x, pes = walkers(elements, 5000, 6), surface(elements)
+    m.set_normalisation(x, pes(x))
+    xt = m.features(x[:n], normalise=True)
+    t = torch.from_numpy(((pes(x[:n]) - m.desc.ymean) / m.desc.ystd).astype(np.float32)).cuda()
+    parts = (n + 255) // 256
+    ws = torch.full((int(lib.pvd_mlp_workspace_bytes(m.D, hidden, n)) + 4096,), 0xA5, dtype=torch.uint8, device='cuda')
+    g, y = (torch.full((k + 16,), 7.0, dtype=torch.float32, device='cuda') for k in (m.grads.numel(), n))
+    lp, loss = (torch.full((k + 4,), 7.0, dtype=torch.float64, device='cuda') for k in (parts, 1))
+    rc = lib.pvd_mlp_loss_grads(ctypes.byref(m.desc), xt.data_ptr(), t.data_ptr(), n, g.data_ptr(), y.data_ptr(),
+                                lp.data_ptr(), loss.data_ptr(), ws.data_ptr(), N.stream_handle())
+    assert rc == 0, lib.pvd_mlp_last_error()
+    assert (g[-16:] == 7).all() and (y[-16:] == 7).all() and (lp[parts:] == 7).all() and (loss[1:] == 7).all()
+    assert (ws[-4096:] == 0xA5).all()
+    net, xn = network(m, x[:n])
+    lo, yo, go = net.loss_grads(xt.cpu().numpy().T.copy(), t.cpu().numpy().astype(np.float64))
+    tol = 5e-4 if n > 2000 else 2.0 ** -8
+    assert np.linalg.norm(y[:n].cpu().numpy() - yo) <= 2.0 ** -8 * max(np.linalg.norm(yo), np.sqrt(n))
+    assert abs(float(loss[0]) - lo) <= 4 * tol * lo
+    assert abs(float(lp[:parts].sum()) / n - float(loss[0])) <= 1e-12 * lo
+    flat, o, H, D = g.cpu().numpy(), 0, m.H, m.D
+    for k, sz in (('W0', H * D), ('b0', H), ('W1', H * H), ('b1', H), ('W2', H * H), ('b2', H), ('w3', H), ('b3', 1)):
+        a, b = flat[o:o + sz], go[k].reshape(-1)
+        o += sz
+        assert np.linalg.norm(a - b) <= 4 * tol * np.linalg.norm(b), k
