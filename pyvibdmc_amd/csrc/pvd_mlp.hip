@@ -216,8 +216,10 @@ PVD_DEV void mlp_descriptor(const MlpNet& M, const R* x, float* f, float* scratc
 // Training: forward and backward of a batch (k_mlp_fwd_bwd), the weight gradients from the BF16
 // operands that it leaves (k_mlp_wgrad), and the sums of both kernels' parts (k_mlp_collect).
 
-// What the three kernels share.  Batch element b of row u at [u * np + b], np = n rounded up to 32.
+// What the three kernels share.  Batch element b of operand row u at [u * ld + b]; elements from n to
+// np, n rounded up to 32, are zero.
 struct TrainBuf {
+  __bf16* x;      // the features (32 rows, zero beyond D)
   __bf16* h[2];   // silu(z_0), silu(z_1)
   __bf16* dz[3];  // dL/dz_l
   float* Y;       // network outputs
@@ -225,7 +227,7 @@ struct TrainBuf {
   float* P;       // per batch slice: W0, W1, W2 gradients
   const float* XT;
   const float* T;
-  long long n, np;
+  long long n, np, ld;
 };
 
 template <int H>
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(2 * H, H == 256 ? 2 : 1) void k_mlp_fwd_bwd(MlpNet 
   __shared__ float s_dy[32];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, col = lane & 15;
-  const long long base = 32ll * blockIdx.x, n = D.n, np = D.np;
+  const long long base = 32ll * blockIdx.x, n = D.n, ld = D.ld;
   const long long w0 = base + 2 * col;
   const bool ok[2] = {w0 < n, w0 + 1 < n};
   auto unit = [&](int m, int i) { return 32 * wv + 16 * m + 4 * g + i; };
@@ -269,27 +271,30 @@ __global__ __launch_bounds__(2 * H, H == 256 ? 2 : 1) void k_mlp_fwd_bwd(MlpNet 
   weights(Wa, M.Wf[1]);
   f32x4 z[3][2][2];
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
   {  // layer 0
-    bf16x8 W0[2];
+    bf16x8 W0[2], v[2];
 #pragma unroll
     for (int m = 0; m < 2; ++m) W0[m] = M.Wf[0][(2 * wv + m) * 64 + lane];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      bf16x8 v;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int k = 8 * g + j;
-        v[j] = (__bf16)((ok[t] && k < M.D) ? D.XT[(long long)k * n + w0 + t] : 0.0f);
+        v[t][j] = (__bf16)((ok[t] && k < M.D) ? D.XT[(long long)k * n + w0 + t] : 0.0f);
       }
 #pragma unroll
-      for (int m = 0; m < 2; ++m) z[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W0[m], v, zero, 0, 0, 0) + b[0][m];
+      for (int m = 0; m < 2; ++m) z[0][t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W0[m], v[t], zero, 0, 0, 0) + b[0][m];
+    }
+    if (wv == 0) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) *(bf16x2*)(D.x + (8 * g + j) * ld + w0) = bf16x2{v[0][j], v[1][j]};
     }
   }
   weights(Wb, M.Wf[2]);
   // a pair of batch elements of every unit to the weight gradient's operands (zero past the batch),
   // and both to the rows of the next product
   auto publish = [&](const float (&x)[2][2][4], __bf16* to, bf16x8* rows) {
-    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
     bf16x8 u[2];
 #pragma unroll
     for (int m = 0; m < 2; ++m)
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(2 * H, H == 256 ? 2 : 1) void k_mlp_fwd_bwd(MlpNet 
           u[t][4 * m + i] = (__bf16)x[t][m][i];
           v[t] = ok[t] ? u[t][4 * m + i] : (__bf16)0.0f;
         }
-        if (to) *(bf16x2*)(to + unit(m, i) * np + w0) = v;
+        if (to) *(bf16x2*)(to + unit(m, i) * ld + w0) = v;
       }
     if (rows) {
 #pragma unroll
@@ -429,8 +434,8 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(int Din, TrainBuf D) {
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   if (tile < 2 * TI * TI) {
     const int l = 1 + tile / (TI * TI), ob = tile / TI % TI * 64 + 32 * (wv >> 1), ib = tile % TI * 64 + 32 * (wv & 1);
-    const __bf16* pa = D.dz[l] + (ob + col) * D.np + 8 * g;
-    const __bf16* pb = D.h[l - 1] + (ib + col) * D.np + 8 * g;
+    const __bf16* pa = D.dz[l] + (ob + col) * D.ld + 8 * g;
+    const __bf16* pb = D.h[l - 1] + (ib + col) * D.ld + 8 * g;
     f32x4 acc[2][2];
 #pragma unroll
     for (int q = 0; q < 4; ++q) acc[q >> 1][q & 1] = zero;
@@ -439,8 +444,8 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(int Din, TrainBuf D) {
       bf16x8 A[2], Bv[2];
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        A[q] = *(const bf16x8*)(pa + 16 * q * D.np + k);
-        Bv[q] = *(const bf16x8*)(pb + 16 * q * D.np + k);
+        A[q] = *(const bf16x8*)(pa + 16 * q * D.ld + k);
+        Bv[q] = *(const bf16x8*)(pb + 16 * q * D.ld + k);
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -454,21 +459,15 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(int Din, TrainBuf D) {
     return;
   }
   const int ob = (tile - 2 * TI * TI) * 64 + 16 * wv;
-  const __bf16* pa = D.dz[0] + (ob + col) * D.np + 8 * g;
+  const __bf16* pa = D.dz[0] + (ob + col) * D.ld + 8 * g;
+  const __bf16* pb = D.x + col * D.ld + 8 * g;
   f32x4 acc[2] = {zero, zero};
+#pragma unroll 4
   for (long long k = k0; k < k1; k += 32) {
     const bf16x8 A = *(const bf16x8*)(pa + k);
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int u = 16 * q + col;
-      bf16x8 v;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const long long e = k + 8 * g + j;
-        v[j] = (__bf16)(u < Din && e < D.n ? D.XT[(long long)u * D.n + e] : 0.0f);
-      }
-      if (16 * q < Din) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, v, acc[q], 0, 0, 0);
-    }
+    for (int q = 0; q < 2; ++q)
+      acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, *(const bf16x8*)(pb + 16 * q * D.ld + k), acc[q], 0, 0, 0);
   }
 #pragma unroll
   for (int q = 0; q < 2; ++q)
@@ -1350,20 +1349,24 @@ namespace {
 
 // The training buffers in a workspace, and their bytes (64 of them to align its start)
 size_t train_layout(int D, int H, int64_t n, char* ws, TrainBuf& B) {
-  const int64_t np = (n + 31) / 32 * 32, slice = H == 256 ? train_slice<256>() : train_slice<128>();
+  // rows 320 bytes past a multiple of 4 KB: the 16 rows that a wave reads at once lie in different
+  // channels (8192 elements, width 256, rows of 16 KB: weight gradients 37 us, 20 so)
+  const int64_t np = (n + 31) / 32 * 32, ld = (np + 2047 - 160) / 2048 * 2048 + 160, slice = H == 256 ? train_slice<256>() : train_slice<128>();
   size_t at = 0;
   auto take = [&](size_t bytes) {
     char* p = ws + at;
     at += (bytes + 63) / 64 * 64;
     return p;
   };
-  for (auto& h : B.h) h = (__bf16*)take(2 * (size_t)H * np);
-  for (auto& d : B.dz) d = (__bf16*)take(2 * (size_t)H * np);
+  B.x = (__bf16*)take(2 * 32 * (size_t)ld);
+  for (auto& h : B.h) h = (__bf16*)take(2 * (size_t)H * ld);
+  for (auto& d : B.dz) d = (__bf16*)take(2 * (size_t)H * ld);
   B.Y = (float*)take(4 * (size_t)np);
   B.B = (float*)take(4 * (size_t)(np / 32) * (4 * H + 1));
   B.P = (float*)take(4 * (size_t)((np + slice - 1) / slice) * ((size_t)H * D + 2 * (size_t)H * H));
   B.n = n;
   B.np = np;
+  B.ld = ld;
   return at + 64;
 }
 int64_t train_bytes(int D, int H, int64_t n) {
