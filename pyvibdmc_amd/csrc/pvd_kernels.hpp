@@ -95,8 +95,8 @@ struct Cand {
 constexpr int CAND_CAP = 4096;   // candidates the replay sorts in LDS
 constexpr int CAND_G = 131072;   // candidates the global-memory replay sorts (2 KILL_CAP)
 // scratch of the global-memory replay: keys and bucketed keys (8 B each), order and bucketed
-// order (4 B each), family starts (4 B), split depths (1 B) per candidate
-constexpr size_t RSG_BYTES = (size_t)CAND_G * (8 + 8 + 4 + 4 + 4 + 1);
+// order (4 B each), family starts (4 B) per candidate
+constexpr size_t RSG_BYTES = (size_t)CAND_G * (8 + 8 + 4 + 4 + 4);
 constexpr int LIST_SUB = 8;       // sub-lists per list (spreads the appends' counters)
 constexpr int SUB_CAP = 32768;    // entries per sub-list and step
 constexpr int LIST_CAP = LIST_SUB * SUB_CAP;
@@ -1283,7 +1283,12 @@ enum { RC_DONE = 0, RC_FEW = 1, RC_MANY = 2, RC_OTHER = 3 };
 // counts (4 B per bucket, one per candidate), split depth (1 B)
 constexpr int RC_BUCKETS = CAND_CAP;
 constexpr int RC_LDS = 25 * CAND_CAP;
-constexpr int RP_LDS = RP_CAP * (int)sizeof(Piece) > RC_LDS ? RP_CAP * (int)sizeof(Piece) : RC_LDS;
+// the order of the global-memory replay's candidates: a word each, and 16-bit bucket counts in the
+// place of the histogram
+constexpr int RO_BUCKETS = 16384, RO_CAP = 31 * 1024;
+constexpr int RO_BMAX = 64;          // the largest bucket that it ranks
+constexpr int RO_PAD = RO_BMAX + 4;  // words before the first and after the last that it may read
+constexpr int RP_LDS = std::max(std::max(RP_CAP * (int)sizeof(Piece), RC_LDS), 4 * (RO_CAP + 2 * RO_PAD));
 
 PVD_DEV int dexp(double w) { return (int)((__double_as_longlong(w) >> 52) & 0x7FF) - 1023; }
 
@@ -1706,14 +1711,13 @@ static_assert(RCG_BUCKETS * (int)sizeof(int) <= RP_LDS && RCG_BUCKETS % RP_NT ==
 constexpr int RG_U = 4;  // loads in flight per thread in the streaming loops
 
 // the replay scratch: keys, bucketed keys (8 B each), walker slots, bucketed slots, family-p
-// slots (4 B each), split depths (1 B), CAND_G of each
+// slots (4 B each), CAND_G of each
 struct RsgView {
   unsigned long long* key;
   unsigned long long* bkey;
   int* ord;
   int* bord;
   int* start;
-  unsigned char* dep;
 };
 PVD_DEV RsgView rsg_view(unsigned char* rsg) {
   RsgView v;
@@ -1722,13 +1726,172 @@ PVD_DEV RsgView rsg_view(unsigned char* rsg) {
   v.ord = reinterpret_cast<int*>(v.bkey + CAND_G);
   v.bord = v.ord + CAND_G;
   v.start = v.bord + CAND_G;
-  v.dep = reinterpret_cast<unsigned char*>(v.start + CAND_G);
   return v;
 }
 
 PVD_DEV double key_weight(unsigned long long k) {
   constexpr unsigned long long MANT = (1ull << 52) - 1;
   return __longlong_as_double((long long)(((0x7FFull - (k & 0x7FFull)) << 52) | (MANT - (k >> 11))));
+}
+
+PVD_DEV unsigned long long weight_key(double w) {
+  constexpr unsigned long long MANT = (1ull << 52) - 1;
+  const unsigned long long wb = (unsigned long long)__double_as_longlong(w);
+  return ((MANT - (wb & MANT)) << 11) | (0x7FFull - ((wb >> 52) & 0x7FFull));
+}
+PVD_DEV int key_exp(unsigned long long k) { return (int)(0x7FFull - (k & 0x7FFull)) - 1023; }
+// times a candidate's family is halved, `last` being the key of the family where the kills run out,
+// in octave Es (equal keys that matter are ties, which the replay declines)
+PVD_DEV int key_depth(unsigned long long k, unsigned long long last, int Es) {
+  const int e = key_exp(k);
+  return e < Es ? 0 : e - Es + (k < last ? 1 : 0);
+}
+
+// Sorting of the C <= RO_CAP collected candidates that leaves them where they are (the keys and
+// slots in the global scratch) and orders 4-byte words in LDS: a colour that alternates from one
+// occupied bucket to the next, 10 key bits below the bucket's, the exponent above eT, the
+// candidate's index.  A counting sort on 14 bits of the key; then every word counts the smaller ones
+// behind and the larger ones before it in its bucket (as far as the colour holds) and moves by that.
+// Words that agree in the 10 bits are then put in the order of their whole keys, which is also where
+// equal mantissas meet (they share a bucket and its 10 bits): tie_e is the highest octave in which
+// they do.
+// False where a bucket is too full.
+// Moving keys and slots instead took two passes of scattered accesses to L2, about one line a
+// cycle from the one CU, and a thread's run of the sorted keys for every octave as much again
+// (22 000 candidates: 65 and 38 us; now 28 000, with no cut at 1.25 K, 42 and 14).
+PVD_DEV bool order_candidates(int C, const unsigned long long* key, unsigned long long kmin, unsigned long long kmax,
+                              int eT, unsigned* cnt, unsigned* word, int* s_i, int& tie_e) {
+  constexpr int NT = RP_NT, U = 8, WPT = RO_BUCKETS / 2 / NT;
+  const int tid = threadIdx.x;
+  kmin &= ~0x7FFull;
+  const unsigned long long span = kmax - kmin;
+  const int bsh = max(11, (span >> 14) == 0ull ? 0 : 64 - __clzll((long long)span) - 14);
+  const int ssh = max(11, bsh - 10);
+  const unsigned smask = (1u << (bsh - ssh)) - 1u;
+  auto bucket = [&](unsigned long long k) { return (int)((k - kmin) >> bsh); };  // < RO_BUCKETS
+  for (int b = tid; b < RO_BUCKETS / 2; b += NT) cnt[b] = 0;
+  __syncthreads();
+  // pass 0 counts, pass 1 places
+  auto sweep = [&](auto f) {
+    for (int q0 = 0; q0 < C; q0 += U * NT) {
+      unsigned long long kk[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        kk[u] = q < C ? key[q] : 0ull;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        if (q < C) f(q, kk[u]);
+      }
+    }
+    __syncthreads();
+  };
+  auto bump = [&](int b) {  // the bucket's counter before it is raised
+    const int sh = 16 * (b & 1);
+    return (int)((atomicAdd(&cnt[b >> 1], 1u << sh) >> sh) & 0xFFFFu);
+  };
+  sweep([&](int, unsigned long long k) { (void)bump(bucket(k)); });
+  unsigned c2[WPT];
+  int loc = 0, mx = 0;  // entries, and occupied buckets above bit 16
+#pragma unroll
+  for (int u = 0; u < WPT; ++u) {
+    c2[u] = cnt[tid * WPT + u];
+    const int a = (int)(c2[u] & 0xFFFFu), b = (int)(c2[u] >> 16);
+    loc += a + b + (((a > 0) + (b > 0)) << 16);
+    mx = max(mx, max(a, b));
+  }
+  int tot;
+  int st = block_excl_scan<NT>(loc, s_i, tot);
+#pragma unroll
+  for (int u = 0; u < WPT; ++u) {  // bucket starts and colours (each thread rewrites only its own buckets)
+    auto next = [&](int n) {
+      const unsigned v = (unsigned)(st & 0x7FFF) | ((unsigned)(st >> 16) & 1u) << 15;
+      st += n + ((n > 0) << 16);
+      return v;
+    };
+    const unsigned a = next((int)(c2[u] & 0xFFFFu));
+    cnt[tid * WPT + u] = a | next((int)(c2[u] >> 16)) << 16;
+  }
+  if (block_max<NT>(mx, s_i) > RO_BMAX) return false;
+  sweep([&](int q, unsigned long long k) {
+    const unsigned sub = (unsigned)((k - kmin) >> ssh) & smask;
+    const int r = bump(bucket(k));
+    word[r & 0x7FFF] = (unsigned)(r >> 15) << 31 | sub << 21 | (unsigned)(key_exp(k) - eT) << 15 | (unsigned)q;
+  });
+  auto before = [&](unsigned a, unsigned b) {  // by whole keys, then by index
+    const unsigned long long ka = key[a & 0x7FFFu], kb = key[b & 0x7FFFu];
+    if (ka >> 11 == kb >> 11) tie_e = max(tie_e, min(key_exp(ka), key_exp(kb)));
+    return ka < kb || (ka == kb && (a & 0x7FFFu) < (b & 0x7FFFu));
+  };
+  if (tid == 0) {  // the colour ends at both ends
+    word[-1] = ~word[0];
+    word[C] = ~word[C - 1];
+  }
+  __syncthreads();
+  constexpr int EPT = RO_CAP / NT, RU = 4;
+  unsigned own[EPT];
+  int to[EPT];
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int d = tid + e * NT;
+    to[e] = d;
+    if (e * NT < C) {
+      bool up = d < C, down = d < C;
+      own[e] = up ? word[d] : 0u;
+      for (int i = 1; __any(up || down); i += RU) {  // at most RO_BMAX + RU words away
+        unsigned v[RU], w[RU];
+#pragma unroll
+        for (int k = 0; k < RU; ++k) {
+          v[k] = word[d - i - k];
+          w[k] = word[d + i + k];
+        }
+#pragma unroll
+        for (int k = 0; k < RU; ++k) {
+          up = up && (int)(v[k] ^ own[e]) >= 0;
+          down = down && (int)(w[k] ^ own[e]) >= 0;
+          to[e] += (down && w[k] < own[e] ? 1 : 0) - (up && v[k] > own[e] ? 1 : 0);
+        }
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < EPT; ++e)
+    if (tid + e * NT < C) word[to[e]] = own[e];
+  __syncthreads();
+  if (tid == 0) {
+    word[-1] = ~word[0];
+    word[C] = ~word[C - 1];
+  }
+  __syncthreads();
+  unsigned runs = 0;  // runs of equal bits that start at this thread's entries
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int d = tid + e * NT;
+    if (d < C) {
+      const unsigned w = word[d];
+      if ((w ^ word[d + 1]) >> 21 == 0u && (w ^ word[d - 1]) >> 21 != 0u) runs |= 1u << e;
+    }
+  }
+  __syncthreads();
+  for (; runs; runs &= runs - 1u) {
+    const int d = tid + (__ffs((int)runs) - 1) * NT;
+    const unsigned bits = word[d] >> 21;
+    for (int i = 1; word[d + i] >> 21 == bits; ++i) {
+      const unsigned w = word[d + i];
+      int j = i;
+      for (; j > 0; --j) {
+        const unsigned v = word[d + j - 1];
+        if (!before(w, v)) break;
+        word[d + j] = v;
+      }
+      word[d + j] = w;
+    }
+  }
+  tie_e = block_max<NT>(tie_e, s_i);  // barriers: the words are in order
+  return true;
 }
 
 template <typename R>
@@ -1769,16 +1932,15 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
   int* ord = rv.ord;
   int* bord = rv.bord;
   int* start = rv.start;
-  unsigned char* dep = rv.dep;
-  auto kexp = [](unsigned long long k) { return (int)(0x7FFull - (k & 0x7FFull)) - 1023; };
+  auto kexp = [](unsigned long long k) { return key_exp(k); };
   auto kmant = [](unsigned long long k) { return MANT - (k >> 11); };
   // 1. the cut: T0, or, when the lists hold over a quarter more than about 1.25 K walkers
-  //    (at a steady state list A holds the last step's 2 K split pieces), the lowest
-  //    histogram edge with at most 1.25 K entries at or above it: every later pass is over
-  //    the walkers >= the cut only
+  //    (at a steady state list A holds the last step's 2 K split pieces) and more than the LDS
+  //    order takes, the lowest histogram edge with at most 1.25 K entries at or above it: every
+  //    later pass is over the walkers >= the cut only
   double T = T0;
   const int lim = min(CAND_G, max(K + K / 4, 1024));
-  refined = nl > lim + lim / 4;
+  refined = nl > max(lim + lim / 4, RO_CAP);
   if (refined) {
     for (int b = tid; b < TH_BINS; b += NT) hist[b] = 0;
     __syncthreads();
@@ -1806,35 +1968,50 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
   if (tid == 0) s_sh[3] = 0;
   __syncthreads();
   unsigned long long kmin = ~0ull, kmax = 0ull;
-  for (int q0 = 0; q0 < nl; q0 += U * NT) {
-    Cand c[U];
+  const int eT = dexp(T);
+  const unsigned long long mT = (unsigned long long)__double_as_longlong(T) & MANT;
+  int etop = -0x40000000, above = 0;  // above: mantissas at or above T's
+  // wave w reads sub-list w % 8 of each list, one half of it
+  constexpr int UC = 8;
+  static_assert(NT / PVD_WAVE == 2 * LIST_SUB, "two waves to a sub-list");
+  const int cw = __builtin_amdgcn_readfirstlane(tid / PVD_WAVE);
+  for (int list = 0; list < nlists; ++list) {
+    const int sub = list * LIST_SUB + cw % LIST_SUB, ns = subn[sub];
+    const Cand* from = A.cand + (size_t)sub * SUB_CAP;
+    for (int q0 = cw / LIST_SUB * PVD_WAVE; q0 < ns; q0 += 2 * PVD_WAVE * UC) {
+      Cand c[UC];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = q0 + u * NT + tid;
-      if (q < nl) {
-        c[u] = A.cand[phys(q)];
-      } else {
-        c[u].w = -1.0;
-        c[u].slot = 0;
+      for (int u = 0; u < UC; ++u) {
+        const int q = q0 + 2 * PVD_WAVE * u + lane_id();
+        if (q < ns) {
+          c[u] = from[q];
+        } else {
+          c[u].w = -1.0;
+          c[u].slot = 0;
+        }
       }
-    }
+      unsigned long long bal[UC];
+      int got = 0;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool in = c[u].w >= T;
-      const unsigned long long bal = __ballot(in);
-      if (bal) {
-        const int lead = __ffsll((long long)bal) - 1;
-        int base = 0;
-        if (lane_id() == lead) base = atomicAdd(&s_sh[3], __popcll(bal));
-        base = __shfl(base, lead, PVD_WAVE);
-        const int o = base + __popcll(bal & ((1ull << lane_id()) - 1ull));
-        if (in && o < CAND_G) {
-          const unsigned long long wb = (unsigned long long)__double_as_longlong(c[u].w);
-          const unsigned long long k = ((MANT - (wb & MANT)) << 11) | (0x7FFull - ((wb >> 52) & 0x7FFull));
+      for (int u = 0; u < UC; ++u) {
+        bal[u] = __ballot(c[u].w >= T);
+        got += __popcll(bal[u]);
+      }
+      int at = 0;
+      if (got > 0 && lane_id() == 0) at = atomicAdd(&s_sh[3], got);
+      at = __shfl(at, 0, PVD_WAVE);
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const int o = at + __popcll(bal[u] & ((1ull << lane_id()) - 1ull));
+        at += __popcll(bal[u]);
+        if (c[u].w >= T && o < CAND_G) {
+          const unsigned long long k = weight_key(c[u].w);
           key[o] = k;
           ord[o] = c[u].slot;
           kmin = k < kmin ? k : kmin;
           kmax = k > kmax ? k : kmax;
+          etop = max(etop, key_exp(k));
+          above += MANT - (k >> 11) >= mT ? 1 : 0;
         }
       }
     }
@@ -1847,223 +2024,255 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
   const int C = s_sh[3];
   if (C > CAND_G) return RC_MANY;
   if (C == 0) return RC_FEW;
-  // 2. candidates by decreasing mantissa (then exponent): counting sort on 14 bits of the key
-  //    above its minimum (an order-preserving map of the keys' own range onto the buckets: the
-  //    candidates of a steady state lie in a band about a tenth of an octave wide, which the
-  //    top mantissa bits would crowd into a tenth of the buckets), then each entry ranked
-  //    inside its bucket
-  constexpr int BPT = RCG_BUCKETS / NT;
-  const unsigned long long kspan = kmax - kmin;
-  const int bsh = (kspan >> 14) == 0ull ? 0 : 64 - __clzll((long long)kspan) - 14;
-  auto bucket = [&](unsigned long long k) { return (int)((k - kmin) >> bsh); };  // < RCG_BUCKETS
-  for (int b = tid; b < RCG_BUCKETS; b += NT) bcnt[b] = 0;
-  __syncthreads();
-  for (int q0 = 0; q0 < C; q0 += U * NT) {
-    unsigned long long kk[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = q0 + u * NT + tid;
-      kk[u] = q < C ? key[q] : 0ull;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (q0 + u * NT + tid < C) atomicAdd(&bcnt[bucket(kk[u])], 1);
-  }
-  __syncthreads();
-  int bmax;
-  {
-    int loc = 0, mx = 0;
-    for (int u = 0; u < BPT; ++u) {
-      const int c = bcnt[tid * BPT + u];
-      loc += c;
-      mx = max(mx, c);
-    }
-    int tot;
-    const int ex = block_excl_scan<NT>(loc, s_i, tot);
-    int st = ex;
-    for (int u = 0; u < BPT; ++u) {
-      const int c = bcnt[tid * BPT + u];
-      bcnt[tid * BPT + u] = st;  // bucket starts (each thread rewrites only its own buckets)
-      st += c;
-    }
-    bmax = block_max<NT>(mx, s_i);
-  }
-  if (bmax > RCG_BMAX) return RC_OTHER;  // the in-bucket rank costs bucket size squared
-  for (int q0 = 0; q0 < C; q0 += U * NT) {
-    unsigned long long kk[U];
-    int oo[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = q0 + u * NT + tid;
-      kk[u] = q < C ? key[q] : 0ull;
-      oo[u] = q < C ? ord[q] : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (q0 + u * NT + tid < C) {
-        const int d = atomicAdd(&bcnt[bucket(kk[u])], 1);  // bcnt ends as the bucket ends
-        bkey[d] = kk[u];
-        bord[d] = oo[u];
-      }
-  }
-  __syncthreads();
-  // ranks: U entries per thread at a time, the first RK keys of each one's bucket in flight
-  constexpr int RK = 4;
-  for (int q0 = 0; q0 < C; q0 += U * NT) {
-    unsigned long long kq[U];
-    int oq[U], bs[U], be[U], rank[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = q0 + u * NT + tid;
-      kq[u] = q < C ? bkey[q] : 0ull;
-      oq[u] = q < C ? bord[q] : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = q0 + u * NT + tid;
-      const int bk = q < C ? bucket(kq[u]) : 0;
-      bs[u] = q < C ? (bk > 0 ? bcnt[bk - 1] : 0) : 0;
-      be[u] = q < C ? bcnt[bk] : 0;
-      rank[u] = 0;
-    }
-#pragma unroll
-    for (int i = 0; i < RK; ++i)
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int x = bs[u] + i, q = q0 + u * NT + tid;
-        if (x < be[u]) {
-          const unsigned long long ki = bkey[x];
-          rank[u] += (ki < kq[u] || (ki == kq[u] && x < q)) ? 1 : 0;
-        }
-      }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int q = q0 + u * NT + tid;
-      for (int x0 = bs[u] + RK; x0 < be[u]; x0 += 8) {  // larger buckets: eight loads in flight
-        unsigned long long k8[8];
-#pragma unroll
-        for (int v = 0; v < 8; ++v) k8[v] = x0 + v < be[u] ? bkey[x0 + v] : ~0ull;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-          const int x = x0 + v;
-          rank[u] += (x < be[u] && (k8[v] < kq[u] || (k8[v] == kq[u] && x < q))) ? 1 : 0;
-        }
-      }
-      if (q < C) {
-        key[bs[u] + rank[u]] = kq[u];
-        ord[bs[u] + rank[u]] = oq[u];
-      }
-    }
-  }
-  __syncthreads();
-  // 3. the top octave, and the highest octave in which two equal mantissas meet
-  int etop = -0x40000000, tie_e = -0x40000000;
-  for (int j0 = 0; j0 < C; j0 += U * NT) {
-    unsigned long long kk[U], kn[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int j = j0 + u * NT + tid;
-      kk[u] = j < C ? key[j] : 0ull;
-      kn[u] = j + 1 < C ? key[j + 1] : 0ull;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int j = j0 + u * NT + tid;
-      if (j < C) {
-        etop = max(etop, kexp(kk[u]));
-        if (j + 1 < C && (kn[u] >> 11) == (kk[u] >> 11)) tie_e = max(tie_e, min(kexp(kk[u]), kexp(kn[u])));
-      }
-    }
-  }
   etop = block_max<NT>(etop, s_i);
-  tie_e = block_max<NT>(tie_e, s_i);
-  const int eT = dexp(T);
-  const unsigned long long mT = (unsigned long long)__double_as_longlong(T) & MANT;
   if (etop - eT > 40) return RC_OTHER;
-  // 4. octaves from the top: each family's run of kill indices, until K are used; in the
-  //    octave of T only the entries of value >= T count.  Thread tid holds the candidates
-  //    [j0, j1) in sorted order: its entry count, one block scan, then its families' runs.
-  auto fam = [&](unsigned long long kj, int E) -> int {
-    const int ej = kexp(kj);
-    if (!(ej >= E && (E > eT || kmant(kj) >= mT))) return 0;
-    const int d = ej - E;
-    return d >= 20 ? KILL_CAP + 1 : min(1 << d, KILL_CAP + 1);
-  };
-  const int P = (C + NT - 1) / NT;
-  const int j0 = min(C, tid * P), j1 = min(C, j0 + P);
-  int base = 0, Es = 0;
+  int tie_e = -0x40000000, base = 0, Es = 0, p = 0, startp = 0;
   bool found = false;
-  for (int E = etop; E >= eT; --E) {
-    int loc = 0;
-    for (int jb = j0; jb < j1; jb += U) {
-      unsigned long long kk[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (jb + u < j1) loc = min(loc + fam(kk[u], E), KILL_CAP + 1);
-    }
-    // a thread's count is clamped above K: the block sums stay in int, and every later
-    // thread still starts at or beyond K
-    int tot;
-    const int ex = block_excl_scan<NT>(loc, s_i, tot);
-    int st = base + ex;
-    for (int jb = j0; jb < j1 && st < K; jb += U) {
-      unsigned long long kk[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int j = jb + u;
-        const int v = j < j1 ? fam(kk[u], E) : 0;
-        if (v > 0 && st < K) {
-          const int hi = min(st + v, K);
-          for (int t = st; t < hi; ++t) A.asg[t] = j;
-          if (st + v >= K) {
-            s_sh[0] = j;
-            s_sh[1] = st;
+  // 2. candidates by decreasing mantissa (then exponent), their order in LDS where it fits
+  unsigned* word = reinterpret_cast<unsigned*>(bcnt) + RO_PAD;
+  if (C <= RO_CAP && order_candidates(C, key, kmin, kmax, eT, reinterpret_cast<unsigned*>(hist), word, s_i, tie_e)) {
+    // octaves from the top: each family's run of kill indices, until K are used; in the octave of T
+    // only the entries of value >= T count.  A wave holds a contiguous run of the order, 64 at a time.
+    (void)block_excl_scan<NT>(above, s_i, above);
+    const int wv = tid / PVD_WAVE, run = ((C + NT - 1) / NT) * PVD_WAVE;
+    const int a = min(C, wv * run), b = min(C, a + run);
+    for (int E = etop; E >= eT && !found; --E) {
+      auto fam = [&](int j) -> int {
+        if (j >= b || (E == eT && j >= above)) return 0;
+        const int d = (int)((word[j] >> 15) & 63u) - (E - eT);
+        return d < 0 ? 0 : d >= 20 ? KILL_CAP + 1 : min(1 << d, KILL_CAP + 1);
+      };
+      int loc = 0;
+      for (int j = a + lane_id(); j < b; j += PVD_WAVE) loc += fam(j);
+      int tot;
+      const int ex = block_excl_scan<NT>(loc, s_i, tot);
+      int st = base + __shfl(ex, 0, PVD_WAVE);
+      for (int j0 = a; j0 < b && st < K; j0 += PVD_WAVE) {
+        const int j = j0 + lane_id(), v = fam(j);
+        int inc;
+        if (!__any(v > 1)) {  // one entry a family, as a rule
+          const unsigned long long one = __ballot(v > 0);
+          inc = __popcll(one & ((2ull << lane_id()) - 1ull));
+        } else {
+          inc = wave_incl_scan(v);
+        }
+        const int from = st + inc - v;
+        if (v > 0 && from < K) {
+          const int o = (int)(word[j] & 0x7FFFu), hi = min(from + v, K);
+          for (int t = from; t < hi; ++t) A.asg[t] = o;
+          if (from + v >= K) {
+            s_sh[0] = o;
+            s_sh[1] = from;
           }
         }
-        st += v;
+        st += __shfl(inc, PVD_WAVE - 1, PVD_WAVE);
+      }
+      base += tot;
+      __syncthreads();
+      if (base >= K) {
+        Es = E;
+        found = true;
       }
     }
-    base += tot;
+  } else {
+    // the order does not fit: keys and slots are moved.  Counting sort on 14 bits of the key
+    //    above its minimum (an order-preserving map of the keys' own range onto the buckets: the
+    //    candidates of a steady state lie in a band about a tenth of an octave wide, which the
+    //    top mantissa bits would crowd into a tenth of the buckets), then each entry ranked
+    //    inside its bucket
+    constexpr int BPT = RCG_BUCKETS / NT;
+    const unsigned long long kspan = kmax - kmin;
+    const int bsh = (kspan >> 14) == 0ull ? 0 : 64 - __clzll((long long)kspan) - 14;
+    auto bucket = [&](unsigned long long k) { return (int)((k - kmin) >> bsh); };  // < RCG_BUCKETS
+    for (int b = tid; b < RCG_BUCKETS; b += NT) bcnt[b] = 0;
     __syncthreads();
-    if (base >= K) {
-      Es = E;
-      found = true;
-      break;
+    for (int q0 = 0; q0 < C; q0 += U * NT) {
+      unsigned long long kk[U];
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        kk[u] = q < C ? key[q] : 0ull;
+      }
+  #pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (q0 + u * NT + tid < C) atomicAdd(&bcnt[bucket(kk[u])], 1);
+    }
+    __syncthreads();
+    int bmax;
+    {
+      int loc = 0, mx = 0;
+      for (int u = 0; u < BPT; ++u) {
+        const int c = bcnt[tid * BPT + u];
+        loc += c;
+        mx = max(mx, c);
+      }
+      int tot;
+      const int ex = block_excl_scan<NT>(loc, s_i, tot);
+      int st = ex;
+      for (int u = 0; u < BPT; ++u) {
+        const int c = bcnt[tid * BPT + u];
+        bcnt[tid * BPT + u] = st;  // bucket starts (each thread rewrites only its own buckets)
+        st += c;
+      }
+      bmax = block_max<NT>(mx, s_i);
+    }
+    if (bmax > RCG_BMAX) return RC_OTHER;  // the in-bucket rank costs bucket size squared
+    for (int q0 = 0; q0 < C; q0 += U * NT) {
+      unsigned long long kk[U];
+      int oo[U];
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        kk[u] = q < C ? key[q] : 0ull;
+        oo[u] = q < C ? ord[q] : 0;
+      }
+  #pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (q0 + u * NT + tid < C) {
+          const int d = atomicAdd(&bcnt[bucket(kk[u])], 1);  // bcnt ends as the bucket ends
+          bkey[d] = kk[u];
+          bord[d] = oo[u];
+        }
+    }
+    __syncthreads();
+    // ranks: U entries per thread at a time, the first RK keys of each one's bucket in flight
+    constexpr int RK = 4;
+    for (int q0 = 0; q0 < C; q0 += U * NT) {
+      unsigned long long kq[U];
+      int oq[U], bs[U], be[U], rank[U];
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        kq[u] = q < C ? bkey[q] : 0ull;
+        oq[u] = q < C ? bord[q] : 0;
+      }
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        const int bk = q < C ? bucket(kq[u]) : 0;
+        bs[u] = q < C ? (bk > 0 ? bcnt[bk - 1] : 0) : 0;
+        be[u] = q < C ? bcnt[bk] : 0;
+        rank[u] = 0;
+      }
+  #pragma unroll
+      for (int i = 0; i < RK; ++i)
+  #pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int x = bs[u] + i, q = q0 + u * NT + tid;
+          if (x < be[u]) {
+            const unsigned long long ki = bkey[x];
+            rank[u] += (ki < kq[u] || (ki == kq[u] && x < q)) ? 1 : 0;
+          }
+        }
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * NT + tid;
+        for (int x0 = bs[u] + RK; x0 < be[u]; x0 += 8) {  // larger buckets: eight loads in flight
+          unsigned long long k8[8];
+  #pragma unroll
+          for (int v = 0; v < 8; ++v) k8[v] = x0 + v < be[u] ? bkey[x0 + v] : ~0ull;
+  #pragma unroll
+          for (int v = 0; v < 8; ++v) {
+            const int x = x0 + v;
+            rank[u] += (x < be[u] && (k8[v] < kq[u] || (k8[v] == kq[u] && x < q))) ? 1 : 0;
+          }
+        }
+        if (q < C) {
+          key[bs[u] + rank[u]] = kq[u];
+          ord[bs[u] + rank[u]] = oq[u];
+        }
+      }
+    }
+    __syncthreads();
+    // 3. the highest octave in which two equal mantissas meet
+    tie_e = -0x40000000;
+    for (int j0 = 0; j0 < C; j0 += U * NT) {
+      unsigned long long kk[U], kn[U];
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + u * NT + tid;
+        kk[u] = j < C ? key[j] : 0ull;
+        kn[u] = j + 1 < C ? key[j + 1] : 0ull;
+      }
+  #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + u * NT + tid;
+        if (j < C) {
+          if (j + 1 < C && (kn[u] >> 11) == (kk[u] >> 11)) tie_e = max(tie_e, min(kexp(kk[u]), kexp(kn[u])));
+        }
+      }
+    }
+    tie_e = block_max<NT>(tie_e, s_i);
+    // 4. octaves from the top: each family's run of kill indices, until K are used; in the
+    //    octave of T only the entries of value >= T count.  Thread tid holds the candidates
+    //    [j0, j1) in sorted order: its entry count, one block scan, then its families' runs.
+    auto fam = [&](unsigned long long kj, int E) -> int {
+      const int ej = kexp(kj);
+      if (!(ej >= E && (E > eT || kmant(kj) >= mT))) return 0;
+      const int d = ej - E;
+      return d >= 20 ? KILL_CAP + 1 : min(1 << d, KILL_CAP + 1);
+    };
+    const int P = (C + NT - 1) / NT;
+    const int j0 = min(C, tid * P), j1 = min(C, j0 + P);
+    for (int E = etop; E >= eT; --E) {
+      int loc = 0;
+      for (int jb = j0; jb < j1; jb += U) {
+        unsigned long long kk[U];
+  #pragma unroll
+        for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
+  #pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (jb + u < j1) loc = min(loc + fam(kk[u], E), KILL_CAP + 1);
+      }
+      // a thread's count is clamped above K: the block sums stay in int, and every later
+      // thread still starts at or beyond K
+      int tot;
+      const int ex = block_excl_scan<NT>(loc, s_i, tot);
+      int st = base + ex;
+      for (int jb = j0; jb < j1 && st < K; jb += U) {
+        unsigned long long kk[U];
+  #pragma unroll
+        for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
+  #pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int j = jb + u;
+          const int v = j < j1 ? fam(kk[u], E) : 0;
+          if (v > 0 && st < K) {
+            const int hi = min(st + v, K);
+            for (int t = st; t < hi; ++t) A.asg[t] = j;
+            if (st + v >= K) {
+              s_sh[0] = j;
+              s_sh[1] = st;
+            }
+          }
+          st += v;
+        }
+      }
+      base += tot;
+      __syncthreads();
+      if (base >= K) {
+        Es = E;
+        found = true;
+        break;
+      }
     }
   }
   if (!found) return RC_FEW;
   if (tie_e >= Es) return RC_OTHER;
-  const int p = s_sh[0], startp = s_sh[1];
+  p = s_sh[0];
+  startp = s_sh[1];
   const int r = K - startp;
   const double cpw = key_weight(key[p]);
   const int cps = ord[p];
   const int Dp = dexp(cpw) - Es;
   const int m = 1 << Dp;
   if (Dp > 13) return RC_OTHER;  // the family's slots must fit the scratch
-  // split depth of each candidate (read by the copy kernel)
-  for (int jb = j0; jb < j1; jb += U) {
-    unsigned long long kk[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int j = jb + u;
-      if (j < j1) {
-        const int ej = kexp(kk[u]);
-        dep[j] = (unsigned char)(ej < Es ? 0 : ej - Es + (j < p ? 1 : 0));
-      }
-    }
-  }
   // 5. the slots of family p: the kill slots of its full levels (any order: the weights
   //    below rank them by slot), then its own
   int* sp = start;
   if (tid == 0) s_sh[3] = 0;
   __syncthreads();
-  for (int t0 = 0; t0 < startp; t0 += U * NT) {
+  for (int t0 = 0; t0 < startp && m > 1; t0 += U * NT) {
     int aa[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -2109,11 +2318,11 @@ __global__ __launch_bounds__(RP_NT) void k_cont_replay(StepArgs<R> A) {
   __shared__ int s_ncur, s_npend, s_nfin, s_fail, s_next;
   __shared__ double s_d[RP_NT / PVD_WAVE];
   __shared__ int s_i[RP_NT / PVD_WAVE];
-  __shared__ int s_K, s_nc;
+  __shared__ int s_K;
   __shared__ int s_subn[2 * LIST_SUB];
   __shared__ double s_a0n, s_a1n;
   __shared__ int s_sh[4];
-  __shared__ int s_hist[TH_BINS];
+  __shared__ int s_hist[std::max(TH_BINS, RO_BUCKETS / 2)];
   const int par = A.par;
   Ctrl* C = A.ctrl;
   const int np1 = par ^ 1;
@@ -2136,12 +2345,13 @@ __global__ __launch_bounds__(RP_NT) void k_cont_replay(StepArgs<R> A) {
     for (int base = 0; base < nwords || base == 0; base += RP_NT * KW) {
       const int span = min(nwords - base, RP_NT * KW);
       const int per = (span + RP_NT - 1) / RP_NT;
-      const int w0 = base + tid * per;
+      // a wave takes a contiguous run of words, 64 at a time
+      const int w0 = base + tid / PVD_WAVE * (per * PVD_WAVE) + lane_id();
       unsigned long long m[KW];
       int pc = 0;
 #pragma unroll
       for (int u = 0; u < KW; ++u) {
-        m[u] = (u < per && w0 + u < base + span) ? A.kmask[w0 + u] : 0ull;
+        m[u] = (u < per && w0 + u * PVD_WAVE < base + span) ? A.kmask[w0 + u * PVD_WAVE] : 0ull;
         pc += __popcll(m[u]);
       }
       if (base == 0) {
@@ -2155,20 +2365,32 @@ __global__ __launch_bounds__(RP_NT) void k_cont_replay(StepArgs<R> A) {
       }
       int tot;
       const int ex = block_excl_scan<RP_NT>(pc, s_i, tot);
-      int o = kbase + ex;
+      int from = kbase + __shfl(ex, 0, PVD_WAVE);
 #pragma unroll
       for (int u = 0; u < KW; ++u) {
-        unsigned long long mm = m[u];
-        while (mm) {
-          const int b = __ffsll((long long)mm) - 1;
-          mm &= mm - 1ull;
-          if (o < KILL_CAP) kl[o] = (w0 + u) * PVD_WAVE + b;
-          ++o;
+        if (u < per) {
+          unsigned long long mm = m[u];
+          const int inc = wave_incl_scan((int)__popcll(mm));
+          int o = from + inc - __popcll(mm);
+          while (mm) {
+            const int b = __ffsll((long long)mm) - 1;
+            mm &= mm - 1ull;
+            if (o < KILL_CAP) kl[o] = (w0 + u * PVD_WAVE) * PVD_WAVE + b;
+            ++o;
+          }
+          from += __shfl(inc, PVD_WAVE - 1, PVD_WAVE);
         }
       }
       kbase += tot;
     }
     const int k = kbase;
+    // the candidate counts of this step, a lane each (one thread's loads would wait for each other);
+    // the next step's weight kernel starts from zero
+    if (tid < 2 * LIST_SUB) {
+      unsigned* cnt = list_count(A, tid / LIST_SUB, tid % LIST_SUB);
+      s_subn[tid] = (int)min(*cnt, (unsigned)SUB_CAP + 1u);
+      *cnt = 0u;
+    }
     {
       // one pass: wave partials, combined by one thread in a fixed order
       constexpr int NW = RP_NT / PVD_WAVE;
@@ -2199,15 +2421,6 @@ __global__ __launch_bounds__(RP_NT) void k_cont_replay(StepArgs<R> A) {
       s_a1n = a1n;
       C->ncopy = 0;
       C->gc_n = 0;
-      // the candidate count of this step; the next step's weight kernel starts from zero
-      s_nc = 0;
-      for (int c = 0; c < LIST_SUB; ++c) {
-        s_subn[c] = (int)min(*list_count(A, 0, c), (unsigned)SUB_CAP + 1u);
-        s_subn[LIST_SUB + c] = (int)min(*list_count(A, 1, c), (unsigned)SUB_CAP + 1u);
-        s_nc += s_subn[c];
-        *list_count(A, 0, c) = 0u;
-        *list_count(A, 1, c) = 0u;
-      }
       C->kills[par] = k;
       C->sumw[par] = a1;
       C->sumwe[par] = a0;
@@ -2261,9 +2474,11 @@ __global__ __launch_bounds__(RP_NT) void k_cont_replay(StepArgs<R> A) {
         A.tr_deaths[step] = code;  // which replay ran (and why the lists did not serve)
       }
       float g = C->cand_g;
+      int nc = 0;
+      for (int c = 0; c < LIST_SUB; ++c) nc += s_subn[c];
       if (!(g > 0.0f)) g = 0.5f;
       if (t0 > 0.0 && cut > 0.0) g = (float)(t0 / cut);
-      else if (C->cand_t > 0.0) g *= s_nc > 0 ? powf((float)s_nc / (float)th_target(K), 0.2f) : 0.5f;
+      else if (C->cand_t > 0.0) g *= nc > 0 ? powf((float)nc / (float)th_target(K), 0.2f) : 0.5f;
       g = fminf(0.98f, fmaxf(0.02f, g));
       C->cand_g = g;
       C->cand_t = cut > 0.0 ? fmax(A.thresh_lo, cut * g) : 0.0;
@@ -2637,11 +2852,13 @@ __global__ __launch_bounds__(TILE) void k_cont_copy(StepArgs<R> A) {
   int ks, o;
   if (gn > 0) {
     const RsgView rv = rsg_view(A.rsg);
-    const int gp = C->gc_p;
+    const int gp = C->gc_p, es = dexp(C->gc_w) - C->gc_dp;
+    const unsigned long long last = weight_key(C->gc_w);
     for (int j = t; j < gn; j += (int)(gridDim.x * TILE)) {  // the candidates may outnumber the threads
       if (j == gp) continue;
-      const int d = rv.dep[j];
-      if (d > 0) A.w[rv.ord[j]] = ldexp(key_weight(rv.key[j]), -d);
+      const unsigned long long k = rv.key[j];
+      const int d = key_depth(k, last, es);
+      if (d > 0) A.w[rv.ord[j]] = ldexp(key_weight(k), -d);
     }
     if (t >= C->ncopy) return;
     ks = A.klist[t];
@@ -2651,7 +2868,8 @@ __global__ __launch_bounds__(TILE) void k_cont_copy(StepArgs<R> A) {
       if (t >= C->gc_start) A.w[ks] = ldexp(C->gc_w, -(C->gc_dp + 1));
     } else {
       o = rv.ord[j];
-      A.w[ks] = ldexp(key_weight(rv.key[j]), -(int)rv.dep[j]);
+      const unsigned long long k = rv.key[j];
+      A.w[ks] = ldexp(key_weight(k), -key_depth(k, last, es));
     }
   } else {
     if (t >= C->ncopy) return;
