@@ -42,6 +42,13 @@ class _NumpyDraws:
         return np.random.random(n)
 
 
+def _shrink(a, n):
+    """The first n rows of an array of this module's own, which gives the rest of its memory back: a
+    large block shrinks in place (a copy of a million walkers took 5 ms, most of it page faults)."""
+    a.resize((n,) + a.shape[1:], refcheck=False)
+    return a
+
+
 class _Logger:
     def __init__(self, fname, overwrite=False, enabled=True):
         self.fl = open(fname, 'w' if overwrite else 'a') if enabled else None
@@ -148,7 +155,7 @@ class DMC_Sim:
             if ss.shape[0] != self.num_walkers:
                 print("WARNING: NUMBER OF STARTING GEOMETRIES DOES NOT EQUAL NUM_WALKERS VARIABLE. MAKE SURE THIS IS"
                       "INTENTIONAL.")
-            coords = ss.copy()
+            coords = ss  # only read: the upload ends before this returns
         if type(self.atoms) is not list:
             self.atoms = [self.atoms]
         if self.masses is None:
@@ -301,7 +308,7 @@ class DMC_Sim:
         N.check(N.load().pvd_sim_get_walkers(self._h, N.ptr(buf), N.ptr(wb), cap, N.byref(n), N.stream_handle()),
                 'pvd_sim_get_walkers')
         n = n.value
-        return buf[:n].copy(), (None if wb is None else wb[:n].copy())
+        return _shrink(buf, n), (None if wb is None else _shrink(wb, n))
 
     @property
     def _walker_coords(self):
@@ -550,9 +557,9 @@ class DMC_Sim:
         N.check(N.load().pvd_sim_desc_end(self._h, N.ptr(desc), N.ptr(par), N.ptr(pw), N.byref(npar),
                                           N.stream_handle()), 'pvd_sim_desc_end')
         k = npar.value
-        rec = dict(coords=par[:k].copy(), desc_wts=desc[:k].copy())
+        rec = dict(coords=_shrink(par, k), desc_wts=_shrink(desc, k))
         if pw is not None:
-            rec['parent_wts'] = pw[:k].copy()
+            rec['parent_wts'] = _shrink(pw, k)
         self.wfns = getattr(self, 'wfns', [])
         self.wfns.append((start_step, rec))
         if self.write_files:
