@@ -427,10 +427,21 @@ template <int H>
 __global__ __launch_bounds__(256) void k_mlp_wgrad(int Din, TrainBuf D) {
   constexpr int TI = H / 64;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = lane >> 4, col = lane & 15, tile = blockIdx.x;
-  const long long k0 = (long long)blockIdx.y * train_slice<H>();
+  const int g = lane >> 4, col = lane & 15;
+  // eight slices and more: all tiles of a slice on one XCD (workgroups go to the eight in turn), whose
+  // L2 then reads the slice's 1.3 MB (H = 256) once, instead of each XCD every slice
+  constexpr int TILES = 2 * TI * TI + TI;
+  const int slices = (int)((D.np + train_slice<H>() - 1) / train_slice<H>());
+  int slice = blockIdx.x / TILES, tile = blockIdx.x % TILES;
+  if (slices >= 8) {
+    const int i = blockIdx.x / 8;
+    slice = (int)(blockIdx.x % 8) + 8 * (i / TILES);
+    tile = i % TILES;
+    if (slice >= slices) return;
+  }
+  const long long k0 = (long long)slice * train_slice<H>();
   const long long k1 = k0 + train_slice<H>() < D.np ? k0 + train_slice<H>() : D.np;
-  float* P = D.P + (long long)blockIdx.y * ((long long)H * Din + 2 * H * H);
+  float* P = D.P + (long long)slice * ((long long)H * Din + 2 * H * H);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   if (tile < 2 * TI * TI) {
     const int l = 1 + tile / (TI * TI), ob = tile / TI % TI * 64 + 32 * (wv >> 1), ib = tile % TI * 64 + 32 * (wv & 1);
@@ -1466,7 +1477,8 @@ int launch_grads(const MlpNet& N, TrainBuf B, float* grads, double* loss_parts, 
   const int D = N.D;
   const unsigned slices = (unsigned)((B.np + train_slice<H>() - 1) / train_slice<H>());
   hipLaunchKernelGGL(k_mlp_fwd_bwd<H>, dim3((unsigned)(B.np / 32)), dim3(2 * H), 0, st, N, B);
-  hipLaunchKernelGGL(k_mlp_wgrad<H>, dim3(2 * (H / 64) * (H / 64) + H / 64, slices), dim3(256), 0, st, D, B);
+  const unsigned rounds = slices >= 8 ? (slices + 7) / 8 * 8 : slices;  // see k_mlp_wgrad
+  hipLaunchKernelGGL(k_mlp_wgrad<H>, dim3((2 * (H / 64) * (H / 64) + H / 64) * rounds), dim3(256), 0, st, D, B);
   const long long blocks = ((long long)H * D + 2 * H * H + 255) / 256 + (4 * H + 16) / 16 + (B.n + 255) / 256 + (loss ? 1 : 0);
   hipLaunchKernelGGL(k_mlp_collect<H>, dim3((unsigned)blocks), dim3(256), 0, st, D, B, grads, loss_parts, loss);
   MHIP(hipGetLastError());
