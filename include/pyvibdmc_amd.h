@@ -184,6 +184,17 @@ int pvd_sim_status(pvd_sim* sim, int32_t* status, int64_t* fail_step, int32_t* n
 int pvd_sim_trajectory(pvd_sim* sim, int64_t t0, int32_t count, double* vref, double* pop,
                        int32_t* births, int32_t* deaths, double* eff_t);
 
+/* Runs of many discrete steps go to launches that keep the walkers on chip and whose workgroups wait
+ * for each other.  Such a launch first waits until all of them run, gate_us microseconds at most;
+ * otherwise a second one takes its steps, with those of its workgroups that start within team_us.
+ * Negative: the defaults (50 000 and up to 42 000 more by chance, 2 000).  gate_us = 0 gives every
+ * launch up, which leaves all steps to the second.  No counterpart in the reference. */
+int pvd_sim_resident_waits(pvd_sim* sim, int64_t gate_us, int64_t team_us);
+/* How the steps so far were run: counts[0] launches of several workgroups with the walkers kept on
+ * chip, counts[1] launches given up for the second form, counts[2] redistributions of the walkers
+ * over the workgroups.  Synchronous.  No counterpart in the reference. */
+int pvd_sim_counts(pvd_sim* sim, int64_t* counts, void* stream);
+
 /* Descendant weighting window (pyvibdmc.py:739-747, 663-672, 856-872).  end() writes
  * desc_wts (host, n_parent), parent coords (host, (n_parent, M, d)) and parent weights
  * (host or NULL). */

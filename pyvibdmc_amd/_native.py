@@ -65,6 +65,8 @@ _SIGS = {
     'pvd_sim_start': (C.c_int, [_P, _P]),
     'pvd_sim_start_external': (C.c_int, [_P, _P, _P]),
     'pvd_sim_run': (C.c_int, [_P, C.c_int32, _P]),
+    'pvd_sim_resident_waits': (C.c_int, [_P, C.c_int64, C.c_int64]),
+    'pvd_sim_counts': (C.c_int, [_P, _P, _P]),
     'pvd_sim_run_timed': (C.c_int, [_P, C.c_int32, _P, C.POINTER(C.c_float), C.POINTER(C.c_int32)]),
     'pvd_bench_plane_copy': (C.c_int, [_P, _P, C.c_int32, C.c_int64, C.c_int64, C.c_int32, _P,
                                        C.POINTER(C.c_float)]),

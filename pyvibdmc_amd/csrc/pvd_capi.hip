@@ -385,6 +385,8 @@ int pvd_sim_create(const pvd_config* cfg, pvd_sim** out) {
     return fail(E_HIP, std::string("init: ") + hipGetErrorString(e));
   }
   s->epoch_next = 1;
+  s->res_gate_wait = RES_WAIT;
+  s->res_team_wait = RES_TEAM_WAIT;
   {
     const char* e = std::getenv("PVD_GRAPHS");
     s->use_graphs = !(e && e[0] == '0');
@@ -665,6 +667,26 @@ int pvd_sim_trajectory(pvd_sim* s, int64_t t0, int32_t count, double* vref, doub
   if (births) HIPCHK(hipMemcpy(births, s->tr_births + t0, sizeof(int) * count, hipMemcpyDeviceToHost));
   if (deaths) HIPCHK(hipMemcpy(deaths, s->tr_deaths + t0, sizeof(int) * count, hipMemcpyDeviceToHost));
   if (eff_t) HIPCHK(hipMemcpy(eff_t, s->tr_dteff + t0, sizeof(double) * count, hipMemcpyDeviceToHost));
+  return 0;
+}
+
+int pvd_sim_resident_waits(pvd_sim* s, int64_t gate_us, int64_t team_us) {
+  if (!s) return fail(E_BAD, "null argument");
+  s->res_gate_wait = gate_us < 0 ? RES_WAIT : 100ull * (unsigned long long)std::min<int64_t>(gate_us, 10000000);
+  s->res_team_wait = team_us < 0 ? RES_TEAM_WAIT : 100ull * (unsigned long long)std::min<int64_t>(team_us, 10000000);
+  return 0;
+}
+
+int pvd_sim_counts(pvd_sim* s, int64_t* counts, void* stream) {
+  if (!s || !counts) return fail(E_BAD, "null argument");
+  unsigned w[RES_SYNCW] = {};
+  if (s->xch) {
+    HIPCHK(hipMemcpyAsync(w, s->xch + RES_XSYNC, sizeof(w), hipMemcpyDeviceToHost, (hipStream_t)stream));
+    HIPCHK(hipStreamSynchronize((hipStream_t)stream));
+  }
+  counts[0] = w[RES_N_OPEN];
+  counts[1] = w[RES_N_CLOSED];
+  counts[2] = w[RES_N_SPREAD];
   return 0;
 }
 

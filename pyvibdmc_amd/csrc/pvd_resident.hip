@@ -10,6 +10,7 @@ constexpr int RES_LDS = 160 * 1024 - 5 * 1024;
 
 struct Instance {
   const void* fn;
+  const void* rest;
   int W, ntmax, stride;
 };
 
@@ -20,8 +21,9 @@ struct Instance {
 // where a walker needs more than the 128 registers a wave of 1024 threads has.
 template <typename R, int NP, bool IS, int MS, int W, int NTM>
 Instance shapes(bool small) {
-  if (small) return Instance{(const void*)k_resident<R, NP, IS, MS, 2, 512, false>, 2, 512, res_stride<R, NP>()};
-  return Instance{(const void*)k_resident<R, NP, IS, MS, W, NTM, true>, W, NTM, res_stride<R, NP>()};
+  const void* rest = (const void*)k_resident_rest<R, NP, IS, MS, NTM>;
+  if (small) return Instance{(const void*)k_resident<R, NP, IS, MS, 2, 512, false>, rest, 2, 512, res_stride<R, NP>()};
+  return Instance{(const void*)k_resident<R, NP, IS, MS, W, NTM, true>, rest, W, NTM, res_stride<R, NP>()};
 }
 
 template <typename R>
@@ -47,7 +49,7 @@ Instance instance(const pvd_sim* s, bool small) {
     if (s->np == 9 && (ms & MS_PES_WATER)) return shapes<R, 9, false, MS_PES_WATER, 6, 512>(small);
     if (s->np == 9) return shapes<R, 9, false, MS_ANY, 6, 512>(small);
   }
-  return Instance{nullptr, 0, 0, 0};
+  return Instance{nullptr, nullptr, 0, 0, 0};
 }
 
 // Workgroups, threads and LDS of the resident launch, or fn = nullptr where it does not serve:
@@ -56,13 +58,14 @@ Instance instance(const pvd_sim* s, bool small) {
 // the grid must be resident at once.
 struct Plan {
   const void* fn;
-  int grid, nt, capl;
+  const void* rest;
+  int grid, nt, capl, capb;
   size_t lds;
 };
 
 template <typename R>
 Plan make_plan(pvd_sim* s, bool who) {
-  Plan P{nullptr, 0, 0, 0, 0};
+  Plan P{nullptr, nullptr, 0, 0, 0, 0, 0};
   const long long n0 = s->cfg.num_walkers;
   const int gmax = std::min(s->cus, RES_MAXG);
   const int share = 256;
@@ -94,9 +97,11 @@ Plan make_plan(pvd_sim* s, bool who) {
     return P;
   }
   P.fn = I.fn;
+  P.rest = I.rest;
   P.grid = g;
   P.nt = nt;
   P.capl = capl;
+  P.capb = capb;
   return P;
 }
 
@@ -145,6 +150,9 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
   A.pop_hi = S.pop_hi;
   A.branch_every = s->cfg.branch_every > 0 ? s->cfg.branch_every : 1;
   A.capl = P.capl;
+  A.capb = P.capb;
+  A.gate_wait = s->res_gate_wait;
+  A.team_wait = s->res_team_wait;
   A.who_on = s->who_on ? 1 : 0;
   A.rng = S.rng;
   A.pes.kind = S.pes.kind;
@@ -168,10 +176,11 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
     A.steps = std::min(RES_STEPS, n_steps - done);
     A.par = (int)(s->next_step & 1);
     void* args[] = {&A};
-    s->res_gate += 2;
-    for (unsigned second = 0; second < (P.grid > 1 ? 2u : 1u); ++second) {
-      A.gate = s->res_gate | second;
-      HIPCHK(hipLaunchCooperativeKernel(P.fn, dim3(P.grid), dim3(P.nt), args, (unsigned)P.lds, st));
+    A.set = (int)(s->res_launches & 1);
+    HIPCHK(hipLaunchCooperativeKernel(P.fn, dim3(P.grid), dim3(P.nt), args, (unsigned)P.lds, st));
+    if (P.grid > 1) {
+      ++s->res_launches;
+      HIPCHK(hipLaunchKernel(P.rest, dim3(P.grid), dim3(P.nt), args, 0, st));
     }
     s->next_step += A.steps;
     s->epoch_next += 2 * (unsigned)A.steps + 2;  // a failed launch retraces its steps under new epochs

@@ -18,11 +18,13 @@
 // Every workgroup waits for every other one, so the launch is cooperative (all workgroups
 // resident, and the runtime runs one cooperative grid of a process at a time).  Another process on
 // the device may still hold some of the CUs, or wait on the rest of them itself, so a launch first
-// makes sure that all its workgroups run: each reports, and workgroup 0 opens the gate, or gives the
-// launch up after a while with nothing changed and its CUs free; a second launch with the same
-// arguments then does the steps (it ends at once where the first did them).  Waits are bounded and
-// end in ST_SPIN.  Records are single 64-bit words (epoch | payload) stored and read with relaxed
-// agent-scope atomics, so a word is valid by itself and publishing needs no fence.
+// makes sure that all its workgroups run: they are counted, and the first of them opens the gate when
+// the count is full, or closes it after a while with nothing changed and the CUs free.  A second
+// launch with the same arguments, k_resident_rest, ends at once behind an open gate; behind a closed
+// one the workgroups of it that do run, one or all, take the steps, with the walkers in the global
+// planes.  Waits on other workgroups' records are bounded and end in ST_SPIN.  Records are single
+// 64-bit words (epoch | payload) stored and read with relaxed agent-scope atomics, so a word is valid
+// by itself and publishing needs no fence.
 #pragma once
 #include "pvd_sim.hpp"
 
@@ -32,13 +34,25 @@ constexpr int RES_MAXG = 256;  // workgroups of a resident launch
 // least steps between redistributions that only even out the rounds: one costs 15 us at 1M walkers,
 // unevenness a round of five (plain 1M: 17.0 us a step at 16, 15.9 at 32, 16.1 at 48)
 constexpr int RES_REB = 32;
-// words of the exchange area: records (4 per workgroup, by step parity), acceptance counts (by
-// parity), barrier words, arrivals, and the gate
-constexpr size_t RES_XWORDS = (size_t)RES_MAXG * (2 * 4 + 2 + 1 + 1) + 1;
-// how long workgroup 0 waits for the others, in ticks of 10 ns: in the first launch 0.2 s and up to
-// 0.17 s more by chance (two processes that wait on each other's CUs should not give up together), in
-// the second, which has nothing behind it, and for the gate itself 60 s
-constexpr unsigned long long RES_WAIT1 = 20000000ull, RES_WAIT1_MORE = 1ull << 24, RES_WAIT2 = 6000000000ull;
+// Exchange area, in 64-bit words: records (4 per workgroup, by step parity), acceptance counts (by
+// parity), barrier words; then two sets of RES_SET 32-bit words (the launches of a simulation use them
+// in turn, each clearing the next one's), then the simulation's own words.
+constexpr size_t RES_XSYNC = (size_t)RES_MAXG * (2 * 4 + 2 + 1);
+// words of a set, each on a line of its own: workgroups that reported, the gate, workgroups that
+// joined the second launch (RES_SHUT: no more), how many take part
+enum : int { RES_ARRIVED = 0, RES_GATE = 32, RES_JOINED = 64, RES_TEAM = 96, RES_SET = 128 };
+// the simulation's words, behind the sets: the last gate was closed, launches whose gate opened and
+// was closed, redistributions of the walkers
+enum : int { RES_CLOSED = 2 * RES_SET, RES_N_OPEN, RES_N_CLOSED, RES_N_SPREAD, RES_SYNCW };
+constexpr size_t RES_XWORDS = RES_XSYNC + (RES_SYNCW + 1) / 2;
+constexpr unsigned RES_OPEN = 1u, RES_SHUT = 0x80000000u;
+// How long the first workgroup waits for the others, in ticks of 10 ns: at the gate 50 ms and up to
+// 42 ms more by chance (two processes that wait on each other's CUs should not give up together),
+// longer than another launch of this kind holds its CUs; a 64th of that where the last gate was
+// closed.  In the second launch, which goes on with those that are there, 2 ms.  Nobody waits for
+// the first workgroup's word longer than 60 s.
+constexpr unsigned long long RES_WAIT = 5000000ull, RES_WAIT_MORE = 1ull << 22, RES_TEAM_WAIT = 200000ull,
+                             RES_WAIT_MAX = 6000000000ull;
 constexpr unsigned RES_CLAMP = 1u << 22;  // a workgroup's published count: beyond any population bound served
 constexpr long long RES_SPIN = 1ll << 24;
 
@@ -69,8 +83,9 @@ struct ResArgs {
   int* tr_deaths;
   long long cap, tmax;
   double dt, alpha, n0, pop_lo, pop_hi;
-  int par, branch_every, steps, capl, who_on;
-  unsigned gate;  // tag of this launch's gate: even for a first launch, odd for the second
+  int par, branch_every, steps, capl, capb, who_on;
+  int set;                                    // which set of words this launch uses
+  unsigned long long gate_wait, team_wait;  // see RES_WAIT
   Rng rng;
   PesArgs<R> pes;
   TrialArgs<R> trial;
@@ -241,13 +256,15 @@ __global__ __launch_bounds__(NTMAX) void k_resident(ResArgs<R> A) {
     asm volatile("" : "+s"(p));
     return p;
   };
-  if (A.ctrl->status != ST_OK) return;
-  const bool second = (A.gate & 1u) != 0u;
-  {
-    uint64_t* xarr = A.xch + (size_t)RES_MAXG * 11;
-    if (second && ld_relaxed(xarr + RES_MAXG) == (((uint64_t)(A.gate - 1u) << 32) | 1u)) return;
-    if (G > 1 && tid == 0) st_relaxed(xarr + blk, (uint64_t)A.gate);
+  bool first = false;  // the workgroup that watches the gate (thread 0)
+  const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+  if (G > 1 && tid == 0) {
+    unsigned* sync = reinterpret_cast<unsigned*>(A.xch + RES_XSYNC);
+    if (blk == 0)  // nobody uses the other set: the launches before this one have ended
+      for (int k = 0; k < 4; ++k) st_relaxed_u(sync + (A.set ^ 1) * RES_SET + 32 * k, 0u);
+    if (A.ctrl->status == ST_OK) first = fetch_add_relaxed(sync + A.set * RES_SET + RES_ARRIVED, 1u) == 0u;
   }
+  if (A.ctrl->status != ST_OK) return;
   int par = A.par;
   const int be = A.branch_every, n0i = (int)A.n0;
   const double pop_hi = A.pop_hi, pop_lo = A.pop_lo, n0 = A.n0, alpha = A.alpha;
@@ -365,36 +382,32 @@ __global__ __launch_bounds__(NTMAX) void k_resident(ResArgs<R> A) {
   }
   load_share();
   if (G > 1) {
-    uint64_t* xarr = xch + (size_t)RES_MAXG * 11;
-    uint64_t* xgate = xarr + RES_MAXG;
-    const unsigned gate = cold()->gate;
-    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    if (blk == 0) {
-      const unsigned long long wait = second ? RES_WAIT2 : RES_WAIT1 + (t0 & (RES_WAIT1_MORE - 1));
-      __syncthreads();  // s_late is clear
-      for (int r = tid; r < G; r += NT)
-        while (ld_relaxed(xarr + r) != (uint64_t)gate) {
-          if (__builtin_amdgcn_s_memrealtime() - t0 > wait) {
-            s_late = 1;
+    if (tid == 0) {
+      unsigned* sync = reinterpret_cast<unsigned*>(xch + RES_XSYNC);
+      unsigned* set = sync + cold()->set * RES_SET;
+      unsigned f = 0;
+      if (first) {
+        const unsigned long long most = cold()->gate_wait + (cold()->gate_wait ? t0 & (RES_WAIT_MORE - 1) : 0);
+        const unsigned long long wait = ld_relaxed_u(sync + RES_CLOSED) ? most >> 6 : most;
+        f = RES_OPEN;
+        while (wait == 0 || ld_relaxed_u(set + RES_ARRIVED) != (unsigned)G) {
+          if (__builtin_amdgcn_s_memrealtime() - t0 >= wait) {
+            f = RES_SHUT;
             break;
           }
           __builtin_amdgcn_s_sleep(1);
         }
-      __syncthreads();
-      if (tid == 0) st_relaxed(xgate, ((uint64_t)gate << 32) | (s_late ? 2u : 1u));
-    } else if (tid == 0) {
-      uint64_t f = ld_relaxed(xgate);
-      while ((unsigned)(f >> 32) != gate && __builtin_amdgcn_s_memrealtime() - t0 < 2 * RES_WAIT2) {
-        __builtin_amdgcn_s_sleep(1);
-        f = ld_relaxed(xgate);
+        st_relaxed_u(set + RES_GATE, f);
+        st_relaxed_u(sync + RES_CLOSED, f == RES_SHUT ? 1u : 0u);
+        fetch_add_relaxed(sync + (f == RES_OPEN ? RES_N_OPEN : RES_N_CLOSED), 1u);
+      } else {
+        while ((f = ld_relaxed_u(set + RES_GATE)) == 0u && __builtin_amdgcn_s_memrealtime() - t0 < RES_WAIT_MAX)
+          __builtin_amdgcn_s_sleep(1);
       }
-      s_late = f == (((uint64_t)gate << 32) | 1u) ? 0 : 1;
+      s_late = f == RES_OPEN ? 0 : 1;
     }
     __syncthreads();
-    if (s_late) {
-      if (second && blk == 0) lost();
-      return;
-    }
+    if (s_late) return;
   }
   __syncthreads();
 
@@ -695,6 +708,7 @@ __global__ __launch_bounds__(NTMAX) void k_resident(ResArgs<R> A) {
       });
       finish();
       if (last) break;
+      if (blk == 0 && tid == 0) fetch_add_relaxed(reinterpret_cast<unsigned*>(xch + RES_XSYNC) + RES_N_SPREAD, 1u);
       since = 0;
       if (!meet(epoch)) {
         lost();
@@ -762,6 +776,338 @@ __global__ __launch_bounds__(NTMAX) void k_resident(ResArgs<R> A) {
       C->status_step = (long long)step;
       C->status = fail;
     }
+  }
+}
+
+// The steps of a launch whose gate was closed, by those of G workgroups that run.  They take the G
+// shares of k_resident in turn, with the walkers in the global planes, and follow its partition and
+// its sums, so the results are the same whoever takes part.  A step is two passes over the shares (one
+// more with importance sampling) and a meeting; it is bound by those and by HBM.
+template <typename R, int NP, bool IS, int MS, int NTMAX>
+__global__ __launch_bounds__(NTMAX) void k_resident_rest(ResArgs<R> A) {
+  __shared__ double s_d[16];
+  __shared__ __align__(16) int4 s_t[16];
+  __shared__ int4 s_res[4];
+  __shared__ double s_s0[4], s_vref;
+  __shared__ int s_nb[4], s_acc[4], s_late, s_rank, s_team;
+  // the shares: first slot and walkers now; copies, and those of the 64 records' earlier shares
+  __shared__ int s_base[RES_MAXG], s_cnt[RES_MAXG], s_tot[RES_MAXG], s_ex[RES_MAXG];
+  const int NT = blockDim.x, G = gridDim.x, tid = threadIdx.x;
+  const int ln = lane_id(), wv = __builtin_amdgcn_readfirstlane(tid / PVD_WAVE), nwv = NT / PVD_WAVE;
+  unsigned* sync = reinterpret_cast<unsigned*>(A.xch + RES_XSYNC);
+  unsigned* set = sync + A.set * RES_SET;
+  if (A.ctrl->status != ST_OK || ld_relaxed_u(set + RES_GATE) != RES_SHUT) return;
+  if (tid == 0) {
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    const unsigned at = fetch_add_relaxed(set + RES_JOINED, 1u);
+    unsigned team = 0;
+    if (at == 0u) {
+      while (ld_relaxed_u(set + RES_JOINED) < (unsigned)G && __builtin_amdgcn_s_memrealtime() - t0 < A.team_wait)
+        __builtin_amdgcn_s_sleep(1);
+      team = __hip_atomic_fetch_or(set + RES_JOINED, RES_SHUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      st_relaxed_u(set + RES_TEAM, team);
+    } else if (!(at & RES_SHUT)) {
+      while ((team = ld_relaxed_u(set + RES_TEAM)) == 0u && __builtin_amdgcn_s_memrealtime() - t0 < RES_WAIT_MAX)
+        __builtin_amdgcn_s_sleep(1);
+    }
+    s_rank = (int)at;
+    s_team = (int)team;  // 0: too late to take part
+    s_late = 0;
+    s_vref = A.ctrl->vref[A.par];
+  }
+  if (tid < 16) {
+    s_d[tid] = 0.0;
+    s_t[tid] = int4{0, 0, 0, 0};
+    if (tid < 4) {
+      s_res[tid] = int4{0, 0, 0, 0};
+      s_s0[tid] = 0.0;
+      s_nb[tid] = 0;
+      s_acc[tid] = 0;
+    }
+  }
+  __syncthreads();
+  const int rank = s_rank, team = s_team;
+  if (team == 0) return;
+  int par = A.par, n = A.ctrl->n[par], since = 0;
+  unsigned long long step = A.ctrl->step[par];
+  unsigned epoch = A.ctrl->epoch[par];
+  double eff = A.ctrl->eff_t;
+  const unsigned long long end = step + (unsigned long long)A.steps;
+  const int be = A.branch_every;
+  // what the passes leave for each other, by slot: the copies, with importance sampling the energy
+  int* cs = reinterpret_cast<int*>(A.ext);
+  R* es = A.ext + A.cap;
+  auto shares = [&]() {
+    for (int v = tid; v < G; v += NT) {
+      s_base[v] = (int)((long long)n * v / G);
+      s_cnt[v] = (int)((long long)n * (v + 1) / G) - s_base[v];
+    }
+  };
+  shares();
+  __syncthreads();
+  for (; step < end;) {
+    const bool branch = be <= 1 || step % (unsigned long long)be == 0;
+    const double vref = s_vref;
+    double dte = A.dt;
+    const R* src = A.buf[par];
+    if constexpr (IS) {
+      uint64_t* xacc = A.xch + (size_t)RES_MAXG * (8 + (step & 1));
+      R* mv = A.buf[par];
+      for (int v = rank; v < G; v += team) {
+        const int base = s_base[v], cnt = s_cnt[v];
+        int acc = 0;
+        for (int k = 0; k * NT < cnt; ++k) {
+          const int i = base + k * NT + tid;
+          bool a = false;
+          if (k * NT + tid < cnt) {
+            R y[NP], disp[NP];
+            double um, ub;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) y[p] = mv[p * A.cap + i];
+            draw_step<R, NP, false, true>(A, (long long)i, step, disp, um, ub, false);
+            const R ke = is_move_fast<R, NP, MS>(A, disp, um, y, a);
+            const R pot = pes_eval_s<R, NP, MS>(A.pes, y);
+            es[i] = pot + ke;
+            if (a) {
+#pragma unroll
+              for (int p = 0; p < NP; ++p) mv[p * A.cap + i] = y[p];
+            }
+          }
+          acc += __popcll(__ballot(a));
+        }
+        if (ln == 0) s_t[wv].x = acc;
+        __syncthreads();
+        if (wv == 0) {
+          const int t = dpp_sum16(s_t[ln & 15].x);
+          if (ln == 0) st_relaxed(xacc + v, ((uint64_t)epoch << 32) | (unsigned)t);
+        }
+        __syncthreads();
+      }
+      for (int g = wv; g * PVD_WAVE < G; g += nwv) {
+        const int r = g * PVD_WAVE + ln;
+        uint64_t f = 0;
+        if (r < G) {
+          f = ld_relaxed(xacc + r);
+          if (!res_poll(xacc + r, epoch, f)) s_late = 1;
+        }
+        const int got = dpp_sum((int)(uint32_t)f);
+        if (ln == 0) s_acc[g] = got;
+      }
+      __syncthreads();
+      dte = dte * ((double)(unsigned)((s_acc[0] + s_acc[1]) + (s_acc[2] + s_acc[3])) / (double)n);
+    }
+    // copies and the shares' records
+    uint64_t* rec = A.xch + (size_t)(step & 1) * RES_MAXG * 4;
+    for (int v = rank; v < G; v += team) {
+      const int base = s_base[v], cnt = s_cnt[v];
+      double sce = 0.0;
+      int bad = 0, copies = 0, births = 0;
+      for (int k = 0; k * NT < cnt; ++k) {
+        const int i = base + k * NT + tid;
+        if (k * NT + tid < cnt) {
+          double E;
+          int c = 1;
+          if constexpr (IS) {
+            E = (double)es[i];
+            if (branch) {
+              const float u = (float)draw_u<R, false>(A, (long long)i, step, RNG_BRANCH);
+              c = branch_copies<true>(E, vref, dte, (double)u, A.pop_hi, bad);
+            }
+          } else {
+            R y[NP], disp[NP];
+            double um, ub;
+            draw_step<R, NP, false, false>(A, (long long)i, step, disp, um, ub, branch);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) y[p] = src[p * A.cap + i] + disp[p];
+            E = (double)pes_eval_s<R, NP, MS>(A.pes, y);
+            if (branch) c = branch_copies<sizeof(R) == 4>(E, vref, dte, ub, A.pop_hi, bad);
+          }
+          cs[i] = c;
+          copies += c;
+          births += c > 1 ? c - 1 : 0;
+          sce += (double)c * E;
+        }
+      }
+      copies = dpp_sum(copies);
+      births = dpp_sum(births);
+      sce = dpp_sum(sce);
+      const bool anybad = __any(bad != 0);
+      if (ln == 0) {
+        s_t[wv] = int4{(int)min((unsigned)copies, RES_CLAMP), births, anybad ? 1 : 0, 0};
+        s_d[wv] = sce;
+      }
+      __syncthreads();
+      if (wv == 0) {
+        const int4 wt = s_t[ln & 15];
+        const uint64_t bits = (uint64_t)__double_as_longlong(dpp_sum16(s_d[ln & 15]));
+        const int total = dpp_sum16(wt.x);
+        uint32_t word = ((uint32_t)dpp_sum16(wt.y) & 0x7FFFFFFFu) | (__any(wt.z != 0) ? 0x80000000u : 0u);
+        word = ln == 2 ? (uint32_t)bits : word;
+        word = ln == 1 ? (uint32_t)(bits >> 32) : word;
+        word = ln == 0 ? min((unsigned)total, RES_CLAMP) : word;
+        if (ln < 4) st_relaxed(rec + 4 * v + ln, ((uint64_t)epoch << 32) | word);
+      }
+      __syncthreads();
+    }
+    // all records, reduced as in k_resident
+    for (int g = wv; g * PVD_WAVE < G; g += nwv) {
+      const int r = g * PVD_WAVE + ln;
+      int tot = 0, nbt = 0, flag = 0;
+      double s0 = 0.0;
+      if (r < G) {
+        uint64_t f[4];
+        bool ok = true;
+        static_for<4>([&](auto J) {
+          f[J] = ld_relaxed(rec + 4 * r + J);
+          ok = res_poll(rec + 4 * r + J, epoch, f[J]) && ok;
+        });
+        if (!ok) s_late = 1;
+        tot = (int)(uint32_t)f[0];
+        s0 = __longlong_as_double((long long)(f[1] << 32 | (uint64_t)(uint32_t)f[2]));
+        nbt = (int)((uint32_t)f[3] & 0x7FFFFFFFu);
+        flag = (int)((uint32_t)f[3] >> 31);
+      }
+      const int inc = dpp_scan(tot), mx = dpp_max(tot);
+      if (r < G) {
+        s_tot[r] = tot;
+        s_ex[r] = inc - tot;
+      }
+      nbt = dpp_sum(nbt);
+      s0 = dpp_sum(s0);
+      const bool anyflag = __any(flag != 0);
+      if (ln == 0) {
+        s_res[g] = int4{lane_of(inc, 63), 0, mx, anyflag ? 1 : 0};
+        s_s0[g] = s0;
+        s_nb[g] = nbt;
+      }
+    }
+    __syncthreads();
+    const int tot = (s_res[0].x + s_res[1].x) + (s_res[2].x + s_res[3].x);
+    const int mx = max(max(s_res[0].z, s_res[1].z), max(s_res[2].z, s_res[3].z));
+    int st = ST_OK;
+    if (s_late) st = ST_SPIN;
+    else if (s_res[0].w | s_res[1].w | s_res[2].w | s_res[3].w) st = ST_WEIGHT;
+    else if ((double)tot < A.pop_lo || (double)tot > A.pop_hi) st = ST_POP;
+    else if (tot > A.cap) st = ST_CAPACITY;
+    if (st != ST_OK) {
+      // the walkers are those of the failed step, in place (with importance sampling, moved)
+      if (tid == 0 && (rank == 0 || st == ST_SPIN)) {
+        Ctrl* C = A.ctrl;
+        C->n[par] = n;
+        C->vref[par] = vref;
+        C->step[par] = step;
+        C->epoch[par] = epoch + 1;
+        C->eff_t = eff;
+        C->status_step = (long long)step;
+        C->status = st;
+      }
+      return;
+    }
+    auto first_slot = [&](int v) {  // of share v's survivors
+      int pre = s_ex[v];
+      for (int g = 0; g < v / PVD_WAVE; ++g) pre += s_res[g].x;
+      return pre;
+    };
+    // survivors to their np.repeat positions, share by share
+    for (int v = rank; v < G; v += team) {
+      const int base = s_base[v], cnt = s_cnt[v];
+      int at = first_slot(v);
+      R* dst = A.buf[par ^ 1];
+      const int* wsrc = A.who[par];
+      int* wdst = A.who[par ^ 1];
+      for (int k = 0; k * NT < cnt; ++k) {
+        const int i = base + k * NT + tid;
+        const int c = k * NT + tid < cnt ? cs[i] : 0;
+        int t, nb;
+        const int o = wave_copies(c, t, nb);
+        if (ln == 0) s_t[wv].x = t;
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < nwv; ++w) {
+          const int x = s_t[w].x;
+          before += w < wv ? x : 0;
+          all += x;
+        }
+        if (c > 0) {
+          R y[NP];
+#pragma unroll
+          for (int p = 0; p < NP; ++p) y[p] = src[p * A.cap + i];
+          if constexpr (!IS) {
+            R disp[NP];
+            double um, ub;
+            draw_step<R, NP, false, false>(A, (long long)i, step, disp, um, ub, branch);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) y[p] = y[p] + disp[p];
+          }
+          const int w = A.who_on ? wsrc[i] : 0;
+          for (int q = 0; q < c; ++q) {
+            const int to = at + before + o + q;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) dst[p * A.cap + to] = y[p];
+            if (A.who_on) wdst[to] = w;
+          }
+        }
+        at += all;
+        __syncthreads();
+      }
+    }
+    const double vbar = ((s_s0[0] + s_s0[1]) + (s_s0[2] + s_s0[3])) / (double)tot;
+    const double corr = (double)(tot - (int)A.n0) / A.n0;
+    const double vnew = vbar - (A.alpha * corr);
+    if (IS && (long long)step < A.tmax) eff = branch ? (step == 0 ? 0.0 : eff) + dte : 0.0;
+    if (rank == 0 && tid == 0 && (long long)step < A.tmax) {
+      A.tr_vref[step] = vnew;
+      A.tr_pop[step] = (double)tot;
+      const int nbt = (s_nb[0] + s_nb[1]) + (s_nb[2] + s_nb[3]);
+      A.tr_births[step] = nbt;
+      A.tr_deaths[step] = n + nbt - tot;
+      if (IS) A.tr_dteff[step] = eff;
+    }
+    // the partition that k_resident would have now
+    const int even = (tot + G - 1) / G;
+    ++since;
+    const bool spread = mx > A.capb || ((mx + NT - 1) / NT > (even + NT - 1) / NT && since >= RES_REB);
+    __syncthreads();
+    n = tot;
+    if (spread) {
+      since = 0;
+      shares();
+    } else {
+      for (int v = tid; v < G; v += NT) {
+        s_base[v] = first_slot(v);
+        s_cnt[v] = s_tot[v];
+      }
+    }
+    if (tid == 0) s_vref = vnew;
+    par ^= 1;
+    ++step;
+    ++epoch;
+    // everyone's survivors before anyone's next step
+    uint64_t* xbar = A.xch + (size_t)RES_MAXG * 10;
+    store_complete();
+    __syncthreads();
+    if (tid == 0) {
+      fence_release();
+      st_relaxed(xbar + rank, ((uint64_t)epoch << 32) | 1u);
+    }
+    for (int r = tid; r < team; r += NT) {
+      uint64_t f = ld_relaxed(xbar + r);
+      if (!res_poll(xbar + r, epoch, f)) s_late = 1;
+    }
+    __syncthreads();
+    fence_acquire();
+  }
+  Ctrl* C = A.ctrl;
+  if (rank == 0 && tid == 0) {
+    C->n[par] = n;
+    C->vref[par] = s_vref;
+    C->step[par] = step;
+    C->epoch[par] = epoch;
+    C->eff_t = eff;
+  }
+  if (tid == 0 && s_late) {
+    C->status_step = (long long)step;
+    C->status = ST_SPIN;
   }
 }
 

@@ -60,7 +60,8 @@ struct pvd_sim {
   uint64_t* drec;
   unsigned* accs;
   uint64_t* xch;  // exchange words of the resident steps (discrete weighting)
-  unsigned res_gate;  // tag of the last resident launch
+  unsigned res_launches;  // resident launches of more than one workgroup so far
+  unsigned long long res_gate_wait, res_team_wait;  // see RES_WAIT
   double* tr_vref;
   double* tr_pop;
   double* tr_dteff;
