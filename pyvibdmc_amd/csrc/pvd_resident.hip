@@ -88,10 +88,8 @@ Plan make_plan(pvd_sim* s, bool who) {
     (void)hipGetLastError();
     return P;
   }
-  int per_cu = 0, coop = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, I.fn, nt, P.lds) != hipSuccess ||
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, I.fn, nt, P.lds) != hipSuccess ||
       (long long)per_cu * s->cus < g) {
     (void)hipGetLastError();
     return P;
@@ -107,11 +105,10 @@ Plan make_plan(pvd_sim* s, bool who) {
 
 }  // namespace
 
-// Steps of one cooperative launch at most (a bound on how long one kernel runs: about 60 ms at a
-// million walkers), and the fewest for which it is used: a call costs about 40 us more than a step
-// kernel's launch does (the cooperative queue, the second launch, walkers in and out).  us a step
-// in calls of 16 steps, here and launch per step: water 1 000 walkers 6.7, 9.0; 100 000 6.9, 10.5;
-// 1 000 000 17.5, 20.9; with importance sampling 34.5, 51.1; cluster 200 000 13.2, 17.3.
+// Steps of one launch at most (a bound on how long one kernel runs: about 60 ms at a million
+// walkers), and the fewest for which it is used: a call costs about 20 us more than a step kernel's
+// launch does (the second launch, walkers in and out).  us a step in calls of 16 steps, here and
+// launch per step: @@
 constexpr int RES_STEPS = 4096;
 constexpr int RES_MIN = 16;
 
@@ -177,7 +174,7 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
     A.par = (int)(s->next_step & 1);
     void* args[] = {&A};
     A.set = (int)(s->res_launches & 1);
-    HIPCHK(hipLaunchCooperativeKernel(P.fn, dim3(P.grid), dim3(P.nt), args, (unsigned)P.lds, st));
+    HIPCHK(hipLaunchKernel(P.fn, dim3(P.grid), dim3(P.nt), args, P.lds, st));
     if (P.grid > 1) {
       ++s->res_launches;
       HIPCHK(hipLaunchKernel(P.rest, dim3(P.grid), dim3(P.nt), args, 0, st));

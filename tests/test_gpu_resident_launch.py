@@ -1,0 +1,77 @@
+"""What launching the resident discrete steps costs: the first of a process, and two simulations on
+two streams."""
+import os
+import subprocess
+import sys
+import threading
+import time
+
+import pytest
+
+from tests.conftest import ROOT
+from tests.test_gpu_resident import make
+
+pytestmark = pytest.mark.gpu
+
+FIRST = """
+import sys, time
+sys.path.insert(0, {root!r})
+import torch
+from tests.test_gpu_resident import make
+from pyvibdmc_amd import _native as N
+sim = make('water', 5000, 1000, 'fp32')
+sim._start()
+N.check(N.load().pvd_sim_run(sim._h, 5, N.stream_handle()))
+for _ in range(5):
+    torch.cuda.synchronize()
+    t = time.perf_counter()
+    N.check(N.load().pvd_sim_run(sim._h, 150, N.stream_handle()))
+    torch.cuda.synchronize()
+    print((time.perf_counter() - t) * 1e6)
+"""
+
+
+def test_first_resident_launch_of_a_process():
+    """150 steps of 5 000 walkers take 0.7 ms.  The first launch of a process also brings the code to
+    the device (0.4 ms a code object and 1 ms a megabyte); a queue of its own would be 3.7 ms more."""
+    out = subprocess.run([sys.executable, '-c', FIRST.format(root=ROOT)], capture_output=True, text=True, timeout=100,
+                         env=dict(os.environ), cwd=ROOT)
+    assert out.returncode == 0, out.stderr
+    us = [float(x) for x in out.stdout.split()]
+    print('us', us)
+    assert us[0] - min(us[1:]) < 3000
+
+
+def test_small_simulations_on_two_streams_overlap():
+    """Two simulations of 5 000 walkers (20 workgroups each) on two streams run beside each other."""
+    import torch
+    from pyvibdmc_amd import _native as N
+    lib = N.load()
+    sims = [make('water', 5000, 10 ** 5, 'fp32', seed=s) for s in (1, 2)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+
+    def go(i):
+        with torch.cuda.stream(streams[i]):
+            if not sims[i]._started:
+                sims[i]._start()
+            N.check(lib.pvd_sim_run(sims[i]._h, 3000, N.stream_handle()))
+            streams[i].synchronize()
+
+    def together():
+        th = [threading.Thread(target=go, args=(i,)) for i in range(2)]
+        [t.start() for t in th]
+        [t.join() for t in th]
+
+    def ms(f):
+        t = time.perf_counter()
+        f()
+        return (time.perf_counter() - t) * 1e3
+
+    go(0), go(1)
+    turn = min(ms(lambda: (go(0), go(1))) for _ in range(3))
+    both = min(ms(together) for _ in range(3))
+    print('in turn', turn, 'together', both)
+    assert both < 0.8 * turn
+    for s in sims:
+        assert s._status()[0] == 0
