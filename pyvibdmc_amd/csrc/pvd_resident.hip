@@ -108,7 +108,8 @@ Plan make_plan(pvd_sim* s, bool who) {
 // Steps of one launch at most (a bound on how long one kernel runs: about 60 ms at a million
 // walkers), and the fewest for which it is used: a call costs about 20 us more than a step kernel's
 // launch does (the second launch, walkers in and out).  us a step in calls of 16 steps, here and
-// launch per step: @@
+// launch per step: water 1 000 walkers 4.3, 9.0; 100 000 4.8, 10.7;
+// 1 000 000 15.3, 21.0; with importance sampling 31.4, 50.5; cluster with it, 500 000 36.0, 56.9.
 constexpr int RES_STEPS = 4096;
 constexpr int RES_MIN = 16;
 
