@@ -190,9 +190,8 @@ int pvd_sim_trajectory(pvd_sim* sim, int64_t t0, int32_t count, double* vref, do
  * Negative: the defaults (50 000 and up to 42 000 more by chance, 2 000).  gate_us = 0 gives every
  * launch up, which leaves all steps to the second.  No counterpart in the reference. */
 int pvd_sim_resident_waits(pvd_sim* sim, int64_t gate_us, int64_t team_us);
-/* How the steps so far were run: counts[0] launches of several workgroups with the walkers kept on
- * chip, counts[1] launches given up for the second form, counts[2] redistributions of the walkers
- * over the workgroups.  Synchronous.  No counterpart in the reference. */
+/* How the steps so far were run: counts[0] launches with the walkers kept on chip, counts[1]
+ * launches given up for the second form, counts[2] redistributions of the walkers over the workgroups.  Synchronous.  No counterpart in the reference. */
 int pvd_sim_counts(pvd_sim* sim, int64_t* counts, void* stream);
 
 /* Descendant weighting window (pyvibdmc.py:739-747, 663-672, 856-872).  end() writes

@@ -5,7 +5,8 @@ parallel and links them into ``pyvibdmc_amd/libpyvibdmc_amd.so`` in place:
 * ``pvd_capi.hip``: the C ABI entry points and auxiliary kernels;
 * ``pvd_step_f32.hip`` / ``pvd_step_f64.hip``: the step kernels and their launches for
   float and double walkers;
-* ``pvd_resident.hip``: many discrete steps per launch, the walkers kept on chip;
+* ``pvd_resident.hip``: many discrete steps per launch, the walkers kept on chip, and
+  ``pvd_resident_form.hip``: its kernels, an object per form;
 * ``pvd_mlp.hip``: the surrogate kernels.
 """
 import os
@@ -23,13 +24,15 @@ ARCH = os.environ.get('PVD_OFFLOAD_ARCH', 'gfx950')
 FLAGS = ['-O3', f'--offload-arch={ARCH}', '-std=c++17', '-fPIC', '-ffp-contract=off',
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops']
 
-# pvd_resident.hip: machine-level hoisting moves the constants of the mathematical functions out of
+# pvd_resident_form.hip: machine-level hoisting moves the constants of the mathematical functions out of
 # the step loop and spills them (FP64 triatomics: 104 spilled registers against none).
-EXTRA = {'pvd_resident.hip': ['-mllvm', '-disable-machine-licm']}
+NO_HOIST = ['-mllvm', '-disable-machine-licm']
+FORMS = 12  # RF_COUNT of pvd_resident.hpp
 
-TARGETS = [
-    ('libpyvibdmc_amd.so', ['pvd_capi.hip', 'pvd_step_f32.hip', 'pvd_step_f64.hip', 'pvd_resident.hip', 'pvd_mlp.hip']),
-]
+# object, source and the flags that it adds
+UNITS = [(s + '.o', s + '.hip', []) for s in ('pvd_capi', 'pvd_step_f32', 'pvd_step_f64', 'pvd_resident', 'pvd_mlp')] + \
+    [(f'pvd_resident_{k}.o', 'pvd_resident_form.hip', NO_HOIST + [f'-DPVD_FORM={k}']) for k in range(FORMS)]
+TARGETS = [('libpyvibdmc_amd.so', UNITS)]
 
 
 def hipcc():
@@ -58,14 +61,14 @@ def _run(cmd, what, verbose):
 def build(verbose=True, only=None):
     outs = []
     os.makedirs(OBJ, exist_ok=True)
-    for lib, srcs in TARGETS:
+    for lib, units in TARGETS:
         if only and lib not in only:
             continue
-        src_paths = [os.path.join(CSRC, s) for s in srcs]
-        if not all(os.path.exists(p) for p in src_paths):
+        if not all(os.path.exists(os.path.join(CSRC, src)) for _, src, _ in units):
             continue
-        objs = [os.path.join(OBJ, os.path.splitext(s)[0] + '.o') for s in srcs]
-        jobs = [([hipcc()] + FLAGS + EXTRA.get(os.path.basename(sp), []) + ['-c', sp, '-o', o], os.path.basename(sp)) for sp, o in zip(src_paths, objs)]
+        objs = [os.path.join(OBJ, o) for o, _, _ in units]
+        jobs = [([hipcc()] + FLAGS + extra + ['-c', os.path.join(CSRC, src), '-o', o], os.path.basename(o))
+                for o, (_, src, extra) in zip(objs, units)]
         workers = max(1, min(len(jobs), int(os.environ.get('MAX_JOBS', '0')) or (os.cpu_count() or 1)))
         with ThreadPoolExecutor(max_workers=workers) as ex:
             for f in [ex.submit(_run, c, w, verbose) for c, w in jobs]:
@@ -94,7 +97,7 @@ def asan_runtime():
 
 def build_asan(verbose=True):
     """Build ASAN_LIB (after build(), whose other objects it links); returns its path."""
-    others = [os.path.join(OBJ, s) for s in ('pvd_step_f32.o', 'pvd_step_f64.o', 'pvd_resident.o', 'pvd_mlp.o')]
+    others = [os.path.join(OBJ, o) for o, _, _ in UNITS if o != 'pvd_capi.o']
     if not all(os.path.exists(o) for o in others):
         build(verbose)
     obj = os.path.join(OBJ, 'pvd_capi_asan.o')

@@ -684,7 +684,7 @@ int pvd_sim_counts(pvd_sim* s, int64_t* counts, void* stream) {
     HIPCHK(hipMemcpyAsync(w, s->xch + RES_XSYNC, sizeof(w), hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
   }
-  counts[0] = w[RES_N_OPEN];
+  counts[0] = (int64_t)s->res_alone + w[RES_N_OPEN];
   counts[1] = w[RES_N_CLOSED];
   counts[2] = w[RES_N_SPREAD];
   return 0;

@@ -8,46 +8,26 @@ namespace {
 // Largest dynamic LDS a workgroup of k_resident may ask for: 160 KB less its static arrays.
 constexpr int RES_LDS = 160 * 1024 - 5 * 1024;
 
-struct Instance {
-  const void* fn;
-  const void* rest;
-  int W, ntmax, stride;
-};
-
-// FP32 and FP64 plain steps for the fused component counts, and FP32 importance sampling with the
-// compiled trials.  Two shapes each: `small`, at most two rounds of 512 threads per workgroup (the
-// step is latency then: fewer rounds to rank, 256 registers a wave), and W rounds of up to 1024
-// threads, which hold the population's whole range, 1.5 N0, wherever the LDS holds N0.  ntmax 512
-// where a walker needs more than the 128 registers a wave of 1024 threads has.
-template <typename R, int NP, bool IS, int MS, int W, int NTM>
-Instance shapes(bool small) {
-  const void* rest = (const void*)k_resident_rest<R, NP, IS, MS, NTM>;
-  if (small) return Instance{(const void*)k_resident<R, NP, IS, MS, 2, 512, false>, rest, 2, 512, res_stride<R, NP>()};
-  return Instance{(const void*)k_resident<R, NP, IS, MS, W, NTM, true>, rest, W, NTM, res_stride<R, NP>()};
-}
-
 template <typename R>
 Instance instance(const pvd_sim* s, bool small) {
   const int ms = s->mspec;
   if constexpr (sizeof(R) == 4) {
     if (s->is) {
-      if (s->np == 9 && ms == (MS_PES_WATER | MS_TRIAL_WATER))
-        return shapes<R, 9, true, MS_PES_WATER | MS_TRIAL_WATER, 6, 1024>(small);
-      if (s->np == 9 && ms == MS_TRIAL_WATER) return shapes<R, 9, true, MS_TRIAL_WATER, 6, 1024>(small);
-      if (s->np == 18 && ms == (MS_PES_CLUSTER | MS_TRIAL_CLUSTER))
-        return shapes<R, 18, true, MS_PES_CLUSTER | MS_TRIAL_CLUSTER, 6, 512>(small);
+      if (s->np == 9 && ms == (MS_PES_WATER | MS_TRIAL_WATER)) return res_instance<RF_WATER_IS>(small);
+      if (s->np == 9 && ms == MS_TRIAL_WATER) return res_instance<RF_TRIATOMIC_IS>(small);
+      if (s->np == 18 && ms == (MS_PES_CLUSTER | MS_TRIAL_CLUSTER)) return res_instance<RF_CLUSTER_IS>(small);
     } else {
-      if (s->np == 1) return shapes<R, 1, false, MS_ANY, 6, 1024>(small);
-      if (s->np == 3) return shapes<R, 3, false, MS_ANY, 6, 1024>(small);
-      if (s->np == 9 && (ms & MS_PES_WATER)) return shapes<R, 9, false, MS_PES_WATER, 6, 1024>(small);
-      if (s->np == 9) return shapes<R, 9, false, MS_ANY, 6, 1024>(small);
-      if (s->np == 18 && (ms & MS_PES_CLUSTER)) return shapes<R, 18, false, MS_PES_CLUSTER, 3, 1024>(small);
+      if (s->np == 1) return res_instance<RF_1>(small);
+      if (s->np == 3) return res_instance<RF_3>(small);
+      if (s->np == 9 && (ms & MS_PES_WATER)) return res_instance<RF_WATER>(small);
+      if (s->np == 9) return res_instance<RF_TRIATOMIC>(small);
+      if (s->np == 18 && (ms & MS_PES_CLUSTER)) return res_instance<RF_CLUSTER>(small);
     }
   } else if (!s->is) {
-    if (s->np == 1) return shapes<R, 1, false, MS_ANY, 6, 1024>(small);
-    if (s->np == 3) return shapes<R, 3, false, MS_ANY, 6, 1024>(small);
-    if (s->np == 9 && (ms & MS_PES_WATER)) return shapes<R, 9, false, MS_PES_WATER, 6, 512>(small);
-    if (s->np == 9) return shapes<R, 9, false, MS_ANY, 6, 512>(small);
+    if (s->np == 1) return res_instance<RF_1_F64>(small);
+    if (s->np == 3) return res_instance<RF_3_F64>(small);
+    if (s->np == 9 && (ms & MS_PES_WATER)) return res_instance<RF_WATER_F64>(small);
+    if (s->np == 9) return res_instance<RF_TRIATOMIC_F64>(small);
   }
   return Instance{nullptr, nullptr, 0, 0, 0};
 }
@@ -110,13 +90,20 @@ Plan make_plan(pvd_sim* s, bool who) {
 // launch does (the second launch, walkers in and out).  us a step in calls of 16 steps, here and
 // launch per step: water 1 000 walkers 4.3, 9.0; 100 000 4.8, 10.7;
 // 1 000 000 15.3, 21.0; with importance sampling 31.4, 50.5; cluster with it, 500 000 36.0, 56.9.
+// The first RES_REPAY steps of a simulation that asks for them a few at a time stay with the step
+// kernels: the first launch of a form in a process takes 0.41 ms more (its code, see RF_1), which 5 us
+// a step repay after about 80 (the first 20 steps of a million walkers: 0.46 ms, 0.75 without this rule).
 constexpr int RES_STEPS = 4096;
 constexpr int RES_MIN = 16;
+constexpr int RES_REPAY = 96;
 
 template <typename R>
 int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
   done = 0;
-  if (s->cont || !s->xch || s->htrial || s->cfg.pes.kind == PES_EXTERNAL || n_steps < RES_MIN) return 0;
+  s->steps_asked += n_steps;
+  if (s->cont || !s->xch || s->htrial || s->cfg.pes.kind == PES_EXTERNAL || n_steps < RES_MIN ||
+      s->steps_asked < RES_REPAY)
+    return 0;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
@@ -176,7 +163,9 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
     void* args[] = {&A};
     A.set = (int)(s->res_launches & 1);
     HIPCHK(hipLaunchKernel(P.fn, dim3(P.grid), dim3(P.nt), args, P.lds, st));
-    if (P.grid > 1) {
+    if (P.grid == 1) {
+      ++s->res_alone;
+    } else {
       ++s->res_launches;
       HIPCHK(hipLaunchKernel(P.rest, dim3(P.grid), dim3(P.nt), args, 0, st));
     }

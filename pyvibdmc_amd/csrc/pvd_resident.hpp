@@ -1113,4 +1113,44 @@ __global__ __launch_bounds__(NTMAX) void k_resident_rest(ResArgs<R> A) {
   }
 }
 
+// The forms: FP32 and FP64 plain steps for the fused component counts, and FP32 importance sampling
+// with the compiled trials.  A form is an object of its own (pvd_resident_form.hip): the first launch
+// out of an object waits until all of its code is on the device, 0.35 ms and 1 ms more a megabyte
+// (all forms together: 1.8 ms).
+enum : int { RF_1, RF_3, RF_WATER, RF_TRIATOMIC, RF_CLUSTER, RF_WATER_IS, RF_TRIATOMIC_IS, RF_CLUSTER_IS, RF_1_F64,
+             RF_3_F64, RF_WATER_F64, RF_TRIATOMIC_F64, RF_COUNT };
+
+// W rounds of at most NTM threads in the shape for large populations
+template <int F>
+struct ResForm;
+#define PVD_RES_FORM(F, R_, NP_, IS_, MS_, W_, NTM_)                \
+  template <>                                                       \
+  struct ResForm<F> {                                               \
+    using R = R_;                                                   \
+    static constexpr int NP = NP_, MS = MS_, W = W_, NTM = NTM_;    \
+    static constexpr bool IS = IS_;                                 \
+  };
+PVD_RES_FORM(RF_1, float, 1, false, MS_ANY, 6, 1024)
+PVD_RES_FORM(RF_3, float, 3, false, MS_ANY, 6, 1024)
+PVD_RES_FORM(RF_WATER, float, 9, false, MS_PES_WATER, 6, 1024)
+PVD_RES_FORM(RF_TRIATOMIC, float, 9, false, MS_ANY, 6, 1024)
+PVD_RES_FORM(RF_CLUSTER, float, 18, false, MS_PES_CLUSTER, 3, 1024)
+PVD_RES_FORM(RF_WATER_IS, float, 9, true, (MS_PES_WATER | MS_TRIAL_WATER), 6, 1024)
+PVD_RES_FORM(RF_TRIATOMIC_IS, float, 9, true, MS_TRIAL_WATER, 6, 1024)
+PVD_RES_FORM(RF_CLUSTER_IS, float, 18, true, (MS_PES_CLUSTER | MS_TRIAL_CLUSTER), 6, 512)
+PVD_RES_FORM(RF_1_F64, double, 1, false, MS_ANY, 6, 1024)
+PVD_RES_FORM(RF_3_F64, double, 3, false, MS_ANY, 6, 1024)
+PVD_RES_FORM(RF_WATER_F64, double, 9, false, MS_PES_WATER, 6, 512)
+PVD_RES_FORM(RF_TRIATOMIC_F64, double, 9, false, MS_ANY, 6, 512)
+#undef PVD_RES_FORM
+
+// a form's kernels in one of its two shapes
+struct Instance {
+  const void* fn;
+  const void* rest;
+  int W, ntmax, stride;
+};
+template <int F>
+Instance res_instance(bool small);
+
 }  // namespace pvd

@@ -60,7 +60,8 @@ struct pvd_sim {
   uint64_t* drec;
   unsigned* accs;
   uint64_t* xch;  // exchange words of the resident steps (discrete weighting)
-  unsigned res_launches;  // resident launches of more than one workgroup so far
+  unsigned res_launches, res_alone;  // resident launches so far, of several workgroups and of one
+  long long steps_asked;  // steps with the library's own draws so far
   unsigned long long res_gate_wait, res_team_wait;  // see RES_WAIT
   double* tr_vref;
   double* tr_pop;
