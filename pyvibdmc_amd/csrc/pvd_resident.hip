@@ -85,15 +85,20 @@ Plan make_plan(pvd_sim* s, bool who) {
 
 }  // namespace
 
-// Steps of one launch at most (a bound on how long one kernel runs: about 60 ms at a million
-// walkers), and the fewest for which it is used: a call costs about 20 us more than a step kernel's
+// Steps of one launch at most, a bound on how long other streams' kernels that need LDS wait: a launch
+// that fills the LDS (all but the small shape do) holds the CUs for 128 steps, 2 ms for a million
+// triatomics, 4 to 5 ms with importance sampling, on the Partridge-Schwenke surface and for 500 000
+// clusters; 4096 steps were 60 to 180 ms (a library product on another stream beside a million
+// walkers: 58 ms, now 1).  It costs nothing: even shares again make up for the launch (us a step in
+// calls of 4096 and 128 steps: a million walkers 15.9, 15.6; with importance sampling 30.9, 30.9).
+// RES_MIN: the fewest steps for which it is used.  A call costs about 20 us more than a step kernel's
 // launch does (the second launch, walkers in and out).  us a step in calls of 16 steps, here and
 // launch per step: water 1 000 walkers 4.3, 9.0; 100 000 4.8, 10.7;
 // 1 000 000 15.3, 21.0; with importance sampling 31.4, 50.5; cluster with it, 500 000 36.0, 56.9.
 // The first RES_REPAY steps of a simulation that asks for them a few at a time stay with the step
 // kernels: the first launch of a form in a process takes 0.41 ms more (its code, see RF_1), which 5 us
 // a step repay after about 80 (the first 20 steps of a million walkers: 0.46 ms, 0.75 without this rule).
-constexpr int RES_STEPS = 4096;
+constexpr int RES_STEPS = 4096, RES_STEPS_FULL = 128;
 constexpr int RES_MIN = 16;
 constexpr int RES_REPAY = 96;
 
@@ -158,7 +163,7 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
     A.h2s[p] = S.h2s[p];
   }
   while (done < n_steps) {
-    A.steps = std::min(RES_STEPS, n_steps - done);
+    A.steps = std::min(P.lds > RES_LDS / 2 ? RES_STEPS_FULL : RES_STEPS, n_steps - done);
     A.par = (int)(s->next_step & 1);
     void* args[] = {&A};
     A.set = (int)(s->res_launches & 1);

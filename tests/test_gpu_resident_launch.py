@@ -75,3 +75,31 @@ def test_small_simulations_on_two_streams_overlap():
     assert both < 0.8 * turn
     for s in sims:
         assert s._status()[0] == 0
+
+
+def test_other_streams_get_their_turn():
+    """A million walkers fill the LDS of every CU; a kernel of another stream that needs LDS waits for
+    one launch (2 ms), not for all of the 4 000 steps (62 ms).  Of several streams, as one may share a
+    hardware queue with the simulation's."""
+    import torch
+    from pyvibdmc_amd import _native as N
+    sim = make('water', 1_000_000, 10 ** 5, 'fp32')
+    sim._start()
+    a, m = torch.cuda.Stream(), torch.randn(1024, 1024, device='cuda')
+    waits = []
+    for _ in range(3):
+        b = torch.cuda.Stream()
+        for timed in (False, True):
+            torch.cuda.synchronize()
+            if timed:
+                N.check(N.load().pvd_sim_run(sim._h, 4000, a.cuda_stream))
+                time.sleep(5e-3)
+            t = time.perf_counter()
+            with torch.cuda.stream(b):
+                m @ m
+                b.synchronize()
+        waits.append((time.perf_counter() - t) * 1e3)
+    torch.cuda.synchronize()
+    print('ms', waits)
+    assert sim._status()[0] == 0
+    assert min(waits) < 25
