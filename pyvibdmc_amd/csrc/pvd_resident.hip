@@ -64,7 +64,9 @@ Plan make_plan(pvd_sim* s, bool who) {
   if ((long long)g * (capb - capl) * (I.stride + 1) * (long long)sizeof(R) > (long long)sizeof(double) * s->np * s->cap)
     return P;
   P.lds = (size_t)unit * capl;
-  if (hipFuncSetAttribute(I.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.lds) != hipSuccess) {
+  // the same limit from every caller: it belongs to the kernel, and another thread may be between its
+  // own plan, of another size, and its launch
+  if (hipFuncSetAttribute(I.fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS) != hipSuccess) {
     (void)hipGetLastError();
     return P;
   }

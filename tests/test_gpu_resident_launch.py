@@ -103,3 +103,35 @@ def test_other_streams_get_their_turn():
     print('ms', waits)
     assert sim._status()[0] == 0
     assert min(waits) < 25
+
+
+def test_threads_with_plans_of_different_sizes():
+    """Two threads on one kernel whose plans ask for different amounts of LDS (with and without the
+    descendant tracker): every call is served, and the results are those of the runs alone."""
+    import numpy as np
+    import torch
+    from pyvibdmc_amd import _native as N
+    lib = N.load()
+
+    def run(window, stream):
+        with torch.cuda.stream(stream):
+            sim, st = make('water', 300_000, 10 ** 4, 'fp32', seed=7), N.stream_handle()
+            sim._start()
+            if window:
+                N.check(lib.pvd_sim_desc_begin(sim._h, st))
+            for _ in range(60):
+                N.check(lib.pvd_sim_run(sim._h, 24, st))
+            assert sim._status()[0] == 0
+            return sim._get_walkers()[0]
+
+    alone = run(False, torch.cuda.Stream())
+    got, streams = [None, None], [torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def work(i):
+        got[i] = run(bool(i), streams[i])
+
+    th = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    for g in got:  # the tracker does not change the walkers
+        np.testing.assert_array_equal(g, alone)
