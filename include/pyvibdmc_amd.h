@@ -191,7 +191,10 @@ int pvd_sim_trajectory(pvd_sim* sim, int64_t t0, int32_t count, double* vref, do
  * launch up, which leaves all steps to the second.  No counterpart in the reference. */
 int pvd_sim_resident_waits(pvd_sim* sim, int64_t gate_us, int64_t team_us);
 /* How the steps so far were run: counts[0] launches with the walkers kept on chip, counts[1]
- * launches given up for the second form, counts[2] redistributions of the walkers over the workgroups.  Synchronous.  No counterpart in the reference. */
+ * launches given up for the second form, counts[2] redistributions of the walkers over the
+ * workgroups; since the walkers were set, split replays beyond the LDS form (codes 7 and 8 of
+ * pvd_sim_trajectory) counts[3] that ordered their candidates in LDS, counts[4] that moved them.
+ * Synchronous.  No counterpart in the reference. */
 int pvd_sim_counts(pvd_sim* sim, int64_t* counts, void* stream);
 
 /* Descendant weighting window (pyvibdmc.py:739-747, 663-672, 856-872).  end() writes

@@ -680,6 +680,9 @@ int pvd_sim_resident_waits(pvd_sim* s, int64_t gate_us, int64_t team_us) {
 int pvd_sim_counts(pvd_sim* s, int64_t* counts, void* stream) {
   if (!s || !counts) return fail(E_BAD, "null argument");
   unsigned w[RES_SYNCW] = {};
+  Ctrl c;
+  const int rc = read_ctrl(s, c, (hipStream_t)stream);
+  if (rc) return rc;
   if (s->xch) {
     HIPCHK(hipMemcpyAsync(w, s->xch + RES_XSYNC, sizeof(w), hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
@@ -687,6 +690,8 @@ int pvd_sim_counts(pvd_sim* s, int64_t* counts, void* stream) {
   counts[0] = (int64_t)s->res_alone + w[RES_N_OPEN];
   counts[1] = w[RES_N_CLOSED];
   counts[2] = w[RES_N_SPREAD];
+  counts[3] = c.sorts[0];
+  counts[4] = c.sorts[1];
   return 0;
 }
 

@@ -72,6 +72,7 @@ struct Ctrl {
   int gc_start;
   int pad2;
   double gc_w;
+  unsigned sorts[2];  // steps that it ordered in LDS, and moving the candidates
 };
 
 struct TileRec {
@@ -1894,6 +1895,204 @@ PVD_DEV bool order_candidates(int C, const unsigned long long* key, unsigned lon
   return true;
 }
 
+// The same for more candidates, or crowded buckets: keys and slots are moved in the global scratch.
+// A counting sort on 14 bits of the key above its minimum (an order-preserving map of the keys' own
+// range onto the buckets: the candidates of a steady state lie in a band about a tenth of an octave
+// wide, which the top mantissa bits would crowd into a tenth of the buckets), then each entry is
+// ranked inside its bucket.  Then the octaves from the top, until the K kills are used: Es is the
+// octave where they run out, if `found`.
+// False where a bucket is too full.
+PVD_DEV bool move_candidates(int C, int K, const RsgView& rv, unsigned long long kmin, unsigned long long kmax, int etop,
+                             int eT, unsigned long long mT, int* asg, int* bcnt, int* s_i, int* s_sh, int& tie_e,
+                             int& Es, bool& found) {
+  constexpr int NT = RP_NT, U = RG_U;
+  constexpr unsigned long long MANT = (1ull << 52) - 1;
+  const int tid = threadIdx.x;
+  unsigned long long* key = rv.key;
+  unsigned long long* bkey = rv.bkey;
+  int* ord = rv.ord;
+  int* bord = rv.bord;
+  auto kexp = [](unsigned long long k) { return key_exp(k); };
+  auto kmant = [](unsigned long long k) { return MANT - (k >> 11); };
+  int base = 0;
+  constexpr int BPT = RCG_BUCKETS / NT;
+  const unsigned long long kspan = kmax - kmin;
+  const int bsh = (kspan >> 14) == 0ull ? 0 : 64 - __clzll((long long)kspan) - 14;
+  auto bucket = [&](unsigned long long k) { return (int)((k - kmin) >> bsh); };  // < RCG_BUCKETS
+  for (int b = tid; b < RCG_BUCKETS; b += NT) bcnt[b] = 0;
+  __syncthreads();
+  for (int q0 = 0; q0 < C; q0 += U * NT) {
+    unsigned long long kk[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * NT + tid;
+      kk[u] = q < C ? key[q] : 0ull;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (q0 + u * NT + tid < C) atomicAdd(&bcnt[bucket(kk[u])], 1);
+  }
+  __syncthreads();
+  int bmax;
+  {
+    int loc = 0, mx = 0;
+    for (int u = 0; u < BPT; ++u) {
+      const int c = bcnt[tid * BPT + u];
+      loc += c;
+      mx = max(mx, c);
+    }
+    int tot;
+    const int ex = block_excl_scan<NT>(loc, s_i, tot);
+    int st = ex;
+    for (int u = 0; u < BPT; ++u) {
+      const int c = bcnt[tid * BPT + u];
+      bcnt[tid * BPT + u] = st;  // bucket starts (each thread rewrites only its own buckets)
+      st += c;
+    }
+    bmax = block_max<NT>(mx, s_i);
+  }
+  if (bmax > RCG_BMAX) return false;  // the in-bucket rank costs bucket size squared
+  for (int q0 = 0; q0 < C; q0 += U * NT) {
+    unsigned long long kk[U];
+    int oo[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * NT + tid;
+      kk[u] = q < C ? key[q] : 0ull;
+      oo[u] = q < C ? ord[q] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (q0 + u * NT + tid < C) {
+        const int d = atomicAdd(&bcnt[bucket(kk[u])], 1);  // bcnt ends as the bucket ends
+        bkey[d] = kk[u];
+        bord[d] = oo[u];
+      }
+  }
+  __syncthreads();
+  // ranks: U entries per thread at a time, the first RK keys of each one's bucket in flight
+  constexpr int RK = 4;
+  for (int q0 = 0; q0 < C; q0 += U * NT) {
+    unsigned long long kq[U];
+    int oq[U], bs[U], be[U], rank[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * NT + tid;
+      kq[u] = q < C ? bkey[q] : 0ull;
+      oq[u] = q < C ? bord[q] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * NT + tid;
+      const int bk = q < C ? bucket(kq[u]) : 0;
+      bs[u] = q < C ? (bk > 0 ? bcnt[bk - 1] : 0) : 0;
+      be[u] = q < C ? bcnt[bk] : 0;
+      rank[u] = 0;
+    }
+#pragma unroll
+    for (int i = 0; i < RK; ++i)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int x = bs[u] + i, q = q0 + u * NT + tid;
+        if (x < be[u]) {
+          const unsigned long long ki = bkey[x];
+          rank[u] += (ki < kq[u] || (ki == kq[u] && x < q)) ? 1 : 0;
+        }
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * NT + tid;
+      for (int x0 = bs[u] + RK; x0 < be[u]; x0 += 8) {  // larger buckets: eight loads in flight
+        unsigned long long k8[8];
+#pragma unroll
+        for (int v = 0; v < 8; ++v) k8[v] = x0 + v < be[u] ? bkey[x0 + v] : ~0ull;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+          const int x = x0 + v;
+          rank[u] += (x < be[u] && (k8[v] < kq[u] || (k8[v] == kq[u] && x < q))) ? 1 : 0;
+        }
+      }
+      if (q < C) {
+        key[bs[u] + rank[u]] = kq[u];
+        ord[bs[u] + rank[u]] = oq[u];
+      }
+    }
+  }
+  __syncthreads();
+  // the highest octave in which two equal mantissas meet
+  for (int j0 = 0; j0 < C; j0 += U * NT) {
+    unsigned long long kk[U], kn[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = j0 + u * NT + tid;
+      kk[u] = j < C ? key[j] : 0ull;
+      kn[u] = j + 1 < C ? key[j + 1] : 0ull;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = j0 + u * NT + tid;
+      if (j < C) {
+        if (j + 1 < C && (kn[u] >> 11) == (kk[u] >> 11)) tie_e = max(tie_e, min(kexp(kk[u]), kexp(kn[u])));
+      }
+    }
+  }
+  tie_e = block_max<NT>(tie_e, s_i);
+  // octaves from the top: each family's run of kill indices, until K are used; in the
+  //    octave of T only the entries of value >= T count.  Thread tid holds the candidates
+  //    [j0, j1) in sorted order: its entry count, one block scan, then its families' runs.
+  auto fam = [&](unsigned long long kj, int E) -> int {
+    const int ej = kexp(kj);
+    if (!(ej >= E && (E > eT || kmant(kj) >= mT))) return 0;
+    const int d = ej - E;
+    return d >= 20 ? KILL_CAP + 1 : min(1 << d, KILL_CAP + 1);
+  };
+  const int P = (C + NT - 1) / NT;
+  const int j0 = min(C, tid * P), j1 = min(C, j0 + P);
+  for (int E = etop; E >= eT; --E) {
+    int loc = 0;
+    for (int jb = j0; jb < j1; jb += U) {
+      unsigned long long kk[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (jb + u < j1) loc = min(loc + fam(kk[u], E), KILL_CAP + 1);
+    }
+    // a thread's count is clamped above K: the block sums stay in int, and every later
+    // thread still starts at or beyond K
+    int tot;
+    const int ex = block_excl_scan<NT>(loc, s_i, tot);
+    int st = base + ex;
+    for (int jb = j0; jb < j1 && st < K; jb += U) {
+      unsigned long long kk[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = jb + u;
+        const int v = j < j1 ? fam(kk[u], E) : 0;
+        if (v > 0 && st < K) {
+          const int hi = min(st + v, K);
+          for (int t = st; t < hi; ++t) asg[t] = j;
+          if (st + v >= K) {
+            s_sh[0] = j;
+            s_sh[1] = st;
+          }
+        }
+        st += v;
+      }
+    }
+    base += tot;
+    __syncthreads();
+    if (base >= K) {
+      Es = E;
+      found = true;
+      break;
+    }
+  }
+  return true;
+}
+
 template <typename R>
 PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const int* subn, double T0, int* bcnt,
                                 int* s_i, int* s_sh, int* hist, double& cut, bool& refined) {
@@ -1928,12 +2127,8 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
   // key = (inverted mantissa << 11) | inverted exponent; ord holds the walker slot
   const RsgView rv = rsg_view(A.rsg);
   unsigned long long* key = rv.key;
-  unsigned long long* bkey = rv.bkey;
   int* ord = rv.ord;
-  int* bord = rv.bord;
   int* start = rv.start;
-  auto kexp = [](unsigned long long k) { return key_exp(k); };
-  auto kmant = [](unsigned long long k) { return MANT - (k >> 11); };
   // 1. the cut: T0, or, when the lists hold over a quarter more than about 1.25 K walkers
   //    (at a steady state list A holds the last step's 2 K split pieces) and more than the LDS
   //    order takes, the lowest histogram edge with at most 1.25 K entries at or above it: every
@@ -2027,7 +2222,7 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
   etop = block_max<NT>(etop, s_i);
   if (etop - eT > 40) return RC_OTHER;
   int tie_e = -0x40000000, base = 0, Es = 0, p = 0, startp = 0;
-  bool found = false;
+  bool found = false, moved = false;
   // 2. candidates by decreasing mantissa (then exponent), their order in LDS where it fits
   unsigned* word = reinterpret_cast<unsigned*>(bcnt) + RO_PAD;
   if (C <= RO_CAP && order_candidates(C, key, kmin, kmax, eT, reinterpret_cast<unsigned*>(hist), word, s_i, tie_e)) {
@@ -2074,188 +2269,8 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
         found = true;
       }
     }
-  } else {
-    // the order does not fit: keys and slots are moved.  Counting sort on 14 bits of the key
-    //    above its minimum (an order-preserving map of the keys' own range onto the buckets: the
-    //    candidates of a steady state lie in a band about a tenth of an octave wide, which the
-    //    top mantissa bits would crowd into a tenth of the buckets), then each entry ranked
-    //    inside its bucket
-    constexpr int BPT = RCG_BUCKETS / NT;
-    const unsigned long long kspan = kmax - kmin;
-    const int bsh = (kspan >> 14) == 0ull ? 0 : 64 - __clzll((long long)kspan) - 14;
-    auto bucket = [&](unsigned long long k) { return (int)((k - kmin) >> bsh); };  // < RCG_BUCKETS
-    for (int b = tid; b < RCG_BUCKETS; b += NT) bcnt[b] = 0;
-    __syncthreads();
-    for (int q0 = 0; q0 < C; q0 += U * NT) {
-      unsigned long long kk[U];
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + u * NT + tid;
-        kk[u] = q < C ? key[q] : 0ull;
-      }
-  #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (q0 + u * NT + tid < C) atomicAdd(&bcnt[bucket(kk[u])], 1);
-    }
-    __syncthreads();
-    int bmax;
-    {
-      int loc = 0, mx = 0;
-      for (int u = 0; u < BPT; ++u) {
-        const int c = bcnt[tid * BPT + u];
-        loc += c;
-        mx = max(mx, c);
-      }
-      int tot;
-      const int ex = block_excl_scan<NT>(loc, s_i, tot);
-      int st = ex;
-      for (int u = 0; u < BPT; ++u) {
-        const int c = bcnt[tid * BPT + u];
-        bcnt[tid * BPT + u] = st;  // bucket starts (each thread rewrites only its own buckets)
-        st += c;
-      }
-      bmax = block_max<NT>(mx, s_i);
-    }
-    if (bmax > RCG_BMAX) return RC_OTHER;  // the in-bucket rank costs bucket size squared
-    for (int q0 = 0; q0 < C; q0 += U * NT) {
-      unsigned long long kk[U];
-      int oo[U];
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + u * NT + tid;
-        kk[u] = q < C ? key[q] : 0ull;
-        oo[u] = q < C ? ord[q] : 0;
-      }
-  #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (q0 + u * NT + tid < C) {
-          const int d = atomicAdd(&bcnt[bucket(kk[u])], 1);  // bcnt ends as the bucket ends
-          bkey[d] = kk[u];
-          bord[d] = oo[u];
-        }
-    }
-    __syncthreads();
-    // ranks: U entries per thread at a time, the first RK keys of each one's bucket in flight
-    constexpr int RK = 4;
-    for (int q0 = 0; q0 < C; q0 += U * NT) {
-      unsigned long long kq[U];
-      int oq[U], bs[U], be[U], rank[U];
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + u * NT + tid;
-        kq[u] = q < C ? bkey[q] : 0ull;
-        oq[u] = q < C ? bord[q] : 0;
-      }
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + u * NT + tid;
-        const int bk = q < C ? bucket(kq[u]) : 0;
-        bs[u] = q < C ? (bk > 0 ? bcnt[bk - 1] : 0) : 0;
-        be[u] = q < C ? bcnt[bk] : 0;
-        rank[u] = 0;
-      }
-  #pragma unroll
-      for (int i = 0; i < RK; ++i)
-  #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int x = bs[u] + i, q = q0 + u * NT + tid;
-          if (x < be[u]) {
-            const unsigned long long ki = bkey[x];
-            rank[u] += (ki < kq[u] || (ki == kq[u] && x < q)) ? 1 : 0;
-          }
-        }
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + u * NT + tid;
-        for (int x0 = bs[u] + RK; x0 < be[u]; x0 += 8) {  // larger buckets: eight loads in flight
-          unsigned long long k8[8];
-  #pragma unroll
-          for (int v = 0; v < 8; ++v) k8[v] = x0 + v < be[u] ? bkey[x0 + v] : ~0ull;
-  #pragma unroll
-          for (int v = 0; v < 8; ++v) {
-            const int x = x0 + v;
-            rank[u] += (x < be[u] && (k8[v] < kq[u] || (k8[v] == kq[u] && x < q))) ? 1 : 0;
-          }
-        }
-        if (q < C) {
-          key[bs[u] + rank[u]] = kq[u];
-          ord[bs[u] + rank[u]] = oq[u];
-        }
-      }
-    }
-    __syncthreads();
-    // 3. the highest octave in which two equal mantissas meet
-    tie_e = -0x40000000;
-    for (int j0 = 0; j0 < C; j0 += U * NT) {
-      unsigned long long kk[U], kn[U];
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int j = j0 + u * NT + tid;
-        kk[u] = j < C ? key[j] : 0ull;
-        kn[u] = j + 1 < C ? key[j + 1] : 0ull;
-      }
-  #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int j = j0 + u * NT + tid;
-        if (j < C) {
-          if (j + 1 < C && (kn[u] >> 11) == (kk[u] >> 11)) tie_e = max(tie_e, min(kexp(kk[u]), kexp(kn[u])));
-        }
-      }
-    }
-    tie_e = block_max<NT>(tie_e, s_i);
-    // 4. octaves from the top: each family's run of kill indices, until K are used; in the
-    //    octave of T only the entries of value >= T count.  Thread tid holds the candidates
-    //    [j0, j1) in sorted order: its entry count, one block scan, then its families' runs.
-    auto fam = [&](unsigned long long kj, int E) -> int {
-      const int ej = kexp(kj);
-      if (!(ej >= E && (E > eT || kmant(kj) >= mT))) return 0;
-      const int d = ej - E;
-      return d >= 20 ? KILL_CAP + 1 : min(1 << d, KILL_CAP + 1);
-    };
-    const int P = (C + NT - 1) / NT;
-    const int j0 = min(C, tid * P), j1 = min(C, j0 + P);
-    for (int E = etop; E >= eT; --E) {
-      int loc = 0;
-      for (int jb = j0; jb < j1; jb += U) {
-        unsigned long long kk[U];
-  #pragma unroll
-        for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
-  #pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (jb + u < j1) loc = min(loc + fam(kk[u], E), KILL_CAP + 1);
-      }
-      // a thread's count is clamped above K: the block sums stay in int, and every later
-      // thread still starts at or beyond K
-      int tot;
-      const int ex = block_excl_scan<NT>(loc, s_i, tot);
-      int st = base + ex;
-      for (int jb = j0; jb < j1 && st < K; jb += U) {
-        unsigned long long kk[U];
-  #pragma unroll
-        for (int u = 0; u < U; ++u) kk[u] = jb + u < j1 ? key[jb + u] : 0ull;
-  #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int j = jb + u;
-          const int v = j < j1 ? fam(kk[u], E) : 0;
-          if (v > 0 && st < K) {
-            const int hi = min(st + v, K);
-            for (int t = st; t < hi; ++t) A.asg[t] = j;
-            if (st + v >= K) {
-              s_sh[0] = j;
-              s_sh[1] = st;
-            }
-          }
-          st += v;
-        }
-      }
-      base += tot;
-      __syncthreads();
-      if (base >= K) {
-        Es = E;
-        found = true;
-        break;
-      }
-    }
+  } else if (!(moved = move_candidates(C, K, rv, kmin, kmax, etop, eT, mT, A.asg, bcnt, s_i, s_sh, tie_e, Es, found))) {
+    return RC_OTHER;
   }
   if (!found) return RC_FEW;
   if (tie_e >= Es) return RC_OTHER;
@@ -2301,6 +2316,7 @@ PVD_DEV int replay_candidates_g(const StepArgs<R>& A, int K, int nlists, const i
   if (tid == 0) {
     Ctrl* Cw = A.ctrl;
     Cw->gc_n = C;
+    Cw->sorts[moved ? 1 : 0] += 1u;
     Cw->gc_p = p;
     Cw->gc_slot = cps;
     Cw->gc_dp = Dp;
