@@ -31,6 +31,7 @@ sys.path.insert(0, ROOT)
 import numpy as np  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
+VALU_PEAK_GINST = 256 * 2.4  # one wave64 VALU instruction per CU and cycle, 256 CUs at 2.4 GHz
 MFMA_BF16_PEAK_TFLOPS = 2500.0  # dense
 # algorithmic FLOP of one network evaluation: 2 (D H + H H + H H + H), D = 3, H = 128
 MLP_FLOP_PER_WALKER = 2 * (3 * 128 + 128 * 128 + 128 * 128 + 128)
@@ -163,7 +164,9 @@ def train_surrogate(n, epochs, geoms, seed=11):
 
 def run_timed(sim, warmup, steps, events_steps=0):
     """Warm up, then time exactly `steps` fused steps between two device syncs.  Optionally
-    time `events_steps` more launches individually with HIP events on the launch stream."""
+    time `events_steps` more steps launched one at a time, with HIP events on every kernel.  The
+    last value returned: whether the timed steps ran with the walkers kept on chip (k_resident, many
+    steps a launch) and not as single launches."""
     import torch
     from pyvibdmc_amd import _native as N
     lib = N.load()
@@ -171,12 +174,14 @@ def run_timed(sim, warmup, steps, events_steps=0):
     sim._start()
     N.check(lib.pvd_sim_run(sim._h, warmup, st))
     sim._raise_if_failed()
+    before = resident_launches(sim)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     N.check(lib.pvd_sim_run(sim._h, steps, st))
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     sim._raise_if_failed()
+    on_chip = resident_launches(sim) > before
     sim._fetch_traj(0, warmup + steps)
     pops = sim._pop_vs_tau
     # population entering step t = population after step t-1
@@ -196,7 +201,28 @@ def run_timed(sim, warmup, steps, events_steps=0):
         ev_n = float(np.mean(sim._pop_vs_tau[warmup + steps - 1:warmup + steps + events_steps - 1]))
     else:
         ev_n = None
-    return ws, wall, float(np.mean(entering)), kern_ms, ev_n
+    return ws, wall, float(np.mean(entering)), kern_ms, ev_n, on_chip
+
+
+def resident_launches(sim):
+    import ctypes
+    from pyvibdmc_amd import _native as N
+    c = (ctypes.c_int64 * 5)()
+    N.check(N.load().pvd_sim_counts(sim._h, c, N.stream_handle()))
+    return c[0] + c[1]
+
+
+def valu_roofline(form, kernel, rate):
+    """Vector issue of the on-chip steps: `rate` walker-steps/s times the wave instructions of one
+    (counted once by a profiler) against one wave64 instruction per CU and cycle (four SIMDs, four
+    cycles each)."""
+    per = load_traffic(f'k_resident_{form}_valu_per_walker_step')
+    if per is None:
+        return None
+    return {"bound": "valu", "achieved": rate * per / 1e9, "peak": VALU_PEAK_GINST, "unit": "G wave instructions/s",
+            "frac": rate * per / 1e9 / VALU_PEAK_GINST, "kernel": kernel, "valu_wave_inst_per_walker_step": per,
+            "source": "instructions: committed counter profile (profiles/k_resident_counters.md, SQ_INSTS_VALU); "
+                      "rate: the timed region itself"}
 
 
 def continuous_variant(n=100_000, T=10_000):
@@ -387,7 +413,7 @@ def ps_variant(n, steps, epochs, zpe_steps=2000):
     for name, mk in (('analytic', lambda: pv.PartridgeSchwenkeWater()),
                      ('surrogate', lambda: SurrogatePotential(m, pv.PartridgeSchwenkeWater(), judge_every=100))):
         sm = sim(n, 10 + steps + 2, mk(), 7)
-        ws, wall, _, _, _ = run_timed(sm, 10, steps, 0)
+        ws, wall, _, _, _, _ = run_timed(sm, 10, steps, 0)
         del sm
         pot = mk()
         sz = sim(n, zpe_steps, pot, 7)
@@ -405,7 +431,7 @@ def ps_variant(n, steps, epochs, zpe_steps=2000):
     sp = pv.DMC_Sim(num_walkers=n, num_timesteps=10 + steps + 2, atoms=['H', 'H', 'O'], delta_t=5,
                     potential=pv.PartridgeSchwenkeWater(), start_structures=start, precision='fp32', seed=7,
                     write_files=False, equil_steps=10 ** 9, wfn_every=10 ** 9, chkpt_every=10 ** 9)
-    ws, wall, _, _, _ = run_timed(sp, 10, steps, 0)
+    ws, wall, _, _, _, _ = run_timed(sp, 10, steps, 0)
     out['plain_analytic'] = {"value": ws / wall, "unit": "walker-steps/s", "ms_per_step": wall * 1e3 / steps}
     log(f'[bench] PS plain analytic: {ws / wall:.4g} walker-steps/s')
     del sp
@@ -465,7 +491,7 @@ def cluster_study(n, steps, epochs, zpe_steps):
                                                                  judge_stride=1000))):
         pot = mk()
         sim = cluster_sim(n, 10 + steps + 2, 'fp32', pot, 7)
-        ws, wall, mean_n, _, _ = run_timed(sim, 10, steps, 0)
+        ws, wall, mean_n, _, _, _ = run_timed(sim, 10, steps, 0)
         row = {"value": ws / wall, "unit": "walker-steps/s", "ms_per_step": wall * 1e3 / steps}
         if name == 'is_surrogate':
             from pyvibdmc_amd import _native as N
@@ -607,20 +633,21 @@ def main():
 
     if args.is_only:
         sim = make_sim(n, total, precision=args.precision, imp=True)
-        ws2, wall2, _, kern2, _ = run_timed(sim, W, K, min(args.event_steps, 50))
-        print(json.dumps({"is": {"value": ws2 / wall2, "ms_per_step": wall2 * 1e3 / K,
-                                 "step_kernels_us": {nm: t * 1e3 for nm, t in zip(['k_is_move', 'k_discrete'],
+        ws2, wall2, _, kern2, _, on2 = run_timed(sim, W, K, min(args.event_steps, 50))
+        print(json.dumps({"is": {"value": ws2 / wall2, "ms_per_step": wall2 * 1e3 / K, "on_chip": on2,
+                                 "single_step_kernels_us": {nm: t * 1e3 for nm, t in zip(['k_is_move', 'k_discrete'],
                                                                                   kern2 or [])}}}), flush=True)
         return
     log(f'[bench] plain {args.precision} {n} walkers: warmup {W}, timed {K}')
     sim = make_sim(n, total, precision=args.precision)
-    ws, wall, mean_n, kern_ms, ev_n = run_timed(sim, W, K, args.event_steps)
+    ws, wall, mean_n, kern_ms, ev_n, on_chip = run_timed(sim, W, K, args.event_steps)
     value = ws / wall
     ms_per_step = wall * 1e3 / K
     bpw = BYTES_PER_WALKER_STEP[('plain', args.precision, 9)]
     roof = None
     if kern_ms:
-        # the plain discrete step is one kernel (k_discrete, finalised by its last tile)
+        # a step launched by itself is one kernel (k_discrete, finalised by its last tile): the timed
+        # region's kernel for short runs and sizes beyond the LDS, else k_resident is (below)
         k_ms = kern_ms[0]
         bytes_per_launch = bpw * ev_n
         achieved = bytes_per_launch / (k_ms * 1e-3) / 1e9
@@ -634,7 +661,8 @@ def main():
                 "kernel": f"k_discrete<{rname},9> (fused move+PES+branch+compaction)",
                 "avg_launch_us": k_ms * 1e3, "bytes_per_launch": bytes_per_launch,
                 "bytes_per_walker_step": bpw,
-                "step_kernels_us": {"k_discrete": kern_ms[0] * 1e3}}
+                "step_kernels_us": {"k_discrete": kern_ms[0] * 1e3},
+                "launches": "steps launched one at a time after the timed region, with events"}
     log(f'[bench] plain: {value:.4g} walker-steps/s, {ms_per_step * 1e3:.2f} us/step, kernels {kern_ms} ms')
     variants = {}
     del sim
@@ -647,23 +675,34 @@ def main():
         roof["frac_of_copy"] = roof["achieved"] / copy_gbs
         roof["plane_copy_GBs"] = pc_gbs
         roof["frac_of_plane_copy"] = roof["achieved"] / pc_gbs
+    single = None
+    if on_chip:
+        # the timed steps did not run in k_discrete: its block is kept beside theirs
+        single, roof = roof, valu_roofline(f'{args.precision}_np9_{n}',
+                                           "k_resident (128 steps a launch at this size, the walkers in LDS)", value)
     log(f'[bench] device copy: {copy_gbs:.0f} GB/s; 9-plane streaming copy at {n} walkers: {pc_gbs:.0f} GB/s')
 
     if not args.no_variants:
         log('[bench] importance-sampled variant')
         sim = make_sim(n, total, precision=args.precision, imp=True)
-        ws2, wall2, mean2, kern2, ev2 = run_timed(sim, W, K, min(args.event_steps, 50))
+        ws2, wall2, mean2, kern2, ev2, on2 = run_timed(sim, W, K, min(args.event_steps, 50))
         variants['is'] = {"value": ws2 / wall2, "unit": "walker-steps/s", "ms_per_step": wall2 * 1e3 / K,
                           "config": "same PES and walkers, Gaussian-product psi_T (2 stretches + bend), drift and "
                                     "local energy from the trial kernels, Metropolis accept, dt_eff"}
         if kern2:
             names = ['k_is_move', 'k_discrete']
-            variants['is']['step_kernels_us'] = {nm: t * 1e3 for nm, t in zip(names, kern2)}
+            variants['is']['on_chip'] = on2
+            variants['is']['single_step_kernels_us'] = {nm: t * 1e3 for nm, t in zip(names, kern2)}
+            if on2:
+                variants['is']['roofline'] = valu_roofline(f'{args.precision}_np9_is_{n}',
+                                                           "k_resident<IS> (128 steps a launch, the walkers in LDS)",
+                                                           ws2 / wall2)
             bpw_is = BYTES_PER_WALKER_STEP[('is', args.precision, 9)] if args.precision == 'fp32' else None
             if bpw_is:
                 step_ms = sum(kern2)
                 ach = bpw_is * ev2 / (step_ms * 1e-3) / 1e9
-                variants['is']['roofline'] = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                block = 'single_step_roofline' if on2 else 'roofline'
+                variants['is'][block] = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                               "frac": ach / HBM_PEAK_GBS, "bytes_per_walker_step": bpw_is,
                                               "kernels": "k_is_move + k_discrete<float,9,IS> per step (algorithmic "
                                                          "bytes of the step over both kernels' time)"}
@@ -685,7 +724,7 @@ def main():
         spot = SurrogatePotential(model, pv.MorseBendTriatomic(), judge_every=100, judge_stride=100)
         extra = max(0, 101 - (W + K))   # untimed steps after the timing, up to the first judge record
         sim = make_sim(n, W + K + extra + 2, imp=True, pot=spot)
-        ws3, wall3, mean3, _, _ = run_timed(sim, W, K, 0)
+        ws3, wall3, mean3, _, _, _ = run_timed(sim, W, K, 0)
         if extra:
             from pyvibdmc_amd import _native as N
             N.check(N.load().pvd_sim_run(sim._h, extra, N.stream_handle()))
@@ -746,7 +785,7 @@ def main():
                                   f"(exponent argument in FP64), FP64 reductions (vref, population), "
                                   f"Philox draws",
                       "walkers": n, "mean_population": mean_n, "parallelism": "single GPU"},
-           "roofline": roof, "cpu_baseline": cpu, "variants": variants, "zpe": zpe, "time_to_accuracy": tta}
+           "roofline": roof, "single_step_roofline": single, "cpu_baseline": cpu, "variants": variants, "zpe": zpe, "time_to_accuracy": tta}
     print(json.dumps(out), flush=True)
 
 
