@@ -985,8 +985,9 @@ __global__ __launch_bounds__(64 * E_WAVES, 4) void k_mlp_energy(MlpNet M, const 
 // A layer's D registers of unit tiles 2w and 2w + 1 are word 4w + g of a walker's row: the next
 // layer's B operand of input chunk w, lane group g (phys_unit).  Every sum has the order of the
 // H = 128 kernel, the output's included: its 64 products a lane group go through LDS.
-// Six atoms, 1 000 000 walkers FP32: 878 us when the packs were staged through LDS for every 128
-// walkers, 410 now (0.65 PFLOP/s): VALU issue 66 % of the time, matrix cores 28 %, LDS 30 %.  With H = 128
+// Six atoms, 1 000 003 walkers FP32, fallback pass included: 878 us when the packs were staged through
+// LDS for every 128 walkers, 396 now (0.68 PFLOP/s; 487 in a process's first calls, until its clock has
+// risen): VALU issue 66 % of the time, matrix cores 28 %, LDS 30 %.  With H = 128
 // it is slower than the kernel above (six atoms, 200 000 walkers FP64: 71 us against 60).
 template <int NP, int H>
 struct EnergyShape {
