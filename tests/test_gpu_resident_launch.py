@@ -43,36 +43,38 @@ def test_first_resident_launch_of_a_process():
 
 
 def test_small_simulations_on_two_streams_overlap():
-    """Two simulations of 5 000 walkers (20 workgroups each) on two streams run beside each other."""
+    """Two simulations of 5 000 walkers (20 workgroups each) on two streams run beside each other.  Of
+    several pairs of streams, as two streams may share one of the four hardware queues, where work is
+    done in order."""
     import torch
     from pyvibdmc_amd import _native as N
     lib = N.load()
-    sims = [make('water', 5000, 10 ** 5, 'fp32', seed=s) for s in (1, 2)]
-    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
-    torch.cuda.synchronize()
+    sims = [make('water', 5000, 10 ** 6, 'fp32', seed=s) for s in (1, 2)]
+    streams = [torch.cuda.Stream() for _ in range(4)]
 
-    def go(i):
-        with torch.cuda.stream(streams[i]):
+    def go(i, stream):
+        with torch.cuda.stream(stream):
             if not sims[i]._started:
                 sims[i]._start()
             N.check(lib.pvd_sim_run(sims[i]._h, 3000, N.stream_handle()))
-            streams[i].synchronize()
+            stream.synchronize()
 
-    def together():
-        th = [threading.Thread(target=go, args=(i,)) for i in range(2)]
+    def together(a, b):
+        th = [threading.Thread(target=go, args=(i, s)) for i, s in ((0, a), (1, b))]
         [t.start() for t in th]
         [t.join() for t in th]
 
     def ms(f):
+        torch.cuda.synchronize()
         t = time.perf_counter()
         f()
         return (time.perf_counter() - t) * 1e3
 
-    go(0), go(1)
-    turn = min(ms(lambda: (go(0), go(1))) for _ in range(3))
-    both = min(ms(together) for _ in range(3))
+    go(0, streams[0]), go(1, streams[0])
+    turn = min(ms(lambda: (go(0, streams[0]), go(1, streams[0]))) for _ in range(3))
+    both = [ms(lambda: together(a, b)) for k, a in enumerate(streams) for b in streams[k + 1:]]
     print('in turn', turn, 'together', both)
-    assert both < 0.8 * turn
+    assert min(both) < 0.8 * turn
     for s in sims:
         assert s._status()[0] == 0
 
@@ -87,7 +89,7 @@ def test_other_streams_get_their_turn():
     sim._start()
     a, m = torch.cuda.Stream(), torch.randn(1024, 1024, device='cuda')
     waits = []
-    for _ in range(3):
+    for _ in range(4):
         b = torch.cuda.Stream()
         for timed in (False, True):
             torch.cuda.synchronize()
