@@ -73,10 +73,12 @@ def test_launches_in_a_row_from_an_odd_step():
     assert pair('water', 'fp32', 20000, 97 + 4500, 97, None)[0]['rc'] == 0
 
 
-@pytest.mark.parametrize('kw', [dict(DEBUG_alpha=-0.001), dict(DEBUG_alpha=-0.001, imp_samp='water_trial')])
-def test_failure_after_a_redistribution(kw):
+@pytest.mark.parametrize('n,kw', [(122_880, dict(DEBUG_alpha=-0.001)),
+                                  (122_880, dict(DEBUG_alpha=-0.001, imp_samp='water_trial')),
+                                  (480_000, dict(DEBUG_alpha=-0.0005))])  # with launches queued behind the failed one
+def test_failure_after_a_redistribution(n, kw):
     """The retraced steps start from a redistribution, not from the launch's first step."""
-    runs = pair('water', 'fp32', 122_880, 3000, None, kw, spreads=1)
+    runs = pair('water', 'fp32', n, 3000, None, kw, spreads=1)
     assert runs[0]['rc'] != 0 and runs[0]['fail_step'] > 100
 
 
