@@ -188,7 +188,7 @@ int pvd_sim_trajectory(pvd_sim* sim, int64_t t0, int32_t count, double* vref, do
 /* Runs of many discrete steps go to launches that keep the walkers on chip and whose workgroups wait
  * for each other.  Such a launch first waits until all of them run, gate_us microseconds at most;
  * otherwise a second one takes its steps, with those of its workgroups that start within team_us.
- * Negative: the defaults (50 000 and up to 42 000 more by chance, 2 000).  gate_us = 0 gives every
+ * Negative: the defaults (8 000 and up to 10 000 more by chance, 2 000).  gate_us = 0 gives every
  * launch up, which leaves all steps to the second.  No counterpart in the reference. */
 int pvd_sim_resident_waits(pvd_sim* sim, int64_t gate_us, int64_t team_us);
 /* How the steps so far were run: counts[0] launches with the walkers kept on chip, counts[1]

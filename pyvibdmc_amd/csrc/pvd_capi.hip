@@ -196,6 +196,7 @@ int model_spec(const pvd_config& c, int np) {
 int read_ctrl(pvd_sim* s, Ctrl& c, hipStream_t st) {
   HIPCHK(hipMemcpyAsync(&c, s->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  resident_idle(s, st);
   return 0;
 }
 
@@ -236,6 +237,7 @@ void free_sim(pvd_sim* s) {
   for (int i = 0; i < 2; ++i)
     if (s->graph[i]) (void)hipGraphExecDestroy(s->graph[i]);
   drop_surrogate_graphs(s);
+  resident_leave(s);
   if (s->cap_stream) (void)hipStreamDestroy(s->cap_stream);
   void* ptrs[] = {s->coords[0], s->coords[1], s->who[0], s->who[1], s->w, s->E, s->ke, s->kmask,
                   s->ctrl, s->flags, s->gflags, s->rec, s->drec, s->accs, s->xch, s->tr_vref, s->tr_pop, s->tr_dteff, s->tr_births,
@@ -310,10 +312,11 @@ int pvd_sim_create(const pvd_config* cfg, pvd_sim** out) {
   s->cap = cap;
   s->tmax = cfg->num_timesteps > 0 ? cfg->num_timesteps : 1;
   {
-    int dev = 0, cus = 0;
+    int dev = -1, cus = 0;
     if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) ==
                                                  hipSuccess)
       s->cus = cus;
+    s->res_dev = dev;
     if (s->cus < 1) s->cus = 1;
   }
   // tiles of the discrete kernels: at most cap / TILE plus one round of resident workgroups
@@ -366,6 +369,7 @@ int pvd_sim_create(const pvd_config* cfg, pvd_sim** out) {
     if (!s->cont) ALLOC(s->xc[1], sizeof(double) * s->nx * cap);
   }
 #undef ALLOC
+  resident_join(s);
   hipError_t e = hipMemset(s->flags, 0, sizeof(uint64_t) * ntiles);
   if (e == hipSuccess) e = hipMemset(s->gflags, 0, sizeof(uint64_t) * (ntiles / LB_GROUP + 1));
   if (e == hipSuccess) e = hipMemset(s->drec, 0, sizeof(uint64_t) * 3 * ntiles);

@@ -1,9 +1,46 @@
 // Resident discrete steps (pvd_resident.hpp): the launch plan of a simulation and its launches.
+#include <mutex>
+
 #include "pvd_resident.hpp"
 
 namespace pvd {
 
 namespace {
+
+// The simulations of a device that may keep walkers on chip.  A launch's workgroups hold their CUs
+// while they wait for the last of them, so launches on several streams must not each get a part of
+// the CUs: with three of a million walkers, two would wait for each other at their gates whenever the
+// third ends (96 ms step by step, 500 to 600 so, 94 in order).  Launches that together take more than
+// all CUs are therefore put in the order of their calls with events; smaller ones run beside each
+// other.  With one simulation nothing is recorded: a second one's creation ends with a synchronisation
+// of the device after it has joined.
+struct ResDevice {
+  std::mutex mu;
+  std::vector<pvd_sim*> sims;
+  unsigned long long turn = 0;
+};
+constexpr int RES_DEVICES = 64;
+ResDevice& res_device(int dev) {
+  static ResDevice* devices = new ResDevice[RES_DEVICES];  // not destroyed: simulations may outlive static objects
+  return devices[dev];
+}
+
+// the stream waits until what is left of the others' launches fits beside `share` of the CUs
+int res_wait_turn(ResDevice& D, pvd_sim* s, double share, hipStream_t st) {
+  std::vector<pvd_sim*> others;
+  double sum = share;
+  for (pvd_sim* o : D.sims)
+    if (o != s && o->res_turn) {
+      others.push_back(o);
+      sum += o->res_share;
+    }
+  std::sort(others.begin(), others.end(), [](const pvd_sim* a, const pvd_sim* b) { return a->res_turn < b->res_turn; });
+  for (size_t k = 0; k < others.size() && sum > 1.0 + 1e-9; ++k) {
+    HIPCHK(hipStreamWaitEvent(st, others[k]->res_done, 0));
+    sum -= others[k]->res_share;
+  }
+  return 0;
+}
 
 // Largest dynamic LDS a workgroup of k_resident may ask for: 160 KB less its static arrays.
 constexpr int RES_LDS = 160 * 1024 - 5 * 1024;
@@ -41,11 +78,12 @@ struct Plan {
   const void* rest;
   int grid, nt, capl, capb;
   size_t lds;
+  double share;  // of the CUs
 };
 
 template <typename R>
 Plan make_plan(pvd_sim* s, bool who) {
-  Plan P{nullptr, nullptr, 0, 0, 0, 0, 0};
+  Plan P{nullptr, nullptr, 0, 0, 0, 0, 0, 0.0};
   const long long n0 = s->cfg.num_walkers;
   const int gmax = std::min(s->cus, RES_MAXG);
   const int share = 256;
@@ -76,6 +114,7 @@ Plan make_plan(pvd_sim* s, bool who) {
     (void)hipGetLastError();
     return P;
   }
+  P.share = (double)g / ((double)per_cu * s->cus);
   P.fn = I.fn;
   P.rest = I.rest;
   P.grid = g;
@@ -109,7 +148,7 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
   done = 0;
   s->steps_asked += n_steps;
   if (s->cont || !s->xch || s->htrial || s->cfg.pes.kind == PES_EXTERNAL || n_steps < RES_MIN ||
-      s->steps_asked < RES_REPAY)
+      s->steps_asked < RES_REPAY || s->res_dev < 0 || s->res_dev >= RES_DEVICES)
     return 0;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
@@ -164,6 +203,14 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
     A.inv_m[p] = (R)S.inv_m[p];
     A.h2s[p] = S.h2s[p];
   }
+  ResDevice& D = res_device(s->res_dev);
+  std::lock_guard<std::mutex> lock(D.mu);
+  const bool shared = D.sims.size() > 1;
+  if (shared) {
+    if (!s->res_done) HIPCHK(hipEventCreateWithFlags(&s->res_done, hipEventDisableTiming));
+    const int rc = res_wait_turn(D, s, P.share, st);
+    if (rc) return rc;
+  }
   while (done < n_steps) {
     A.steps = std::min(P.lds > RES_LDS / 2 ? RES_STEPS_FULL : RES_STEPS, n_steps - done);
     A.par = (int)(s->next_step & 1);
@@ -180,7 +227,35 @@ int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done) {
     s->epoch_next += 2 * (unsigned)A.steps + 2;  // a failed launch retraces its steps under new epochs
     done += A.steps;
   }
+  if (shared) {
+    HIPCHK(hipEventRecord(s->res_done, st));
+    s->res_share = P.share;
+    s->res_stream = st;
+    s->res_turn = ++D.turn;
+  }
   return 0;
+}
+
+void resident_join(pvd_sim* s) {
+  if (!s->xch || s->res_dev < 0 || s->res_dev >= RES_DEVICES) return;
+  ResDevice& D = res_device(s->res_dev);
+  std::lock_guard<std::mutex> lock(D.mu);
+  D.sims.push_back(s);
+}
+
+void resident_leave(pvd_sim* s) {
+  if (!s->xch || s->res_dev < 0 || s->res_dev >= RES_DEVICES) return;
+  ResDevice& D = res_device(s->res_dev);
+  std::lock_guard<std::mutex> lock(D.mu);
+  D.sims.erase(std::remove(D.sims.begin(), D.sims.end(), s), D.sims.end());
+  if (s->res_done) (void)hipEventDestroy(s->res_done);
+  s->res_done = nullptr;
+}
+
+void resident_idle(pvd_sim* s, hipStream_t st) {
+  if (!s->res_turn || s->res_stream != st) return;
+  std::lock_guard<std::mutex> lock(res_device(s->res_dev).mu);
+  s->res_turn = 0;
 }
 
 template int run_resident<float>(pvd_sim*, int, hipStream_t, int&);

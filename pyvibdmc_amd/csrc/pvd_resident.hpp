@@ -48,12 +48,12 @@ enum : int { RES_ARRIVED = 0, RES_GATE = 32, RES_JOINED = 64, RES_TEAM = 96, RES
 enum : int { RES_CLOSED = 2 * RES_SET, RES_N_OPEN, RES_N_CLOSED, RES_N_SPREAD, RES_SYNCW };
 constexpr size_t RES_XWORDS = RES_XSYNC + (RES_SYNCW + 1) / 2;
 constexpr unsigned RES_OPEN = 1u, RES_SHUT = 0x80000000u;
-// How long the first workgroup waits for the others, in ticks of 10 ns: at the gate 50 ms and up to
-// 42 ms more by chance (two processes that wait on each other's CUs should not give up together),
-// longer than another launch of this kind holds its CUs; a 64th of that where the last gate was
-// closed.  In the second launch, which goes on with those that are there, 2 ms.  Nobody waits for
+// How long the first workgroup waits for the others, in ticks of 10 ns: at the gate 8 ms, longer than
+// another launch of this kind that fills the LDS holds its CUs, and up to 10 ms more by chance (two
+// processes that wait on each other's CUs should not give up together); a 64th of that where the last
+// gate was closed.  In the second launch, which goes on with those that are there, 2 ms.  Nobody waits for
 // the first workgroup's word longer than 60 s.
-constexpr unsigned long long RES_WAIT = 5000000ull, RES_WAIT_MORE = 1ull << 22, RES_TEAM_WAIT = 200000ull,
+constexpr unsigned long long RES_WAIT = 800000ull, RES_WAIT_MORE = 1ull << 20, RES_TEAM_WAIT = 200000ull,
                              RES_WAIT_MAX = 6000000000ull;
 constexpr unsigned RES_CLAMP = 1u << 22;  // a workgroup's published count: beyond any population bound served
 constexpr long long RES_SPIN = 1ll << 24;

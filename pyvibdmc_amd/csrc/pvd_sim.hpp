@@ -62,6 +62,13 @@ struct pvd_sim {
   uint64_t* xch;  // exchange words of the resident steps (discrete weighting)
   unsigned res_launches, res_alone;  // resident launches so far, of several workgroups and of one
   long long steps_asked;  // steps with the library's own draws so far
+  // its place among the device's simulations that keep walkers on chip (ResDevice): device, the stream
+  // and the end of its last launches, the share of the CUs they take, their number (0: they have ended)
+  int res_dev;
+  hipStream_t res_stream;
+  hipEvent_t res_done;
+  double res_share;
+  unsigned long long res_turn;
   unsigned long long res_gate_wait, res_team_wait;  // see RES_WAIT
   double* tr_vref;
   double* tr_pop;
@@ -266,6 +273,11 @@ int do_pes(pvd_sim* s, double* v, hipStream_t st);
 // (all, or none where the resident launch does not serve this simulation, size or stream).
 template <typename R>
 int run_resident(pvd_sim* s, int n_steps, hipStream_t st, int& done);
+// a new simulation is known to the others of its device (before the device is next synchronised); it
+// is no longer; what it launched on a stream has ended
+void resident_join(pvd_sim* s);
+void resident_leave(pvd_sim* s);
+void resident_idle(pvd_sim* s, hipStream_t st);
 
 #define PVD_SIM_OPS(R)                                                                                   \
   template int run_steps<R>(pvd_sim*, int, const double*, const double*, const double*, hipStream_t);  \

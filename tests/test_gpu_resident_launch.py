@@ -79,6 +79,44 @@ def test_small_simulations_on_two_streams_overlap():
         assert s._status()[0] == 0
 
 
+@pytest.mark.parametrize('n', [200_000, 1_000_000])
+def test_large_simulations_on_several_streams_take_turns(n):
+    """Three simulations whose launches take all CUs each: none waits for another's CUs at its gate, so
+    no launch is given up and together they take no longer than in turn."""
+    import torch
+    from pyvibdmc_amd import _native as N
+    from tests.test_gpu_resident_rest import counts
+    lib = N.load()
+    sims = [make('water', n, 10 ** 6, 'fp32', seed=s) for s in (1, 2, 3)]
+    streams = [torch.cuda.Stream() for _ in sims]
+
+    def go(i, steps=1000):
+        with torch.cuda.stream(streams[i]):
+            if not sims[i]._started:
+                sims[i]._start()
+            for _ in range(2):
+                N.check(lib.pvd_sim_run(sims[i]._h, steps // 2, N.stream_handle()))
+            streams[i].synchronize()
+
+    def together():
+        th = [threading.Thread(target=go, args=(i,)) for i in range(3)]
+        [t.start() for t in th]
+        [t.join() for t in th]
+
+    def ms(f):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        f()
+        return (time.perf_counter() - t) * 1e3
+
+    [go(i, 200) for i in range(3)]
+    turn, both = ms(lambda: [go(i) for i in range(3)]), [ms(together) for _ in range(3)]
+    print('in turn', turn, 'together', both)
+    for s in sims:
+        assert s._status()[0] == 0 and counts(s)[1] == 0
+    assert min(both) < 1.3 * turn
+
+
 def test_other_streams_get_their_turn():
     """A million walkers fill the LDS of every CU; a kernel of another stream that needs LDS waits for
     one launch (2 ms), not for all of the 4 000 steps (62 ms).  Of several streams, as one may share a
