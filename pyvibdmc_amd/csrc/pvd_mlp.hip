@@ -1369,7 +1369,7 @@ size_t train_layout(int D, int H, int64_t n, char* ws, TrainBuf& B) {
   // rows 320 bytes past a multiple of 4 KB: the 16 rows that a wave reads at once lie in different
   // channels (8192 elements, width 256, rows of 16 KB: weight gradients 37 us, 20 so); 320 past a
   // multiple of 512 where the rows are shorter than 4 KB, which would else take several times their bytes
-  const int64_t np = (n + 31) / 32 * 32, unit = np <= 2048 ? 256 : 2048, ld = (np + unit - 1 - 160) / unit * unit + 160;
+  const int64_t np = (n + 31) / 32 * 32, unit = np <= 2048 ? 256 : 2048, ld = ((np + unit - 1 - 160) & ~(unit - 1)) + 160;
   const int64_t slice = H == 256 ? train_slice<256>() : train_slice<128>();
   size_t at = 0;
   auto take = [&](size_t bytes) {
